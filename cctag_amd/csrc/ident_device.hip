@@ -17,6 +17,11 @@ long long refine_flops(long long n_iter, long long grid_points, long long cuts, 
 }
 
 namespace {
+int most_cuts(const std::vector<RefineJob>& jobs) {
+  size_t n = 0;
+  for (const RefineJob& r : jobs) n = std::max(n, r.stops.size());
+  return (int)n;
+}
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
@@ -60,15 +65,17 @@ void GpuIdentBackend::ensure(int n_markers, int n_points) {
 
   const size_t o_rj = dev_.reserve(sizeof(RefineJobDev) * nm);
   const size_t o_st = dev_.reserve(sizeof(RefineStateDev) * 2 * nm);
-  const size_t o_gr = dev_.reserve(sizeof(RefineGridDev) * 2 * (size_t)nm * kMaxGrid * kMaxGrid);
-  const size_t o_gm =
-      dev_.reserve(sizeof(double) * 2 * (size_t)nm * kMaxGrid * kMaxGrid * kMaxPairs);
+  const size_t o_pt = dev_.reserve(sizeof(RefinePointDev) * 2 * (size_t)nm * kMaxGrid * kMaxGrid);
+  const size_t o_pa =
+      dev_.reserve(sizeof(double) * 2 * (size_t)nm * kMaxGrid * kMaxGrid * kMaxRefineSums);
+  const size_t o_hm = dev_.reserve(sizeof(RefineHomDev) * (size_t)nm * kMaxGrid * kMaxGrid);
   const size_t o_inv = dev_.reserve(sizeof(float) * kMaxBank * kMaxRatios);
   if (dev_.allocate() != 0) throw std::runtime_error(std::string("hipMalloc: ") + last_error());
   d_ref_jobs_ = dev_.at<RefineJobDev>(o_rj);
   d_work_.state = dev_.at<RefineStateDev>(o_st);
-  d_work_.grid = dev_.at<RefineGridDev>(o_gr);
-  d_work_.gram = dev_.at<double>(o_gm);
+  d_work_.points = dev_.at<RefinePointDev>(o_pt);
+  d_work_.part = dev_.at<double>(o_pa);
+  d_work_.hom = dev_.at<RefineHomDev>(o_hm);
   d_inv_ratio_ = dev_.at<float>(o_inv);
   hip_check(hipMemcpy(d_inv_ratio_, &k_.inv_ratio[0][0], sizeof(float) * kMaxBank * kMaxRatios,
                       hipMemcpyHostToDevice),
@@ -181,7 +188,6 @@ int GpuIdentBackend::pack_refine_jobs(const std::vector<RefineJob>& jobs,
     d.begin_sig = r.begin_sig;
     d.end_sig = r.end_sig;
     d.n_iter = r.n_iter;
-    d.box_inside = box_inside(r, im.w, im.h) ? 1 : 0;
     d.c0x = r.center0.x;
     d.c0y = r.center0.y;
     if (sel_of) {
@@ -213,7 +219,7 @@ void GpuIdentBackend::coarse_centers(const std::vector<RefineJob>& jobs, const H
             "H2D");
   hip_check(hipEventRecord(jobs_copied_, stream_), "event");
   jobs_in_flight_ = true;
-  if (launch_refine_coarse(d_ref_jobs_, n, k_.n_samples, p.imaged_center_n_grid_sample, d_work_,
+  if (launch_refine_coarse(d_ref_jobs_, n, most_cuts(jobs), k_.n_samples, p.imaged_center_n_grid_sample, d_work_,
                            d_centers, stream_) != 0)
     throw std::runtime_error("k_refine coarse launch failed");
 }
@@ -255,7 +261,7 @@ void GpuIdentBackend::refine_gradient(const std::vector<RefineJob>& jobs, const 
                            hipMemcpyHostToDevice, s),
             "H2D");
   const int ns = k_.n_samples;
-  if (launch_refine_coarse(d_ref_jobs_, n, ns, p.imaged_center_n_grid_sample, d_work_,
+  if (launch_refine_coarse(d_ref_jobs_, n, most_cuts(jobs), ns, p.imaged_center_n_grid_sample, d_work_,
                            d_coarse_.as<float>(), s) != 0 ||
       launch_grad_descend(d_grad_jobs_.as<GradJobDev>(), n, grad_steps_, ns, false,
                           d_coarse_.as<float>(), d_gcenters_.as<float>(), d_gcost_.as<double>(),
@@ -332,7 +338,7 @@ void GpuIdentBackend::refine(const std::vector<RefineJob>& jobs, const HostParam
   } else {
     int max_iter = 0;
     for (const RefineJob& r : jobs) max_iter = std::max(max_iter, r.n_iter);
-    if (launch_refine(d_ref_jobs_, n, max_iter, k_.n_samples, p.imaged_center_n_grid_sample,
+    if (launch_refine(d_ref_jobs_, n, max_iter, most_cuts(jobs), k_.n_samples, p.imaged_center_n_grid_sample,
                       d_inv_ratio_, k_.bank_rows, k_.bank_cols, d_work_,
                       h_ref_out_.dev<RefineOutDev>(), h_ref_dist_.dev<float>(), s) != 0)
       throw std::runtime_error("k_refine launch failed");
@@ -378,7 +384,9 @@ void GpuIdentBackend::select_and_refine(const std::vector<CutJob>& cuts,
   hipEventRecord(ev_[2], s);
   int max_iter = 0;
   for (const RefineJob& r : jobs) max_iter = std::max(max_iter, r.n_iter);
-  if (launch_refine(d_ref_jobs_, n, max_iter, k_.n_samples, p.imaged_center_n_grid_sample,
+  // (the stops are selected on the device)
+  const int max_cuts = std::min(p.num_cuts_in_ident_step, kMaxCuts);
+  if (launch_refine(d_ref_jobs_, n, max_iter, max_cuts, k_.n_samples, p.imaged_center_n_grid_sample,
                     d_inv_ratio_, k_.bank_rows, k_.bank_cols, d_work_,
                     h_ref_out_.dev<RefineOutDev>(), h_ref_dist_.dev<float>(), s) != 0)
     throw std::runtime_error("k_refine launch failed");

@@ -37,7 +37,6 @@ struct RefineJobDev {
   float t_can[9], t_inv_can[9], cond[9], cond_inv[9];
   float grid_scale, neighbour0, begin_sig, end_sig;
   int n_iter, n_cuts;
-  int box_inside;  // the outer ellipse's bounding box lies 2 px inside the image
   float c0x, c0y;
   int dist_offset;  // first float of its distances in the packed output
   int sel_index;    // >= 0: the selection whose stops the job takes on the device
@@ -68,39 +67,41 @@ struct RefineStateDev {
   uint32_t sticky;     // bit k: cut k left the image at an earlier grid point
   int pad;
 };
-// One grid point of the current iteration.
-struct RefineGridDev {
-  float H[9], Hi[9];
+// One grid point of an iteration, and its homography in the last one.
+struct RefinePointDev {
   float gx, gy;
-  double cost_local;   // residual sum assuming only this point's own flags
-  int16_t m_local;     // valid cuts under that assumption
-  int16_t has_gram;    // its Gram matrix was stored (the selection may recompute from it)
-  uint32_t oob;        // bit k: a sample of cut k is outside the image
+  uint32_t flagged;    // bit k: cut k left the image at this point or before it
+  uint32_t pad;
 };
-static_assert(sizeof(RefineGridDev) == 96, "grid record size");
-constexpr int kMaxPairs = kMaxCuts * (kMaxCuts + 1) / 2;
+static_assert(sizeof(RefinePointDev) == 16, "one load per grid point");
+struct RefineHomDev {
+  float H[9], Hi[9];
+};
+constexpr int kMaxRefineSums = 26;  // partial sums of a grid point's residual
 // Two sets (by iteration parity): an iteration reads the previous set and
 // writes its own.
 struct RefineWork {
-  RefineStateDev* state;  // 2 x n_jobs
-  RefineGridDev* grid;    // 2 x n_jobs x kMaxGrid^2
-  double* gram;           // 2 x n_jobs x kMaxGrid^2 x kMaxPairs
+  RefineStateDev* state;   // 2 x n_jobs
+  RefinePointDev* points;  // 2 x n_jobs x kMaxGrid^2
+  double* part;            // 2 x n_jobs x kMaxGrid^2 x kMaxRefineSums
+  RefineHomDev* hom;       // n_jobs x kMaxGrid^2
 };
 
 // out: one header per job; dist: per job n_cuts x bank_rows distances from
 // its dist_offset on (invalid cuts' rows are not written).
 // The grid search's first iteration only: per job the centre it moves to
 // (centers: 2 per job, device memory).
-int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int n_samples, int grid_n,
-                         const RefineWork& work, float* centers, hipStream_t s);
+int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int max_cuts, int n_samples,
+                         int grid_n, const RefineWork& work, float* centers, hipStream_t s);
 // The read-out of launch_refine's last kernel at given homographies (9 per
 // job), centres (2 per job) and scores instead of the grid search's choice.
 int launch_refine_readout(const RefineJobDev* jobs, int n_jobs, int n_samples, const float* H,
                           const float* centers, const double* cost, const float* inv_ratio,
                           int bank_rows, int bank_cols, const RefineWork& work, RefineOutDev* out,
                           float* dist, hipStream_t s);
-int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int n_samples, int grid_n,
-                  const float* inv_ratio, int bank_rows, int bank_cols, const RefineWork& work,
+// max_iter, max_cuts: the most iterations and cuts of a job.
+int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int max_cuts, int n_samples,
+                  int grid_n, const float* inv_ratio, int bank_rows, int bank_cols, const RefineWork& work,
                   RefineOutDev* out, float* dist, hipStream_t s);
 
 // Algorithmic FLOPs of the grid search on one marker: n_iter iterations of

@@ -15,6 +15,7 @@
 //                the reference's float operations.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 
 #include "ident_device.hpp"
@@ -34,18 +35,25 @@ struct Img {
   const uint32_t* q;
   int w, h;
   __device__ __forceinline__ uint32_t quad(int x, int y) const { return ((gptr_u32)q)[x + y * w]; }
+  // the same for 0 <= x < w, 0 <= y < h: a 24-bit multiply-add and a 32-bit
+  // byte offset (an image has less than 2^30 pixels)
+  __device__ __forceinline__ uint32_t quad24(uint32_t x, uint32_t y) const {
+    const uint32_t off = (__umul24(y, (uint32_t)w) + x) << 2;
+    return *(gptr_u32)((const __attribute__((address_space(1))) char*)(gptr_u32)q + off);
+  }
 };
 
-// Identification.hpp:197-222: half of the bilinear value at (x, y), from
-// the quad of pixel (floor x, floor y).
-__device__ __forceinline__ float bilinear_of(float x, float y, uint32_t quad) {
-  const int px = (int)x, py = (int)y;
-  const float fx = x - px, fy = y - py;
+// Identification.hpp:197-222: the bilinear value at the offset (fx, fy) into
+// the quad of its pixel, and half of it at (x, y).
+__device__ __forceinline__ float bilinear2(float fx, float fy, uint32_t quad) {
   const float fx1 = 1.0f - fx, fy1 = 1.0f - fy;
   const float w1 = fx1 * fy1, w2 = fx * fy1, w3 = fx1 * fy, w4 = fx * fy;
   const float a = (float)(quad & 255u), b = (float)((quad >> 8) & 255u),
               c = (float)((quad >> 16) & 255u), d = (float)(quad >> 24);
-  return (a * w1 + b * w2 + c * w3 + d * w4) / 2;
+  return a * w1 + b * w2 + c * w3 + d * w4;
+}
+__device__ __forceinline__ float bilinear_of(float x, float y, uint32_t quad) {
+  return bilinear2(x - (int)x, y - (int)y, quad) / 2;
 }
 
 __device__ __forceinline__ void apply_h(float& xr, float& yr, const float* H, float x, float y) {
@@ -352,33 +360,24 @@ __global__ __launch_bounds__(kSelectBlock) void k_select_cuts(const SelectJobDev
 }
 
 // ---------------------------------------------------------------------------
-// Centre refinement, one launch per grid-search iteration.  Block (g, m)
-// of k_refine_iter evaluates grid point g of marker m: its homography, the
-// signals of every selected cut (LDS), their out-of-bounds flags and the
-// residual sum_{k<l} sum_i (s_ki - s_li)^2 over its valid cuts.  The
-// selection that follows an iteration -- the sticky out-of-bounds flags in
-// grid-point order, each grid point's residual over the cuts valid there,
-// the move to the first minimum as the reference's loop does -- is redone
-// by every block of the next launch (and by the final kernel), so an
-// iteration costs one launch.
+// Centre refinement.  An iteration of the grid search evaluates the grid
+// points around the current centre: per point its homography, the samples of
+// every selected cut and the residual sum_{k<l} sum_i (s_ki - s_li)^2 over
+// its valid cuts, taken per sample as m S2_i - S1_i^2 (S1_i and S2_i the sum
+// and the sum of squares of the valid cuts' samples, in double, in cut
+// order; summed in sample order by chunks of kRefineChunk).  The centre then
+// moves to the first minimum, as the reference's loop does.  A cut that
+// leaves the image at a grid point is invalid there and at every later point
+// (Identification.cpp:264-273).
 //
-// A cut flagged at an earlier grid point of the same iteration is invalid
-// at the later ones, which a block cannot see while it runs.  So block g
-// first tests, for the grid points before it, whether each valid cut surely
-// stays inside the image (cut_surely_inside).  When every one does -- the
-// usual case -- the block knows its valid cuts and takes the residual as
-// sum_i (m S2_i - S1_i^2), S1_i and S2_i the sum and the sum of squares of
-// the valid cuts' samples (double, in cut order).  Otherwise it stores the
-// Gram matrix C_kl = sum_i s_ki s_li in double, from which the selection
-// recomputes the residual for any valid set as
-// (m-1) sum_k C_kk - 2 sum_{k<l} C_kl.
-constexpr int kRefineBlock = 256;
+// The search is bound by the instruction issue of the sampling (per sample
+// two quotients, a projective map and a bilinear blend whose rounding is the
+// reference's): a cut proven inside the image needs no bounds test, its two
+// quotients share one reciprocal (div2_rn) and the halving of the samples is
+// left to the end of the sum (an exact power of two).
 constexpr int kFinalBlock = 1024;  // one block per marker: every loop of the read-out in one pass
-constexpr int kRefineChunk = 10;  // samples per sampling work item
-constexpr int kLoadBatch = 10;    // samples whose image reads are issued together
-static_assert(kRefineChunk % kLoadBatch == 0, "whole load batches per chunk");
+constexpr int kRefineChunk = 10;  // samples of a cut whose image reads are in flight together
 constexpr int G2MAX = kMaxGrid * kMaxGrid;
-constexpr int kFuseMaxBlocks = 2048;  // grid blocks up to which the selection is fused
 constexpr int kXcds = 8;               // accelerator complex dies of the MI355X
 
 // getNearbyPoints point g + computeHomographyFromEllipseAndImagedCenter
@@ -413,19 +412,37 @@ __device__ void grid_homography(const RefineJobDev& J, float cur_x, float cur_y,
   inverse3(Hf, Hi);
 }
 
-// extractSignalUsingHomography (Identification.cpp:216-280), first part,
-// one thread per cut: the stop back-projected by Hi, the sample positions
-// from begin*stop to end*stop in the marker plane as the reference's running
-// sums, kept at the start of every kRefineChunk-sample chunk (the chunks'
-// threads then resume the sums from there).
-constexpr int kMaxChunks = (kMaxSamples + kRefineChunk - 1) / kRefineChunk;
-struct CutWalk {
-  float2 start[kMaxChunks];
-  float2 step;
+// extractSignalUsingHomography (Identification.cpp:216-280), first part: the
+// stop back-projected by Hi, the sample positions from begin*stop to
+// end*stop in the marker plane as the reference's running sums.
+__host__ __device__ constexpr int chunks_of(int n_samples) {
+  return (n_samples + kRefineChunk - 1) / kRefineChunk;
+}
+// The residual's terms are summed kSumChunk samples at a time, then the sums.
+constexpr int kSumChunk = 5;
+static_assert(kRefineChunk % kSumChunk == 0, "whole sums per chunk");
+__host__ __device__ constexpr int sum_chunks_of(int n_samples) {
+  return (n_samples + kSumChunk - 1) / kSumChunk;
+}
+constexpr int kMaxSumChunks = sum_chunks_of(kMaxSamples);
+static_assert(kMaxSumChunks <= kMaxRefineSums, "the work buffer's sums");
+
+// A cut's samples: their number n and 1/(n - 1) in double.
+struct Samples {
+  int n;
+  double inv_steps;
 };
 
-__device__ void cut_walk_starts(const float* Hi, float2 stop, float begin_sig, float end_sig,
-                                int n_samples, CutWalk& w) {
+// x / (n - 1), correctly rounded (div_n_product).
+__device__ __forceinline__ float per_step(float x, const Samples& ns) {
+  const double p = div_n_product(x, ns.inv_steps);
+  return div_n_tiny(p) ? x / ((float)ns.n - 1.f) : (float)p;
+}
+
+// The first sample position and the step.
+__device__ __forceinline__ void cut_walk_begin(const float* Hi, float2 stop, float begin_sig,
+                                               float end_sig, const Samples& ns, float2& first,
+                                               float2& step) {
   float bx, by;
   apply_h(bx, by, Hi, stop.x, stop.y);
   float xs, ys, xe, ye;
@@ -443,413 +460,556 @@ __device__ void cut_walk_starts(const float* Hi, float2 stop, float begin_sig, f
     xe = bx;
     ye = by;
   }
-  const float stepX = (xe - xs) / ((float)n_samples - 1.f), stepY = (ye - ys) / ((float)n_samples - 1.f);
-  float x = xs, y = ys;
-  const int nchunk = (n_samples + kRefineChunk - 1) / kRefineChunk;
-  for (int c = 0; c < nchunk; ++c) {
-    w.start[c] = make_float2(x, y);
-    for (int t = 0; t < kRefineChunk; ++t) {
-      x += stepX;
-      y += stepY;
-    }
-  }
-  w.step = make_float2(stepX, stepY);
+  step.x = per_step(xe - xs, ns);
+  step.y = per_step(ye - ys, ns);
+  first = make_float2(xs, ys);
 }
 
-// Whether every sample of a cut surely falls inside the image at the grid
-// point whose homography is H (inverse Hi).  The samples lie, up to the
-// rounding of their running sums and of the mapping (far below a pixel), on
-// the image of the marker-plane segment t * b, t in [begin, end], b = the
-// stop back-projected (homogeneous (b0, b1, b2) = Hi (stop, 1)).  When the
-// projective denominator keeps one sign along t in [0, 1], H maps that
-// segment to a straight one ending at the stop; H maps the unit disk onto
-// the outer ellipse's interior, so with begin * b inside the disk the inner
-// end lies in the ellipse.  Stop and ellipse box 2 px inside the image
-// (box_inside) then keep every sample inside [0, w-1) x [0, h-1).
-__device__ __forceinline__ bool cut_surely_inside(const float* H, const float* Hi, float2 stop,
-                                                  float begin_sig, float end_sig, int w, int h) {
-  if (!(end_sig <= 1.f && stop.x >= 2.f && stop.x <= (float)w - 3.f && stop.y >= 2.f &&
-        stop.y <= (float)h - 3.f))
-    return false;
+// Where the samples of a cut lie at a grid point (homography H, inverse Hi),
+// decided from the two ends of the cut.  The samples are, up to rounding,
+// the images of the marker-plane segment t * b, t in [begin, end], b the stop
+// back-projected (homogeneous b = Hi (stop, 1)).  When the projective
+// denominator keeps its sign between the ends (it is linear in t) the image
+// is the straight segment between the ends' images, so two ends 2 px inside
+// the image keep every sample in [0, w-1) x [0, h-1), and one end 2 px
+// outside puts its own sample outside.  The positions compared here and the
+// samples' own differ by their rounding: a relative 2^-22 or so of the terms'
+// magnitudes over the denominator, below 0.1 px where `steady` holds.  The
+// window on the denominator keeps div2_rn away from the ends of the float
+// range.  Anything else is kUnsure and gets its samples tested.
+enum CutPlace { kInside, kOutside, kUnsure };
+__device__ __forceinline__ CutPlace cut_place(const float* H, const float* Hi, float2 stop,
+                                              float begin_sig, float end_sig, int w, int h) {
   const float b0 = Hi[0] * stop.x + Hi[1] * stop.y + Hi[2];
   const float b1 = Hi[3] * stop.x + Hi[4] * stop.y + Hi[5];
   const float b2 = Hi[6] * stop.x + Hi[7] * stop.y + Hi[8];
-  const float e0 = H[8] * b2, e1 = H[6] * b0 + H[7] * b1 + H[8] * b2;
-  const float scale = fabsf(H[6] * b0) + fabsf(H[7] * b1) + fabsf(H[8] * b2);
-  const bool keeps_sign = (e0 > 0.f) == (e1 > 0.f) && fabsf(e0) > 1e-3f * scale &&
-                          fabsf(e1) > 1e-3f * scale;
-  return keeps_sign && begin_sig * begin_sig * (b0 * b0 + b1 * b1) <= 0.98f * (b2 * b2);
+  bool all_in = true, out = false;
+  float den[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float t = e ? end_sig : begin_sig, p0 = t * b0, p1 = t * b1;
+    const float d = H[6] * p0 + H[7] * p1 + H[8] * b2, ad = fabsf(d);
+    const float s = d < 0.f ? -1.f : 1.f;
+    const float x = s * (H[0] * p0 + H[1] * p1 + H[2] * b2);  // times |d|: the position
+    const float y = s * (H[3] * p0 + H[4] * p1 + H[5] * b2);
+    const float mag = fmaxf(fabsf(H[0] * p0) + fabsf(H[1] * p1) + fabsf(H[2] * b2),
+                            fabsf(H[3] * p0) + fabsf(H[4] * p1) + fabsf(H[5] * b2));
+    const float dmag = fabsf(H[6] * p0) + fabsf(H[7] * p1) + fabsf(H[8] * b2);
+    const bool steady = ad > 0.05f * dmag && mag < 65536.f * ad && ad > 0x1p-60f * fabsf(b2) &&
+                        ad < 0x1p60f * fabsf(b2);
+    den[e] = d;
+    all_in &= steady && x >= 2.f * ad && x <= (float)(w - 3) * ad && y >= 2.f * ad &&
+              y <= (float)(h - 3) * ad;
+    out |= steady && (x < -2.f * ad || x > (float)(w + 1) * ad || y < -2.f * ad ||
+                      y > (float)(h + 1) * ad);
+  }
+  if (out) return kOutside;
+  return all_in && (den[0] > 0.f) == (den[1] > 0.f) ? kInside : kUnsure;
 }
 
-// Second part for samples [c*kRefineChunk, ...) of a cut: mapped by H, half
-// bilinear value; 0 and the flag when out of the image.
-__device__ bool sample_chunk(const Img& im, const float* H, const CutWalk& w, int n_samples, int c,
-                             float* out) {
-  float x = w.start[c].x, y = w.start[c].y;
-  const float stepX = w.step.x, stepY = w.step.y;
-  const int i0 = c * kRefineChunk;
+// u / w and v / w, each correctly rounded: the reciprocal refined by one
+// Newton step, a quotient and two remainder corrections (Markstein, IBM J.
+// Res. Dev. 1990), which is the division's own sequence without its scaling
+// of extreme operands -- w and the quotients are far from the ends of the
+// float range here (cut_place) -- and with the reciprocal shared.
+__device__ __forceinline__ void div2_rn(float u, float v, float w, float& x, float& y) {
+  float r = __builtin_amdgcn_rcpf(w);
+  r = __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
+  float q = u * r;
+  q = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
+  x = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
+  q = v * r;
+  q = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
+  y = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
+}
+
+// Second part for the next N samples of a cut from position p on (advanced
+// past them): mapped by H, twice the half-bilinear value into val[].
+// kInside cuts only, whole chunks.
+template <int N>
+__device__ __forceinline__ void sample_inside(const Img& im, const float* H, float2& p, float2 step,
+                                              float (&val)[N]) {
+  float fx[N], fy[N];
+  uint32_t qd[N];
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    const float u = H[0] * p.x + H[1] * p.y + H[2];
+    const float v = H[3] * p.x + H[4] * p.y + H[5];
+    const float ww = H[6] * p.x + H[7] * p.y + H[8];
+    float xr, yr;
+    div2_rn(u, v, ww, xr, yr);
+    qd[t] = im.quad24((uint32_t)(int)xr, (uint32_t)(int)yr);
+    fx[t] = __builtin_amdgcn_fractf(xr);  // positions are positive: x - (int)x
+    fy[t] = __builtin_amdgcn_fractf(yr);
+    p.x += step.x;
+    p.y += step.y;
+  }
+#pragma unroll
+  for (int t = 0; t < N; ++t) val[t] = bilinear2(fx[t], fy[t], qd[t]);
+}
+
+// The same for any cut and the last, partial chunk (`live` samples left): 0
+// for a sample outside the image; returns whether one is.  BATCH samples'
+// reads are in flight together.
+template <int N, int BATCH>
+__device__ __forceinline__ bool sample_any(const Img& im, const float* H, float2& p, float2 step,
+                                           int live, float* val) {
+  static_assert(N % BATCH == 0, "whole load batches per chunk");
   const float xmax = (float)(im.w - 1), ymax = (float)(im.h - 1);
   bool oob = false;
-  // per group of kLoadBatch samples: positions first, then every corner load
-  // (an outside sample reads pixel (0, 0), so the loads need no branch and
-  // are in flight together), then the values
 #pragma unroll
-  for (int t0 = 0; t0 < kRefineChunk; t0 += kLoadBatch) {
-    float xr[kLoadBatch], yr[kLoadBatch];
-    bool in[kLoadBatch];
+  for (int t0 = 0; t0 < N; t0 += BATCH) {
+    float fx[BATCH], fy[BATCH];
+    bool in[BATCH];
+    uint32_t qd[BATCH];
 #pragma unroll
-    for (int t = 0; t < kLoadBatch; ++t) {
-      apply_h(xr[t], yr[t], H, x, y);
-      const bool live = i0 + t0 + t < n_samples;
-      in[t] = live && xr[t] >= 0.f && xr[t] < xmax && yr[t] >= 0.f && yr[t] < ymax;
-      oob |= live && !in[t];
-      x += stepX;
-      y += stepY;
+    for (int t = 0; t < BATCH; ++t) {
+      float xr, yr;
+      apply_h(xr, yr, H, p.x, p.y);
+      in[t] = t0 + t < live && xr >= 0.f && xr < xmax && yr >= 0.f && yr < ymax;
+      oob |= t0 + t < live && !in[t];
+      // an outside sample reads pixel (0, 0), so the loads need no branch
+      qd[t] = in[t] ? im.quad((int)xr, (int)yr) : im.quad(0, 0);
+      fx[t] = xr - (int)xr;
+      fy[t] = yr - (int)yr;
+      p.x += step.x;
+      p.y += step.y;
     }
-    uint32_t qd[kLoadBatch];
 #pragma unroll
-    for (int t = 0; t < kLoadBatch; ++t) qd[t] = in[t] ? im.quad((int)xr[t], (int)yr[t]) : im.quad(0, 0);
-#pragma unroll
-    for (int t = 0; t < kLoadBatch; ++t) {
-      if (i0 + t0 + t >= n_samples) continue;
-      out[i0 + t0 + t] = in[t] ? bilinear_of(xr[t], yr[t], qd[t]) : 0.f;
-    }
+    for (int t = 0; t < BATCH; ++t) val[t0 + t] = in[t] ? bilinear2(fx[t], fy[t], qd[t]) : 0.f;
   }
   return oob;
 }
 
-__device__ __forceinline__ int pair_offset(int k, int nc) { return k * nc - k * (k - 1) / 2; }
-
-// Row k's share of sum_{k<l valid} sum_i (s_ki - s_li)^2 from the Gram
-// matrix C (packed upper triangle): (m-1) C_kk - 2 sum_{l>k valid} C_kl,
-// valid cuts being the set bits of `valid`.  The row's entries are read
-// kRowBatch at a time (indices clamped into the row, so the reads need no
-// branch and are in flight together) and subtracted in column order,
-// skipping invalid columns as the plain loop does.
-constexpr int kRowBatch = 8;
-__device__ __forceinline__ double gram_row(const double* C, uint32_t valid, int k, int nc, int m) {
-  if (!((valid >> k) & 1u)) return 0.0;
-  const double* row = C + pair_offset(k, nc);
-  const int last = nc - 1 - k;  // row[0 .. last]
-  double acc = (double)(m - 1) * row[0];
-  for (int d0 = 1; d0 <= last; d0 += kRowBatch) {
-    double v[kRowBatch];
-#pragma unroll
-    for (int j = 0; j < kRowBatch; ++j) v[j] = row[min(d0 + j, last)];
-#pragma unroll
-    for (int j = 0; j < kRowBatch; ++j)
-      if (d0 + j <= last && ((valid >> (k + d0 + j)) & 1u)) acc -= 2.0 * v[j];
+// Whether a sample of a cut falls outside the image (the kUnsure cuts).
+__device__ bool samples_leave(const Img& im, const float* H, const float* Hi, float2 stop,
+                              float begin_sig, float end_sig, const Samples& ns) {
+  float2 p, step;
+  cut_walk_begin(Hi, stop, begin_sig, end_sig, ns, p, step);
+  const float xmax = (float)(im.w - 1), ymax = (float)(im.h - 1);
+  for (int i = 0; i < ns.n; ++i) {
+    float xr, yr;
+    apply_h(xr, yr, H, p.x, p.y);
+    if (!(xr >= 0.f && xr < xmax && yr >= 0.f && yr < ymax)) return true;
+    p.x += step.x;
+    p.y += step.y;
   }
-  return acc;
+  return false;
 }
 
-// Sum over the 64 lanes of a wavefront in a fixed tree order (lane 0 holds
-// the result): identical wherever it is evaluated.
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+// A grid point's residual from its chunks' sums (those of the doubled
+// samples); FLT_MAX (never picked) below two valid cuts.
+__device__ __forceinline__ float point_residual(const double* part, int nchunk, int m) {
+  double sum = part[0];
+#pragma unroll
+  for (int c = 1; c < kMaxSumChunks; ++c)
+    if (c < nchunk) sum += part[c];
+  return m < 2 ? FLT_MAX : (float)(0.25 * sum) / (float)(m * (m - 1) / 2);
 }
 
 __device__ __forceinline__ uint32_t cut_bits(int nc) { return nc >= 32 ? ~0u : (1u << nc) - 1u; }
 
-// Selection step of an iteration (what the reference's loop does after
-// evaluating its grid), by wavefront 0 with lane g on grid point g: the
-// sticky out-of-bounds flags in grid-point order (a prefix OR over the
-// lanes), each point's residual (its block's own when the valid cuts are the
-// ones it assumed, otherwise recomputed from its Gram matrix with the same
-// row sums and reduction order), the first minimum, the next centre.  Called
-// by a whole block (one barrier); every block that calls it with the same
-// inputs gets the same state.
-__device__ void pick_state(const RefineJobDev& J, int grid_n, const RefineStateDev& prev,
-                           const RefineGridDev* GM, const double* gram_m, RefineStateDev& S) {
-  const int tid = threadIdx.x, nc = J.n_cuts, G2 = grid_n * grid_n;
-  if (tid < 64) {
-    const uint32_t cuts = cut_bits(nc);
-    const bool on = tid < G2;
-    const uint32_t sp = prev.sticky;
-    uint32_t own = 0;
-    double acc = 0.0;
-    int ml = 0, hg = 0;
-    float gx = 0.f, gy = 0.f;
-    if (on) {
-      const RefineGridDev& G = GM[tid];
-      own = G.oob;
-      acc = G.cost_local;
-      ml = G.m_local;
-      gx = G.gx;
-      gy = G.gy;
-      hg = G.has_gram;
+// What the reference's loop does after evaluating a grid, by wavefront 0
+// with lane g on grid point g: the first minimum among the points with a
+// residual below FLT_MAX becomes the centre, the neighbourhood shrinks;
+// without one the marker has failed.  `sticky`: the cuts flagged by the end
+// of the iteration.
+__device__ __forceinline__ void select_state(bool on, float res, float gx, float gy, uint32_t sticky,
+                                             const RefineStateDev& prev, int grid_n,
+                                             RefineStateDev& S) {
+  const bool pickable = on && res < FLT_MAX;
+  float key = pickable ? res : INFINITY;
+  int idx = pickable ? (int)threadIdx.x : 64;
+  for (int o = 32; o > 0; o >>= 1) {
+    const float k2 = __shfl_xor(key, o, 64);
+    const int i2 = __shfl_xor(idx, o, 64);
+    if (k2 < key || (k2 == key && i2 < idx)) {
+      key = k2;
+      idx = i2;
     }
-    uint32_t run = own;
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t v = __shfl_up(run, o, 64);
-      if (tid >= o) run |= v;
+  }
+  const int b = idx < 64 ? idx : -1;
+  const float bx = __shfl(gx, b < 0 ? 0 : b, 64), by = __shfl(gy, b < 0 ? 0 : b, 64);
+  if (threadIdx.x == 0) {
+    RefineStateDev n = prev;
+    n.sticky = sticky;
+    if (b < 0) {
+      n.ok = 0;
+    } else {
+      n.ok = 1;
+      n.best_g = b;
+      n.cx = bx;
+      n.cy = by;
+      n.neighbour = prev.neighbour / (float)((grid_n - 1) / 2);
+      n.min_res = key;
     }
-    run |= sp;
-    const uint32_t valid = ~run & cuts;
-    const int mv = __popc(valid);
-    const bool same = valid == (~(sp | own) & cuts) && mv == ml;
-    // points whose valid cuts differ from the ones their block assumed, one
-    // at a time over the whole wavefront, as the block itself sums.  Such a
-    // point's block found a flag possible at an earlier point and stored its
-    // Gram matrix; were one missing, the marker fails rather than keep a
-    // residual over the wrong cuts (cut_surely_inside rules that out).
-    const bool lost = __ballot(on && !same && !hg) != 0;
-    for (unsigned long long redo = __ballot(on && !same); redo; redo &= redo - 1) {
-      const int gg = __builtin_ctzll(redo);
-      const uint32_t vg = __shfl(valid, gg, 64);
-      const int mg = __shfl(mv, gg, 64);
-      const double part = tid < nc ? gram_row(gram_m + (size_t)gg * kMaxPairs, vg, tid, nc, mg) : 0.0;
-      const double sum = __shfl(wave_sum(part), 0, 64);
-      if (tid == gg) acc = sum;
-    }
-    const float res = mv < 2 ? FLT_MAX : (float)acc / (float)(mv * (mv - 1) / 2);
-    // the first minimum among the points with two valid cuts and a residual
-    // below FLT_MAX: lexicographic (residual, index) minimum over the lanes
-    const bool pickable = on && mv >= 2 && res < FLT_MAX;
-    float key = pickable ? res : INFINITY;
-    int idx = pickable ? tid : 64;
-    for (int o = 32; o > 0; o >>= 1) {
-      const float k2 = __shfl_xor(key, o, 64);
-      const int i2 = __shfl_xor(idx, o, 64);
-      if (k2 < key || (k2 == key && i2 < idx)) {
-        key = k2;
-        idx = i2;
-      }
-    }
-    const uint32_t sticky = __shfl(run, G2 - 1, 64);
-    const int b = idx < 64 && !lost ? idx : -1;
-    const float bx = __shfl(gx, b < 0 ? 0 : b, 64), by = __shfl(gy, b < 0 ? 0 : b, 64);
-    if (tid == 0) {
-      S.sticky = sticky;
-      S.neighbour = prev.neighbour;
-      if (b < 0) {
-        S.ok = 0;
-        S.best_g = prev.best_g;
-        S.cx = prev.cx;
-        S.cy = prev.cy;
-        S.min_res = prev.min_res;
-      } else {
-        S.ok = 1;
-        S.best_g = b;
-        S.cx = bx;
-        S.cy = by;
-        S.neighbour /= (float)((grid_n - 1) / 2);
-        S.min_res = key;
-      }
+    S = n;
+  }
+}
+
+__device__ __forceinline__ RefineStateDev first_state(const RefineJobDev& J) {
+  RefineStateDev s;
+  s.cx = J.c0x;
+  s.cy = J.c0y;
+  s.neighbour = J.neighbour0;
+  s.min_res = FLT_MAX;
+  s.ok = 1;
+  s.best_g = 0;
+  s.sticky = 0;
+  s.pad = 0;
+  return s;
+}
+
+// The state a marker starts iteration `it` with: the job's start for the
+// first one, otherwise the selection over the previous launch's records
+// (buffers of parity (it - 1) & 1).  In two steps, so that the records are on
+// their way while the block reads its job: lane g of wavefront 0 loads grid
+// point g's, then the whole block takes the state.
+struct PointRecord {
+  RefineStateDev prev;
+  RefinePointDev point;
+  double part[kMaxSumChunks];
+};
+__device__ __forceinline__ void load_records(int it, int m, int n_jobs, int n_samples, int grid_n,
+                                             const RefineWork& W, PointRecord& r) {
+  if (it == 0 || threadIdx.x >= 64) return;
+  const int pb = (it - 1) & 1, g = (int)threadIdx.x < grid_n * grid_n ? threadIdx.x : 0;
+  const size_t at = ((size_t)pb * n_jobs + m) * G2MAX + g;
+  const int last = sum_chunks_of(n_samples) - 1;
+  r.prev = W.state[(size_t)pb * n_jobs + m];
+  r.point = W.points[at];
+#pragma unroll
+  for (int c = 0; c < kMaxSumChunks; ++c) r.part[c] = W.part[at * kMaxRefineSums + min(c, last)];
+}
+__device__ void state_at(const RefineJobDev& J, int it, int n_samples, int grid_n,
+                         const PointRecord& r, RefineStateDev& S) {
+  const int tid = threadIdx.x;
+  if (it == 0) {
+    if (tid == 0) S = first_state(J);
+  } else if (tid < 64) {
+    const int G2 = grid_n * grid_n;
+    const float res = point_residual(r.part, sum_chunks_of(n_samples),
+                                     __popc(~r.point.flagged & cut_bits(J.n_cuts)));
+    if (r.prev.ok) {
+      select_state(tid < G2, res, r.point.gx, r.point.gy, __shfl(r.point.flagged, G2 - 1, 64),
+                   r.prev, grid_n, S);
+    } else if (tid == 0) {
+      S = r.prev;
     }
   }
   __syncthreads();
 }
 
-// The state a marker starts iteration `it` with: the job's start for the
-// first one, otherwise the selection over the previous iteration's grid
-// (buffers of parity (it - 1) & 1).
-__device__ void state_at(const RefineJobDev& J, int it, int m, int n_jobs, int grid_n,
-                         const RefineWork& W, RefineStateDev& S) {
-  const int tid = threadIdx.x;
-  if (it == 0) {
-    if (tid == 0) {
-      S.cx = J.c0x;
-      S.cy = J.c0y;
-      S.neighbour = J.neighbour0;
-      S.min_res = FLT_MAX;
-      S.ok = 1;
-      S.best_g = 0;
-      S.sticky = 0;
-    }
-    __syncthreads();
-    return;
-  }
-  const int pb = (it - 1) & 1;
-  const RefineStateDev& prev = W.state[(size_t)pb * n_jobs + m];
-  if (!prev.ok) {
-    if (tid == 0) S = prev;
-    __syncthreads();
-    return;
-  }
-  pick_state(J, grid_n, prev, W.grid + ((size_t)pb * n_jobs + m) * G2MAX,
-             W.gram + ((size_t)pb * n_jobs + m) * G2MAX * kMaxPairs, S);
-}
+// Two kernels run the search, with the same results: k_refine_iter, one
+// launch per iteration, spreads few markers over the chip; k_refine_search,
+// a block per marker, does the least work for many.
+//
+// k_refine_iter: iteration `it`, block (b, m) on chunks [b * per, (b + 1) *
+// per) of marker m's samples -- the residual is a sum over samples, so a
+// chunk's share needs no other block.  Every block derives the iteration's
+// start from the records the previous launch left (the last selection is the
+// read-out kernel's).
+//
+// A lane takes one cut at one grid point and walks its samples, the grid
+// points side by side: the 25 lanes of a cut sample within a pixel or a few
+// of each other, so a wavefront's load touches few cache lines.  (With a
+// block per grid point the lanes of a load lay on 57 different lines, and
+// the L1's tag lookups, one line per cycle, took as long as the arithmetic.)
+// The chunk's samples meet in LDS, double-buffered with one barrier per
+// chunk; two lanes per grid point and sample then take the sum and the sum
+// of squares over the cuts.
+constexpr int kMaxRefineBlock = (G2MAX * kMaxCuts + 63) / 64 * 64;
 
-// Iteration `it` of the grid search: block (g, m) takes marker m's state --
-// with `fused`, derived from the previous iteration by the block itself
-// (every block of the marker derives the same one; block 0 stores it),
-// otherwise as k_refine_pick left it -- then evaluates grid point g:
-// homography, cut signals in LDS, out-of-bounds flags, Gram matrix and the
-// residual under its own flags.  Buffers alternate with the iteration's
-// parity.  Fusing saves a launch per iteration when few markers leave the
-// chip idle; with many markers the repeated selection costs more than the
-// launch.
-__global__ __launch_bounds__(kRefineBlock) void k_refine_iter(
-    const RefineJobDev* __restrict__ jobs, int it, int n_samples, int grid_n, int fused,
-    RefineWork W) {
+__global__ __launch_bounds__(kMaxRefineBlock) void k_refine_iter(
+    const RefineJobDev* __restrict__ jobs, int it, int per, Samples ns, int grid_n, RefineWork W) {
+  extern __shared__ float sig_lds[];  // [buffer][cut][grid point][sample of the chunk], doubled samples
   __shared__ float gH[G2MAX][9], gHi[G2MAX][9];
-  __shared__ float sig[kMaxCuts][kMaxSamples + 1];
-  __shared__ int oobk[kMaxCuts];
-  __shared__ double sC[kMaxPairs];  // the Gram matrix, or the per-sample terms
-  __shared__ CutWalk walk[kMaxCuts];
+  __shared__ float2 center[G2MAX];
+  __shared__ double term[2][G2MAX * kRefineChunk];
   __shared__ RefineStateDev S;
-  __shared__ int maybe_out;
-  __shared__ uint32_t own_oob;
-  static_assert(kMaxPairs >= kMaxSamples, "sC holds the per-sample terms");
+  __shared__ uint32_t oob[G2MAX];
+  __shared__ int any_oob;
 
+  const int n_samples = ns.n, tid = threadIdx.x, G2 = grid_n * grid_n, nchunk = chunks_of(n_samples);
   // Workgroups are dealt to the 8 XCDs in turn, each XCD with its own L2:
-  // renumber them so that an XCD runs consecutive (grid point, marker)
-  // pairs, i.e. whole markers, and each marker's image area is fetched into
-  // one L2 only.
-  const int n_jobs = gridDim.y, tid = threadIdx.x;
-  int g, m;
+  // renumber them so that an XCD runs consecutive (chunks, marker) pairs,
+  // i.e. whole markers, and each marker's image area is fetched into one L2
+  // only.
+  const int n_jobs = gridDim.y;
+  int b, m;
   {
     const int n = gridDim.x * gridDim.y, hw = blockIdx.y * gridDim.x + blockIdx.x;
     const int x = hw % kXcds, k = hw / kXcds, q = n / kXcds, r = n % kXcds;
     const int logical = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + k;
-    g = logical % gridDim.x;
+    b = logical % gridDim.x;
     m = logical / gridDim.x;
   }
   const RefineJobDev& J = jobs[m];
-  if (it >= J.n_iter) return;
-  const int cb = it & 1;
-  if (fused) {
-    state_at(J, it, m, n_jobs, grid_n, W, S);
-    if (g == 0 && tid == 0) W.state[(size_t)cb * n_jobs + m] = S;
-  } else {
-    if (tid == 0) S = W.state[(size_t)cb * n_jobs + m];
-    __syncthreads();
-  }
-  if (!S.ok) return;
-  const int nc = J.n_cuts;
+  PointRecord rec;
+  load_records(it, m, n_jobs, n_samples, grid_n, W, rec);
+  const int k = tid / G2, g = tid - k * G2;  // the lane's cut and grid point
+  const float2 stop = J.stops[min(k, kMaxCuts - 1)];
+  const int nc = J.n_cuts, n_iter = J.n_iter;
   const Img im{J.quad, J.iw, J.ih};
-  RefineGridDev& GD = W.grid[((size_t)cb * n_jobs + m) * G2MAX + g];
-  // the homographies of grid points 0 .. g, lane p on point p (the block
-  // stores its own for the selection and the read-out)
-  if (tid <= g) {
+  const int c0 = b * per, c1 = min(nchunk, c0 + per);
+  const int width = G2 * kRefineChunk, buf = nc * width;
+  if (it >= n_iter) return;
+  state_at(J, it, n_samples, grid_n, rec, S);
+  if (b == 0 && tid == 0) W.state[(size_t)(it & 1) * n_jobs + m] = S;
+  if (!S.ok) return;
+  if (tid < G2) {
     float Hf[9], Hi[9], qx, qy;
     grid_homography(J, S.cx, S.cy, S.neighbour, tid, grid_n, Hf, Hi, qx, qy);
     for (int r = 0; r < 9; ++r) {
       gH[tid][r] = Hf[r];
       gHi[tid][r] = Hi[r];
     }
-    if (tid == g) {
+    center[tid] = make_float2(qx, qy);
+    oob[tid] = 0;
+    if (b == 0 && it + 1 == J.n_iter) {  // the read-out's, should this point be chosen
+      RefineHomDev& GH = W.hom[(size_t)m * G2MAX + tid];
       for (int r = 0; r < 9; ++r) {
-        GD.H[r] = Hf[r];
-        GD.Hi[r] = Hi[r];
+        GH.H[r] = Hf[r];
+        GH.Hi[r] = Hi[r];
       }
-      GD.gx = qx;
-      GD.gy = qy;
     }
   }
-  if (tid < kMaxCuts) oobk[tid] = 0;
-  if (tid == 0) maybe_out = g > 0 && !J.box_inside;
+  if (tid == blockDim.x - 1) any_oob = 0;
   __syncthreads();
-  const float* sH = gH[g];
-  if (tid < nc) cut_walk_starts(gHi[g], J.stops[tid], J.begin_sig, J.end_sig, n_samples, walk[tid]);
-  // may a valid cut leave the image at a grid point before this one?
-  if (J.box_inside) {
-    for (int p = tid; p < g * nc; p += kRefineBlock) {
-      const int gp = p / nc, k = p - gp * nc;
-      if (!((S.sticky >> k) & 1u) &&
-          !cut_surely_inside(gH[gp], gHi[gp], J.stops[k], J.begin_sig, J.end_sig, J.iw, J.ih))
-        maybe_out = 1;
+  // place the cut, and walk it to the block's first chunk
+  float H[9];
+  float2 p = make_float2(0.f, 0.f), step = p;
+  bool on = k < nc, inside = false;
+  if (on) {
+    float Hi[9];
+    for (int r = 0; r < 9; ++r) {
+      H[r] = gH[g][r];
+      Hi[r] = gHi[g][r];
+    }
+    CutPlace at = cut_place(H, Hi, stop, J.begin_sig, J.end_sig, J.iw, J.ih);
+    inside = at == kInside;
+    if (at == kUnsure && samples_leave(im, H, Hi, stop, J.begin_sig, J.end_sig, ns)) at = kOutside;
+    if (at == kOutside) {
+      atomicOr(&oob[g], 1u << k);
+      any_oob = 1;
+      on = false;
+    } else {
+      cut_walk_begin(Hi, stop, J.begin_sig, J.end_sig, ns, p, step);
+      for (int q = 0; q < c0; ++q) {
+#pragma unroll
+        for (int t = 0; t < kRefineChunk; ++t) {
+          p.x += step.x;
+          p.y += step.y;
+        }
+      }
     }
   }
-  __syncthreads();
-  const int nchunk = (n_samples + kRefineChunk - 1) / kRefineChunk;
-  for (int w = tid; w < nc * nchunk; w += kRefineBlock) {
-    const int k = w / nchunk, c = w - k * nchunk;
-    if (sample_chunk(im, sH, walk[k], n_samples, c, sig[k])) atomicOr(&oobk[k], 1);
-  }
-  __syncthreads();
-  if (tid < 64) {
-    const uint32_t o = (uint32_t)__ballot(tid < nc && oobk[tid] != 0);
-    if (tid == 0) own_oob = o;
-  }
-  __syncthreads();
-  const uint32_t oob = own_oob;
-  const uint32_t valid = ~(S.sticky | oob) & cut_bits(nc);
-  const int mv = __popc(valid);
-  if (!maybe_out) {
-    // the valid cuts are known: per sample, sum and sum of squares over them
-    // in cut order (read kRowBatch cuts at a time, indices clamped, so the
-    // reads are in flight together), then the terms summed in a fixed order
-    for (int i = tid; i < n_samples; i += kRefineBlock) {
-      double s1 = 0.0, s2 = 0.0;
+  // the cuts flagged by grid point q: before the iteration, at q or before it
+  auto flags = [&](int q) {
+    uint32_t f = S.sticky;
+    if (any_oob)
+      for (int r = 0; r <= q; ++r) f |= oob[r];
+    return f;
+  };
+  auto chunk_sum = [&](int c) {  // lane g: grid point g's share of chunk c
+    const double* v = &term[c & 1][tid * kRefineChunk];
+    double* out = W.part + (((size_t)(it & 1) * n_jobs + m) * G2MAX + tid) * kMaxRefineSums +
+                  c * (kRefineChunk / kSumChunk);
+#pragma unroll
+    for (int t0 = 0; t0 < kRefineChunk; t0 += kSumChunk) {
+      double sum = 0.0;
+#pragma unroll
+      for (int t = t0; t < t0 + kSumChunk; ++t)
+        if (c * kRefineChunk + t < n_samples) sum += v[t];
+      if (c * kRefineChunk + t0 < n_samples) out[t0 / kSumChunk] = sum;
+    }
+  };
+  uint32_t valid = 0;
+  for (int c = c0; c < c1; ++c) {
+    float* sig = sig_lds + (per > 1 ? (c & 1) * buf : 0);
+    if (on) {
+      const int live = n_samples - c * kRefineChunk;
+      float val[kRefineChunk];
+      if (inside && live >= kRefineChunk) sample_inside(im, H, p, step, val);
+      else sample_any<kRefineChunk, 1>(im, H, p, step, live, val);
+      float* out = sig + tid * kRefineChunk;  // (cut, grid point) = lane
+#pragma unroll
+      for (int t = 0; t < kRefineChunk; ++t) out[t] = val[t];
+    }
+    __syncthreads();
+    if (c > c0 && tid < G2) chunk_sum(c - 1);
+    // lanes 2w and 2w + 1: sum and sum of squares at (grid point, sample) w
+    // over the valid cuts, in cut order, kRowBatch reads in flight
+    constexpr int kRowBatch = 8;
+    const int w = tid >> 1;
+    const bool squares = tid & 1;
+    if (c == c0) valid = ~flags(min(w / kRefineChunk, G2 - 1)) & cut_bits(nc);
+    if (w < width) {
+      double s = 0.0;
       for (int k0 = 0; k0 < nc; k0 += kRowBatch) {
         float v[kRowBatch];
 #pragma unroll
-        for (int j = 0; j < kRowBatch; ++j) v[j] = sig[min(k0 + j, nc - 1)][i];
+        for (int j = 0; j < kRowBatch; ++j) v[j] = sig[min(k0 + j, nc - 1) * width + w];
 #pragma unroll
-        for (int j = 0; j < kRowBatch; ++j) {
+        for (int j = 0; j < kRowBatch; ++j)
           if (k0 + j < nc && ((valid >> (k0 + j)) & 1u)) {
             const double d = (double)v[j];
-            s1 += d;
-            s2 += d * d;
+            s += squares ? d * d : d;
+          }
+      }
+      const double other = __shfl_xor(s, 1, 64);
+      if (squares) term[c & 1][w] = (double)__popc(valid) * s - other * other;
+    }
+  }
+  __syncthreads();
+  if (tid < G2) chunk_sum(c1 - 1);
+  if (b == 0 && tid < G2)
+    W.points[((size_t)(it & 1) * n_jobs + m) * G2MAX + tid] =
+        RefinePointDev{center[tid].x, center[tid].y, flags(tid), 0u};
+}
+
+// The whole search in one block per marker (at most `iters` iterations; the
+// coarse step is one, its centres go to `centers`).  A lane owns one chunk of
+// kSumChunk samples at one grid point, the grid points side by side as in
+// k_refine_iter, and keeps the sums over the cuts in registers, so no sample
+// goes through LDS; B >= grid_n^2 * sum chunks.  The cuts' running sums are
+// laid out kSearchCuts cuts at a time, which bounds their LDS.
+constexpr int kSearchCuts = 6;
+
+template <int B>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_refine_search(
+    const RefineJobDev* __restrict__ jobs, Samples ns, int grid_n, int iters, RefineWork W,
+    float* __restrict__ centers) {
+  __shared__ float2 start[kSearchCuts][kMaxSumChunks][G2MAX], step[kSearchCuts][G2MAX];
+  __shared__ double part[G2MAX][kMaxSumChunks];
+  __shared__ float gH[G2MAX][9], gHi[G2MAX][9];
+  __shared__ float2 center[G2MAX];
+  __shared__ uint32_t oob[G2MAX], unsure[G2MAX];
+  __shared__ int any_unsure, any_oob;
+  __shared__ RefineStateDev S;
+  const int m = blockIdx.x, n_jobs = gridDim.x, tid = threadIdx.x, n_samples = ns.n;
+  const RefineJobDev& J = jobs[m];
+  const int n_iter = min(J.n_iter, iters), nc = J.n_cuts, G2 = grid_n * grid_n;
+  const Img im{J.quad, J.iw, J.ih};
+  const int nchunk = sum_chunks_of(n_samples);
+  const int c = tid / G2, g = tid - c * G2;  // the lane's chunk and grid point
+  const bool on = c < nchunk;
+  const int live = n_samples - c * kSumChunk;
+  if (tid == 0) S = first_state(J);
+  __syncthreads();
+  for (int it = 0; it < n_iter; ++it) {
+    if (tid < G2) {
+      float Hf[9], Hi[9], qx, qy;
+      grid_homography(J, S.cx, S.cy, S.neighbour, tid, grid_n, Hf, Hi, qx, qy);
+      for (int r = 0; r < 9; ++r) {
+        gH[tid][r] = Hf[r];
+        gHi[tid][r] = Hi[r];
+      }
+      center[tid] = make_float2(qx, qy);
+      oob[tid] = 0;
+      unsure[tid] = 0;
+    }
+    if (tid == B - 1) any_unsure = any_oob = 0;
+    __syncthreads();
+    for (int p = tid; p < G2 * nc; p += B) {
+      const int k = p / G2, gp = p - k * G2;
+      const CutPlace at = cut_place(gH[gp], gHi[gp], J.stops[k], J.begin_sig, J.end_sig, J.iw, J.ih);
+      if (at == kUnsure) {
+        atomicOr(&unsure[gp], 1u << k);
+        any_unsure = 1;
+      }
+      if (at == kOutside ||
+          (at == kUnsure &&
+           samples_leave(im, gH[gp], gHi[gp], J.stops[k], J.begin_sig, J.end_sig, ns))) {
+        atomicOr(&oob[gp], 1u << k);
+        any_oob = 1;
+      }
+    }
+    __syncthreads();
+    // the cuts flagged by grid point q: before the iteration, at q or before it
+    auto flags = [&](int q) {
+      uint32_t f = S.sticky;
+      if (any_oob)
+        for (int r = 0; r <= q; ++r) f |= oob[r];
+      return f;
+    };
+    uint32_t valid = 0, slow = 0;
+    float H[9];
+    if (on) {
+      valid = ~flags(g) & cut_bits(nc);
+      slow = live < kSumChunk ? ~0u : any_unsure ? unsure[g] : 0u;
+      for (int r = 0; r < 9; ++r) H[r] = gH[g][r];
+    }
+    double s1[kSumChunk], s2[kSumChunk];
+#pragma unroll
+    for (int t = 0; t < kSumChunk; ++t) s1[t] = s2[t] = 0.0;
+    for (int k0 = 0; k0 < nc; k0 += kSearchCuts) {
+      const int nk = min(kSearchCuts, nc - k0);
+      for (int p = tid; p < G2 * nk; p += B) {
+        const int k = p / G2, gp = p - k * G2;
+        float2 q, d;
+        cut_walk_begin(gHi[gp], J.stops[k0 + k], J.begin_sig, J.end_sig, ns, q, d);
+        for (int cc = 0; cc < nchunk; ++cc) {
+          start[k][cc][gp] = q;
+#pragma unroll
+          for (int t = 0; t < kSumChunk; ++t) {
+            q.x += d.x;
+            q.y += d.y;
+          }
+        }
+        step[k][gp] = d;
+      }
+      __syncthreads();
+      if (on) {
+        for (int k = 0; k < nk; ++k) {
+          if (!((valid >> (k0 + k)) & 1u)) continue;
+          float2 p = start[k][c][g];
+          float val[kSumChunk];
+          if (!((slow >> (k0 + k)) & 1u)) sample_inside(im, H, p, step[k][g], val);
+          else sample_any<kSumChunk, 1>(im, H, p, step[k][g], live, val);
+#pragma unroll
+          for (int t = 0; t < kSumChunk; ++t) {
+            const double d = (double)val[t];
+            s1[t] += d;
+            s2[t] += d * d;
           }
         }
       }
-      sC[i] = (double)mv * s2 - s1 * s1;
+      __syncthreads();
+    }
+    if (on) {
+      const double mv = (double)__popc(valid);
+      double sum = 0.0;
+#pragma unroll
+      for (int t = 0; t < kSumChunk; ++t)
+        if (t < live) sum += mv * s2[t] - s1[t] * s1[t];
+      part[g][c] = sum;
     }
     __syncthreads();
     if (tid < 64) {
-      double part = 0.0;
-      for (int i = tid; i < n_samples; i += 64) part += sC[i];
-      const double sum = wave_sum(part);
-      if (tid == 0) {
-        GD.cost_local = sum;
-        GD.m_local = (int16_t)mv;
-        GD.has_gram = 0;
-        GD.oob = oob;
-      }
+      const int q = tid < G2 ? tid : 0;
+      const RefineStateDev prev = S;
+      const uint32_t f = flags(q);
+      const float res = point_residual(part[q], nchunk, __popc(~f & cut_bits(nc)));
+      select_state(tid < G2, res, center[q].x, center[q].y, __shfl(f, G2 - 1, 64), prev, grid_n, S);
+    }
+    __syncthreads();
+    if (!S.ok) break;
+  }
+  if (centers) {
+    if (tid == 0) {
+      const bool moved = n_iter >= 1 && S.ok;
+      centers[2 * m] = moved ? S.cx : J.c0x;
+      centers[2 * m + 1] = moved ? S.cy : J.c0y;
     }
     return;
   }
-  double* C = W.gram + (((size_t)cb * n_jobs + m) * G2MAX + g) * kMaxPairs;
-  const int npairs = nc * (nc + 1) / 2;
-  for (int q = tid; q < npairs; q += kRefineBlock) {
-    int k = 0, r = q;
-    while (r >= nc - k) {
-      r -= nc - k;
-      ++k;
-    }
-    const int l = k + r;
-    double acc = 0.0;
-    for (int i = 0; i < n_samples; ++i) acc += (double)sig[k][i] * (double)sig[l][i];
-    C[q] = acc;
-    sC[q] = acc;
+  if (tid == 0) W.state[(size_t)(J.n_iter & 1) * n_jobs + m] = S;
+  if (n_iter > 0 && S.ok && tid < 9) {
+    RefineHomDev& GH = W.hom[(size_t)m * G2MAX + S.best_g];
+    GH.H[tid] = gH[S.best_g][tid];
+    GH.Hi[tid] = gHi[S.best_g][tid];
   }
-  __syncthreads();
-  // residual of this grid point if no earlier grid point of the iteration
-  // flags another cut (the selection checks that and recomputes otherwise)
-  if (tid < 64) {
-    const double part = tid < nc ? gram_row(sC, valid, tid, nc, mv) : 0.0;
-    const double sum = wave_sum(part);
-    if (tid == 0) {
-      GD.cost_local = sum;
-      GD.m_local = (int16_t)mv;
-      GD.has_gram = 1;
-      GD.oob = oob;
-    }
-  }
-}
-
-// The state a marker starts iteration it + 1 with (after k_refine_iter of
-// iteration it), one block per marker; k_refine_init gives iteration 0's.
-__global__ __launch_bounds__(kRefineBlock) void k_refine_pick(const RefineJobDev* __restrict__ jobs,
-                                                              int it, int grid_n, RefineWork W) {
-  __shared__ RefineStateDev S;
-  const int m = blockIdx.x, n_jobs = gridDim.x;
-  const RefineJobDev& J = jobs[m];
-  if (it + 1 > J.n_iter) return;
-  state_at(J, it + 1, m, n_jobs, grid_n, W, S);
-  if (threadIdx.x == 0) W.state[(size_t)((it + 1) & 1) * n_jobs + m] = S;
-}
-
-__global__ __launch_bounds__(kRefineBlock) void k_refine_init(const RefineJobDev* __restrict__ jobs,
-                                                              int grid_n, RefineWork W) {
-  __shared__ RefineStateDev S;
-  const int m = blockIdx.x;
-  state_at(jobs[m], 0, m, gridDim.x, grid_n, W, S);
-  if (threadIdx.x == 0) W.state[m] = S;
 }
 
 // Signals at the last iteration's best grid point, then the per-cut
@@ -862,18 +1022,18 @@ __global__ __launch_bounds__(kRefineBlock) void k_refine_init(const RefineJobDev
 // there.  Signals, median profile, orazio statistics, distance to every
 // bank profile.
 __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
-    const RefineJobDev* __restrict__ jobs, int n_samples, int grid_n,
+    const RefineJobDev* __restrict__ jobs, Samples ns, int grid_n,
     const float* __restrict__ inv_ratio, int bank_rows, int bank_cols, RefineWork W,
     const float* __restrict__ given_H, const float* __restrict__ given_c,
-    const double* __restrict__ given_cost, RefineOutDev* __restrict__ out,
+    const double* __restrict__ given_cost, int searched, RefineOutDev* __restrict__ out,
     float* __restrict__ dist) {
+  const int n_samples = ns.n;
   __shared__ float sig[kMaxCuts][kMaxSamples + 1];
   __shared__ float ordered[kMaxSamples][kMaxCuts];  // per sample, the valid cuts' values sorted
   __shared__ float bar[kMaxSamples];
   __shared__ int valid_cut[kMaxCuts];
   __shared__ int n_valid;
   __shared__ int oob_at[kMaxCuts];
-  __shared__ CutWalk walk[kMaxCuts];
   __shared__ float sH[9], sHi[9];
   __shared__ float stat_mub[kMaxCuts], stat_muw[kMaxCuts], stat_var[kMaxCuts];
   __shared__ float xs[kMaxSamples];
@@ -908,12 +1068,18 @@ __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
     __syncthreads();
   } else {
     // the selection after the last iteration
-    state_at(J, J.n_iter, m, n_jobs, grid_n, W, S);
+    if (!searched) {
+      PointRecord rec;
+      load_records(J.n_iter, m, n_jobs, n_samples, grid_n, W, rec);
+      state_at(J, J.n_iter, n_samples, grid_n, rec, S);
+    } else {
+      if (tid == 0) S = W.state[(size_t)(J.n_iter & 1) * n_jobs + m];
+      __syncthreads();
+    }
     if (S.ok && tid < 9) {
-      const RefineGridDev& GB =
-          W.grid[((size_t)((J.n_iter - 1) & 1) * n_jobs + m) * G2MAX + S.best_g];
-      sH[tid] = GB.H[tid];
-      sHi[tid] = GB.Hi[tid];
+      const RefineHomDev& GH = W.hom[(size_t)m * G2MAX + S.best_g];
+      sH[tid] = GH.H[tid];
+      sHi[tid] = GH.Hi[tid];
     }
     __syncthreads();
   }
@@ -922,12 +1088,20 @@ __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
     return;
   }
   const Img im{J.quad, J.iw, J.ih};
-  if (tid < nc) cut_walk_starts(sHi, J.stops[tid], J.begin_sig, J.end_sig, n_samples, walk[tid]);
-  __syncthreads();
-  const int nchunk = (n_samples + kRefineChunk - 1) / kRefineChunk;
+  const int nchunk = chunks_of(n_samples);
   for (int w = tid; w < nc * nchunk; w += kFinalBlock) {
-    const int k = w / nchunk, c = w - k * nchunk;
-    if (sample_chunk(im, sH, walk[k], n_samples, c, sig[k]) && given) atomicOr(&oob_at[k], 1);
+    const int c = w / nc, k = w - c * nc, live = n_samples - c * kRefineChunk;
+    float2 p, step;
+    cut_walk_begin(sHi, J.stops[k], J.begin_sig, J.end_sig, ns, p, step);
+    for (int q = 0; q < c * kRefineChunk; ++q) {
+      p.x += step.x;
+      p.y += step.y;
+    }
+    float val[kRefineChunk];
+    if (sample_any<kRefineChunk, kRefineChunk>(im, sH, p, step, live, val) && given) atomicOr(&oob_at[k], 1);
+#pragma unroll
+    for (int t = 0; t < kRefineChunk; ++t)
+      if (t < live) sig[k][c * kRefineChunk + t] = val[t] / 2;
   }
   __syncthreads();
   // The outputs live in host memory: they are stored after the last
@@ -1115,29 +1289,89 @@ __global__ __launch_bounds__(64) void k_take_stops(const RefineJobDev* __restric
 }
 
 // The centre the grid search moves to after its first iteration (the job's
-// start when that iteration found no readable grid point).
-__global__ __launch_bounds__(256) void k_refine_coarse_out(const RefineJobDev* __restrict__ jobs,
-                                                           int n_jobs, RefineWork W,
-                                                           float* __restrict__ centers) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n_jobs) return;
+// start when that iteration found no readable grid point), a wavefront per
+// marker.
+__global__ __launch_bounds__(64) void k_refine_coarse_out(const RefineJobDev* __restrict__ jobs,
+                                                          int n_samples, int grid_n,
+                                                          RefineWork W,
+                                                          float* __restrict__ centers) {
+  __shared__ RefineStateDev S;
+  const int m = blockIdx.x;
   const RefineJobDev& J = jobs[m];
-  const RefineStateDev& S = W.state[(size_t)n_jobs + m];  // parity of iteration 1
-  const bool moved = J.n_iter >= 1 && S.ok;
-  centers[2 * m] = moved ? S.cx : J.c0x;
-  centers[2 * m + 1] = moved ? S.cy : J.c0y;
+  const bool searched = J.n_iter >= 1;
+  PointRecord rec;
+  load_records(searched ? 1 : 0, m, gridDim.x, n_samples, grid_n, W, rec);
+  state_at(J, searched ? 1 : 0, n_samples, grid_n, rec, S);
+  if (threadIdx.x == 0) {
+    const bool moved = searched && S.ok;
+    centers[2 * m] = moved ? S.cx : J.c0x;
+    centers[2 * m + 1] = moved ? S.cy : J.c0y;
+  }
+}
+
+Samples samples(int n) { return Samples{n, 1.0 / (double)(n - 1)}; }
+
+// The launches of one search: a lane per cut and grid point, the chunks'
+// sample buffers in dynamic LDS.
+struct SearchShape {
+  int per;      // chunks per block
+  int block;
+  size_t lds;
+};
+SearchShape search_shape(int max_cuts, int grid_n, int per) {
+  const int cuts = std::min(std::max(max_cuts, 1), kMaxCuts), g2 = grid_n * grid_n;
+  const int lanes = std::max(g2 * cuts, 2 * g2 * kRefineChunk);
+  return SearchShape{per, (lanes + 63) / 64 * 64,
+                     sizeof(float) * (per > 1 ? 2 : 1) * cuts * g2 * kRefineChunk};
+}
+
+void launch_iteration(const RefineJobDev* jobs, int n_jobs, int it, const SearchShape& sh,
+                      int n_samples, int grid_n, const RefineWork& work, hipStream_t s) {
+  const dim3 grid((chunks_of(n_samples) + sh.per - 1) / sh.per, n_jobs);
+  k_refine_iter<<<grid, sh.block, sh.lds, s>>>(jobs, it, sh.per, samples(n_samples), grid_n, work);
+}
+
+// Markers from which k_refine_search takes over (22 cuts of 100 samples, 9
+// iterations and the read-out, k_refine_iter against k_refine_search: 128
+// markers 271 / 303 us, 160 markers 320 / 306, 256 markers 381 / 324).
+constexpr int kSearchMinJobs = 150;
+// Chunks per block: as few as keep an iteration's blocks within two per CU
+// (a third of nine wavefronts does not fit beside them; 100 markers 307 us
+// with one chunk, 219 with two; 48 markers 158 / 166).
+constexpr int kIterBlocks = 512;
+int chunks_per_block(int n_jobs, int n_samples) {
+  const int nchunk = chunks_of(n_samples);
+  int per = 1;
+  while (per < nchunk && (long long)n_jobs * ((nchunk + per - 1) / per) > kIterBlocks) ++per;
+  return per;
+}
+
+constexpr int kSearchBlock = 512, kSearchBlockWide = 704;
+static_assert(G2MAX * kMaxSumChunks <= kSearchBlockWide, "a lane per grid point and chunk");
+
+void launch_search(const RefineJobDev* jobs, int n_jobs, int n_samples, int grid_n, int iters,
+                   const RefineWork& work, float* centers, hipStream_t s) {
+  const Samples ns = samples(n_samples);
+  if (grid_n * grid_n * sum_chunks_of(n_samples) <= kSearchBlock)
+    k_refine_search<kSearchBlock><<<n_jobs, kSearchBlock, 0, s>>>(jobs, ns, grid_n, iters, work,
+                                                                  centers);
+  else
+    k_refine_search<kSearchBlockWide><<<n_jobs, kSearchBlockWide, 0, s>>>(jobs, ns, grid_n, iters,
+                                                                          work, centers);
 }
 
 }  // namespace
 
-int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int n_samples, int grid_n,
-                         const RefineWork& work, float* centers, hipStream_t s) {
+int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int max_cuts, int n_samples,
+                         int grid_n, const RefineWork& work, float* centers, hipStream_t s) {
   if (n_jobs <= 0) return 0;
-  const dim3 grid(grid_n * grid_n, n_jobs);
-  k_refine_init<<<n_jobs, kRefineBlock, 0, s>>>(jobs, grid_n, work);
-  k_refine_iter<<<grid, kRefineBlock, 0, s>>>(jobs, 0, n_samples, grid_n, 0, work);
-  k_refine_pick<<<n_jobs, kRefineBlock, 0, s>>>(jobs, 0, grid_n, work);
-  k_refine_coarse_out<<<(n_jobs + 255) / 256, 256, 0, s>>>(jobs, n_jobs, work, centers);
+  if (n_jobs >= kSearchMinJobs) {
+    launch_search(jobs, n_jobs, n_samples, grid_n, 1, work, centers, s);
+  } else {
+    const SearchShape sh = search_shape(max_cuts, grid_n, chunks_per_block(n_jobs, n_samples));
+    launch_iteration(jobs, n_jobs, 0, sh, n_samples, grid_n, work, s);
+    k_refine_coarse_out<<<n_jobs, 64, 0, s>>>(jobs, n_samples, grid_n, work, centers);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -1146,8 +1380,8 @@ int launch_refine_readout(const RefineJobDev* jobs, int n_jobs, int n_samples, c
                           int bank_rows, int bank_cols, const RefineWork& work, RefineOutDev* out,
                           float* dist, hipStream_t s) {
   if (n_jobs <= 0) return 0;
-  k_refine_final<<<n_jobs, kFinalBlock, 0, s>>>(jobs, n_samples, kMaxGrid, inv_ratio, bank_rows,
-                                                 bank_cols, work, H, centers, cost, out, dist);
+  k_refine_final<<<n_jobs, kFinalBlock, 0, s>>>(jobs, samples(n_samples), kMaxGrid, inv_ratio, bank_rows,
+                                                 bank_cols, work, H, centers, cost, 0, out, dist);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
@@ -1165,21 +1399,21 @@ int launch_select_cuts(const SelectJobDev* jobs, int n_jobs, const float4* pts, 
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int n_samples, int grid_n,
-                  const float* inv_ratio, int bank_rows, int bank_cols, const RefineWork& work,
+int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int max_cuts, int n_samples,
+                  int grid_n, const float* inv_ratio, int bank_rows, int bank_cols, const RefineWork& work,
                   RefineOutDev* out, float* dist, hipStream_t s) {
   if (n_jobs <= 0) return 0;
-  const dim3 grid(grid_n * grid_n, n_jobs);
-  const int fused = grid.x * grid.y <= kFuseMaxBlocks;
-  if (!fused) k_refine_init<<<n_jobs, kRefineBlock, 0, s>>>(jobs, grid_n, work);
-  for (int it = 0; it < max_iter; ++it) {
-    k_refine_iter<<<grid, kRefineBlock, 0, s>>>(jobs, it, n_samples, grid_n, fused, work);
-    if (!fused && it + 1 < max_iter)
-      k_refine_pick<<<n_jobs, kRefineBlock, 0, s>>>(jobs, it, grid_n, work);
+  const int searched = n_jobs >= kSearchMinJobs;
+  if (searched) {
+    launch_search(jobs, n_jobs, n_samples, grid_n, max_iter, work, nullptr, s);
+  } else {
+    const SearchShape sh = search_shape(max_cuts, grid_n, chunks_per_block(n_jobs, n_samples));
+    for (int it = 0; it < max_iter; ++it)
+      launch_iteration(jobs, n_jobs, it, sh, n_samples, grid_n, work, s);
   }
-  k_refine_final<<<n_jobs, kFinalBlock, 0, s>>>(jobs, n_samples, grid_n, inv_ratio, bank_rows,
-                                                 bank_cols, work, nullptr, nullptr, nullptr, out,
-                                                 dist);
+  k_refine_final<<<n_jobs, kFinalBlock, 0, s>>>(jobs, samples(n_samples), grid_n, inv_ratio, bank_rows,
+                                                 bank_cols, work, nullptr, nullptr, nullptr,
+                                                 searched, out, dist);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

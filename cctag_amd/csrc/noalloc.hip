@@ -1,7 +1,7 @@
 // The grid search of cctagx_refiner_grid as one call that allocates nothing
 // (include/cctag_amd.h, cctagx_refine_grid_static).  Every device buffer the
 // call needs -- the frame, its quad image, the jobs, the grid search's
-// per-marker state, grid records and Gram matrices, the read-out's outputs
+// per-marker state, grid records and homographies, the read-out's outputs
 // -- lives in `scratch`, a fixed array of device memory that each GPU holds
 // from the library's load until the process ends.  Host code reaches it
 // through the address hipGetSymbolAddress returns on that device; the
@@ -34,12 +34,13 @@ constexpr size_t kImg = 0;
 constexpr size_t kQuad = up256(kImg + kMaxPixels);
 constexpr size_t kJobs = up256(kQuad + 4 * kMaxPixels);
 constexpr size_t kState = up256(kJobs + sizeof(RefineJobDev) * kMaxMarkers);
-constexpr size_t kGrid = up256(kState + sizeof(RefineStateDev) * 2 * kMaxMarkers);
-constexpr size_t kGram = up256(kGrid + sizeof(RefineGridDev) * 2 * kMaxMarkers * kG2);
-constexpr size_t kOut = up256(kGram + sizeof(double) * 2 * (size_t)kMaxMarkers * kG2 * kMaxPairs);
+constexpr size_t kPoints = up256(kState + sizeof(RefineStateDev) * 2 * kMaxMarkers);
+constexpr size_t kPart = up256(kPoints + sizeof(RefinePointDev) * 2 * kMaxMarkers * kG2);
+constexpr size_t kHom = up256(kPart + sizeof(double) * 2 * kMaxMarkers * kG2 * kMaxRefineSums);
+constexpr size_t kOut = up256(kHom + sizeof(RefineHomDev) * kMaxMarkers * kG2);
 constexpr size_t kDist = up256(kOut + sizeof(RefineOutDev) * kMaxMarkers);
 constexpr size_t kScratchBytes = up256(kDist + sizeof(float));
-static_assert(kScratchBytes <= 24309248, "the size the C ABI documents (24.3 MB)");
+static_assert(kScratchBytes <= 11400000, "the size the C ABI documents (11.4 MB)");
 
 constexpr int kMaxDevices = 64;
 
@@ -107,8 +108,9 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
   RefineJobDev* d_jobs = reinterpret_cast<RefineJobDev*>(base + kJobs);
   RefineWork work;
   work.state = reinterpret_cast<RefineStateDev*>(base + kState);
-  work.grid = reinterpret_cast<RefineGridDev*>(base + kGrid);
-  work.gram = reinterpret_cast<double*>(base + kGram);
+  work.points = reinterpret_cast<RefinePointDev*>(base + kPoints);
+  work.part = reinterpret_cast<double*>(base + kPart);
+  work.hom = reinterpret_cast<RefineHomDev*>(base + kHom);
   RefineOutDev* d_out = reinterpret_cast<RefineOutDev*>(base + kOut);
   float* d_dist = reinterpret_cast<float*>(base + kDist);
 
@@ -118,7 +120,7 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
   const IdentConstants kc = ident_constants(hp, std::vector<std::vector<float>>());
   RefineJobDev jobs[kMaxMarkers];
   int job_of[kMaxMarkers];
-  int n_jobs = 0, max_iter = 0;
+  int n_jobs = 0, max_iter = 0, max_cuts = 0;
   float mean_ab = 0.f;
   const std::vector<Pt2> no_stops;
   for (int i = 0; i < n; ++i) {
@@ -148,7 +150,6 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
       d.begin_sig = r.begin_sig;
       d.end_sig = r.end_sig;
       d.n_iter = r.n_iter;
-      d.box_inside = box_inside(r, width, height) ? 1 : 0;
       d.n_cuts = m.n_cuts;
       d.c0x = m.center0[0];
       d.c0y = m.center0[1];
@@ -156,6 +157,7 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
       d.sel_index = -1;
       for (int k = 0; k < m.n_cuts; ++k) d.stops[k] = make_float2(m.stops[k][0], m.stops[k][1]);
       max_iter = std::max(max_iter, r.n_iter);
+      max_cuts = std::max(max_cuts, d.n_cuts);
       job_of[i] = n_jobs++;
     } catch (const std::exception& ex) {
       set_error(std::string("marker ") + std::to_string(i) + ": " + ex.what());
@@ -169,7 +171,7 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
   RefineOutDev out[kMaxMarkers];
   if (n_jobs > 0) {
     CCTAGX_HIP(hipMemcpyAsync(d_jobs, jobs, sizeof(RefineJobDev) * n_jobs, hipMemcpyHostToDevice, s));
-    if (launch_refine(d_jobs, n_jobs, max_iter, kc.n_samples, hp.imaged_center_n_grid_sample,
+    if (launch_refine(d_jobs, n_jobs, max_iter, max_cuts, kc.n_samples, hp.imaged_center_n_grid_sample,
                       nullptr, 0, 0, work, d_out, d_dist, s))
       return CCTAGX_ERR_HIP;
     CCTAGX_HIP(hipMemcpyAsync(out, d_out, sizeof(RefineOutDev) * n_jobs, hipMemcpyDeviceToHost, s));

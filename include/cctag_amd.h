@@ -382,7 +382,7 @@ int cctagx_refiner_times(cctagx_refiner* r, float* descend_us, float* grid_us);
  * + cctagx_refiner_grid in one synchronous call that allocates nothing: the
  * frame (host memory, at most CCTAGX_STATIC_MAX_PIXELS pixels), its quad
  * image, up to CCTAGX_STATIC_MAX_MARKERS markers' jobs and the grid search's
- * state go into one fixed device array of the library (24.3 MB, held by every
+ * state go into one fixed device array of the library (11.4 MB, held by every
  * GPU the library runs on until the process ends); larger inputs return
  * CCTAGX_ERR_CAPACITY.  Runs on the current device's null stream and writes
  * the same centres (n x 2) and ok flags (n) as cctagx_refiner_grid.  All
