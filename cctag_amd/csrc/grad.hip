@@ -26,6 +26,7 @@ struct cctagx_refiner {
   IdentConstants kc{};
   hipStream_t stream = nullptr;
   int max_markers = 0, n = 0;
+  int max_cuts = 0;  // most cuts of a marker set
   int w = 0, h = 0;
   DeviceBuffer img, quad, jobs, H, cost, grad, centers, coarse, start, coarse_of;
   PinnedBuffer h_jobs, h_io;
@@ -61,6 +62,8 @@ int to_host(cctagx_refiner* r, T* dst, const DeviceBuffer& src, size_t count) {
   std::memcpy(dst, r->h_io.as<void>(), bytes);
   return 0;
 }
+
+GradSampling sampling(int fp64) { return fp64 ? GradSampling::fp64 : GradSampling::local; }
 
 void copy9(float* dst, const Mat3& m) {
   for (int i = 0; i < 3; ++i)
@@ -138,6 +141,7 @@ int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* ma
   GradJobDev* hj = r->h_jobs.as<GradJobDev>();
   r->rjobs.clear();
   r->rjob_of.assign(n, -1);
+  r->max_cuts = 0;
   bool have_mean_ab = false;
   float mean_ab = 0.f;
   for (int i = 0; i < n; ++i) {
@@ -162,6 +166,7 @@ int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* ma
       // a quarter of the grid search's first neighbourhood
       d.alpha0 = 0.25f * r->host.imaged_center_neighbour_size * std::max(e.a(), e.b());
       d.n_cuts = m.n_cuts;
+      r->max_cuts = std::max(r->max_cuts, m.n_cuts);
       d.c0x = m.center0[0];
       d.c0y = m.center0[1];
       std::vector<Pt2> stops;
@@ -198,7 +203,7 @@ int cctagx_refiner_cost_grad(cctagx_refiner* r, const float* H, int fp64, double
   if (!r || !H || !cost) return CCTAGX_ERR_ARG;
   if (!r->n) return CCTAGX_ERR_STATE;
   if (int rc = to_device(r, r->H, H, (size_t)9 * r->n)) return rc;
-  if (launch_grad_eval(r->jobs.as<GradJobDev>(), r->n, r->H.as<float>(), r->kc.n_samples, fp64 != 0,
+  if (launch_grad_eval(r->jobs.as<GradJobDev>(), r->n, r->H.as<float>(), r->max_cuts, r->kc.n_samples, fp64 != 0,
                        r->cost.as<double>(), grad ? r->grad.as<double>() : nullptr, r->stream))
     return CCTAGX_ERR_HIP;
   if (int rc = to_host(r, cost, r->cost, r->n)) return rc;
@@ -221,7 +226,7 @@ int cctagx_refiner_descend(cctagx_refiner* r, int steps, int fp64, float* center
   if (!r || steps < 1 || steps > 10000 || !centers || !cost) return CCTAGX_ERR_ARG;
   if (!r->n) return CCTAGX_ERR_STATE;
   CCTAGX_HIP(hipEventRecord(r->ev[0], r->stream));
-  if (launch_grad_descend(r->jobs.as<GradJobDev>(), r->n, steps, r->kc.n_samples, fp64 != 0,
+  if (launch_grad_descend(r->jobs.as<GradJobDev>(), r->n, steps, r->max_cuts, r->kc.n_samples, sampling(fp64),
                           nullptr, r->centers.as<float>(), r->cost.as<double>(), r->stream))
     return CCTAGX_ERR_HIP;
   CCTAGX_HIP(hipEventRecord(r->ev[1], r->stream));
@@ -248,7 +253,7 @@ int cctagx_refiner_refine(cctagx_refiner* r, int steps, int fp64, float* centers
   }
   if (launch_grad_start(r->jobs.as<GradJobDev>(), r->n, r->coarse_of.as<int>(), r->coarse.as<float>(),
                         r->start.as<float>(), r->stream) ||
-      launch_grad_descend(r->jobs.as<GradJobDev>(), r->n, steps, r->kc.n_samples, fp64 != 0,
+      launch_grad_descend(r->jobs.as<GradJobDev>(), r->n, steps, r->max_cuts, r->kc.n_samples, sampling(fp64),
                           r->start.as<float>(), r->centers.as<float>(), r->cost.as<double>(),
                           r->stream))
     return CCTAGX_ERR_HIP;

@@ -24,17 +24,23 @@ struct GradJobDev {
 
 // The quads of a w x h image (w, h >= 2) into quad (w * h words).
 int launch_quads(const uint8_t* img, int w, int h, uint32_t* quad, hipStream_t s);
-int launch_grad_eval(const GradJobDev* jobs, int n, const float* H, int n_samples, bool fp64,
-                     double* cost, double* grad, hipStream_t s);
+// max_cuts: the most cuts of a job.
+int launch_grad_eval(const GradJobDev* jobs, int n, const float* H, int max_cuts, int n_samples,
+                     bool fp64, double* cost, double* grad, hipStream_t s);
 int launch_grad_homography(const GradJobDev* jobs, int n, const float* centers, float* H,
                            hipStream_t s);
 // start (2 per marker) = coarse[coarse_of[m]] when coarse_of[m] >= 0, else
 // the job's c0.
 int launch_grad_start(const GradJobDev* jobs, int n, const int* coarse_of, const float* coarse,
                       float* start, hipStream_t s);
+// How the descent samples: in float at positions relative to the marker
+// (local), in float at image positions (image: the identification's), or in
+// double.
+enum class GradSampling { local, image, fp64 };
 // `steps` descent steps per marker from start (2 per marker) or, when start
 // is null, from the job's c0.
-int launch_grad_descend(const GradJobDev* jobs, int n, int steps, int n_samples, bool fp64,
-                        const float* start, float* centers, double* cost, hipStream_t s);
+int launch_grad_descend(const GradJobDev* jobs, int n, int steps, int max_cuts, int n_samples,
+                        GradSampling sampling, const float* start, float* centers, double* cost,
+                        hipStream_t s);
 
 }  // namespace cctagx

@@ -13,19 +13,22 @@
 //   C    = sum_i sum_{k<l valid} (s_ki - s_li)^2 / (m (m-1) / 2)
 //
 // (pi(w) = (w0/w2, w1/w2); a cut is valid when all its samples are inside
-// the image).  k_grad_eval runs the forward pass and the adjoint pass of one
-// marker per block: dC/ds_ki = 2 (m s_ki - S_i) / pairs with S_i the sum over
+// the image).  One block runs the forward pass and the adjoint pass of a
+// marker: dC/ds_ki = 2 (m s_ki - S_i) / pairs with S_i the sum over
 // valid cuts, lambda = Jpi(w)^T dC/dy, and
 //
 //   dC/dH = sum_k [ sum_i lambda_ki u_ki^T  -  H^-T Jpi(v_k)^T (H_{:,01}^T L_k) v_k^T ]
 //
 // with v_k = H^-1 p_k and L_k = sum_i t_i lambda_ki (the second term is the
-// dependence of the cut direction q_k on H).  The centre gradient chains
-// dC/dH with dH/dc of the closed form, evaluated in forward mode with dual
-// numbers.  Sample positions and interpolation run in T (float in
-// production, double for checking); every sum is in double.
+// dependence of the cut direction q_k on H).  What is asked for are
+// derivatives along directions of H: its free entries, or dH/dc of the closed
+// form (evaluated in forward mode with dual numbers) for the centre; each is
+// contracted cut by cut, without forming dC/dH.  Sample positions and
+// interpolation run in T (float in production, double for checking); every
+// sum is in double.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 
 #include "grad_device.hpp"
@@ -33,332 +36,478 @@
 namespace cctagx {
 namespace {
 
-// Dual number carrying d/dcx and d/dcy (forward mode).
-struct D2 {
-  double v, dx, dy;
+// A dual number carrying one derivative (forward mode).
+struct D1 {
+  double v, d;
 };
-__device__ __forceinline__ D2 dc(double v) { return D2{v, 0.0, 0.0}; }
-__device__ __forceinline__ D2 operator+(D2 a, D2 b) { return D2{a.v + b.v, a.dx + b.dx, a.dy + b.dy}; }
-__device__ __forceinline__ D2 operator-(D2 a, D2 b) { return D2{a.v - b.v, a.dx - b.dx, a.dy - b.dy}; }
-__device__ __forceinline__ D2 operator-(D2 a) { return D2{-a.v, -a.dx, -a.dy}; }
-__device__ __forceinline__ D2 operator*(D2 a, D2 b) {
-  return D2{a.v * b.v, a.dx * b.v + a.v * b.dx, a.dy * b.v + a.v * b.dy};
+__device__ __forceinline__ D1 dc(double v) { return D1{v, 0.0}; }
+__device__ __forceinline__ D1 operator+(D1 a, D1 b) { return D1{a.v + b.v, a.d + b.d}; }
+__device__ __forceinline__ D1 operator-(D1 a, D1 b) { return D1{a.v - b.v, a.d - b.d}; }
+__device__ __forceinline__ D1 operator-(D1 a) { return D1{-a.v, -a.d}; }
+__device__ __forceinline__ D1 operator*(D1 a, D1 b) {
+  return D1{a.v * b.v, a.d * b.v + a.v * b.d};
 }
-__device__ __forceinline__ D2 operator/(D2 a, D2 b) {
-  const double inv = 1.0 / b.v, r = a.v * inv;
-  return D2{r, (a.dx - r * b.dx) * inv, (a.dy - r * b.dy) * inv};
-}
-__device__ __forceinline__ D2 dsqrt(D2 a) {
-  const double r = sqrt(a.v), h = 0.5 / r;
-  return D2{r, a.dx * h, a.dy * h};
+__device__ __forceinline__ D1 operator*(double a, D1 b) { return D1{a * b.v, a * b.d}; }
+__device__ __forceinline__ D1 dsqrt(D1 a) {
+  const double r = sqrt(a.v);
+  return D1{r, a.d * (0.5 / r)};
 }
 
-// Closed-form homography of the ellipse's canonic form and an imaged centre
-// (Identification.cpp:739-798), in double with derivatives w.r.t. (cx, cy).
-__device__ void closed_form(const GradJobDev& J, double cx, double cy, D2 H[9]) {
-  const D2 x{cx, 1.0, 0.0}, y{cy, 0.0, 1.0};
+__device__ __forceinline__ D1 pick(bool first, D1 a, D1 b) {
+  return D1{first ? a.v : b.v, first ? a.d : b.d};
+}
+
+// Entry (row, col) of the closed-form homography of the ellipse's canonic
+// form and an imaged centre (Identification.cpp:739-798), in double with the
+// derivative along cx (along_y false) or cy, in image coordinates relative
+// to (ox, oy).
+__device__ D1 closed_form(const GradJobDev& J, double cx, double cy, int row, int col, bool along_y,
+                          double ox, double oy) {
+  const D1 x{cx, along_y ? 0.0 : 1.0}, y{cy, along_y ? 1.0 : 0.0};
   const float* T = J.t_can;
-  const D2 u = dc(T[0]) * x + dc(T[1]) * y + dc(T[2]);
-  const D2 v = dc(T[3]) * x + dc(T[4]) * y + dc(T[5]);
-  const D2 w = dc(T[6]) * x + dc(T[7]) * y + dc(T[8]);
-  const D2 xc = u / w, yc = v / w;
-  const D2 Q11 = dc(J.Q11), Q22 = dc(J.Q22), Q33 = dc(J.Q33);
-  D2 Hc[9] = {Q33, Q22 * xc * yc, -(Q33 * xc),
-              dc(0.0), -(Q11 * xc * xc) - Q33, -(Q33 * yc),
-              -(Q11 * xc), Q22 * yc, -Q33};
-  const D2 d0 = dsqrt(Q22 * Q33 / Q11 * (Q11 * xc * xc + Q22 * yc * yc + Q33));
-  const D2 d1 = Q33;
-  const D2 d2 = dsqrt(-(Q22 * (Q11 * xc * xc + Q33)));
-  for (int r = 0; r < 3; ++r) {
-    Hc[r * 3 + 0] = Hc[r * 3 + 0] * d0;
-    Hc[r * 3 + 1] = Hc[r * 3 + 1] * d1;
-    Hc[r * 3 + 2] = Hc[r * 3 + 2] * d2;
-  }
+  const D1 u = (double)T[0] * x + (double)T[1] * y + dc(T[2]);
+  const D1 v = (double)T[3] * x + (double)T[4] * y + dc(T[5]);
+  const D1 w = (double)T[6] * x + (double)T[7] * y + dc(T[8]);
+  const double iw = 1.0 / w.v;
+  const D1 rw{iw, -w.d * iw * iw};
+  const D1 xc = u * rw, yc = v * rw;
+  const double Q11 = J.Q11, Q22 = J.Q22, Q33 = J.Q33;
+  const D1 f = Q11 * xc * xc;
+  // the entry's column of the canonic homography, scaled by its diagonal
+  // (all three laid out and one picked: one square root, and no branch -- a
+  // branch per column left the last entry of the third one unset)
+  const D1 c0[3] = {dc(Q33), dc(0.0), -(Q11 * xc)};
+  const D1 c1[3] = {Q22 * xc * yc, -f - dc(Q33), Q22 * yc};
+  const D1 c2[3] = {-(Q33 * xc), -(Q33 * yc), dc(-Q33)};
+  const D1 r0 = (Q22 * Q33 * (1.0 / Q11)) * (f + Q22 * yc * yc + dc(Q33));
+  const D1 r2 = -(Q22 * (f + dc(Q33)));
+  const D1 root = dsqrt(pick(col == 0, r0, r2));
+  const D1 scale = pick(col == 1, dc(Q33), root);
+  D1 h[3];
+  for (int j = 0; j < 3; ++j) h[j] = pick(col == 0, c0[j], pick(col == 1, c1[j], c2[j]));
   const float* Ti = J.t_inv_can;
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-      H[i * 3 + j] = dc(Ti[i * 3 + 0]) * Hc[0 * 3 + j] + dc(Ti[i * 3 + 1]) * Hc[1 * 3 + j] +
-                     dc(Ti[i * 3 + 2]) * Hc[2 * 3 + j];
+  const double o = row == 0 ? ox : row == 1 ? oy : 0.0;
+  D1 e = dc(0.0);
+  for (int j = 0; j < 3; ++j) e = e + ((double)Ti[row * 3 + j] - o * (double)Ti[6 + j]) * (h[j] * scale);
+  return e;
 }
 
-__device__ bool inverse3d(const double* m, double* out) {
-  const double c00 = m[4] * m[8] - m[5] * m[7], c01 = m[5] * m[6] - m[3] * m[8],
-               c02 = m[3] * m[7] - m[4] * m[6];
-  const double det = m[0] * c00 + m[1] * c01 + m[2] * c02;
-  if (!(det != 0.0) || !isfinite(det)) return false;
-  const double id = 1.0 / det;
-  out[0] = c00 * id;
-  out[1] = (m[2] * m[7] - m[1] * m[8]) * id;
-  out[2] = (m[1] * m[5] - m[2] * m[4]) * id;
-  out[3] = c01 * id;
-  out[4] = (m[0] * m[8] - m[2] * m[6]) * id;
-  out[5] = (m[2] * m[3] - m[0] * m[5]) * id;
-  out[6] = c02 * id;
-  out[7] = (m[1] * m[6] - m[0] * m[7]) * id;
-  out[8] = (m[0] * m[4] - m[1] * m[3]) * id;
-  return true;
+// Entry (row, col) of the adjugate of a row-major 3x3 matrix.
+__device__ __forceinline__ double adjugate(const double* m, int row, int col) {
+  const int i1 = (col + 1) % 3, i2 = (col + 2) % 3, j1 = (row + 1) % 3, j2 = (row + 2) % 3;
+  return m[i1 * 3 + j1] * m[i2 * 3 + j2] - m[i1 * 3 + j2] * m[i2 * 3 + j1];
 }
 
-constexpr int kGradBlock = 256;
-constexpr int kLanesPerCut = 8;  // adjoint lanes per cut (kMaxCuts * 8 = kGradBlock)
-static_assert(kMaxCuts * kLanesPerCut == kGradBlock, "one lane group per cut");
+// u / w and v / w, correctly rounded, for w and quotients away from the ends
+// of the float range: the division's own sequence (a Newton step on the
+// reciprocal, two remainder corrections of each quotient; Markstein, IBM J.
+// Res. Dev. 1990) without its scaling, the reciprocal shared.
+__device__ __forceinline__ void div2_rn(float u, float v, float w, float& x, float& y) {
+  float r = __builtin_amdgcn_rcpf(w);
+  r = __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
+  float q = u * r;
+  q = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
+  x = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
+  q = v * r;
+  q = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
+  y = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
+}
 
+constexpr int kLanesPerCut = 8;
+constexpr int kMaxGradBlock = kMaxCuts * kLanesPerCut;
+constexpr int kMaxGradWaves = kMaxGradBlock / 64;
+
+// One marker's evaluation, by a block of kLanesPerCut lanes per cut.  Lane j
+// of a cut takes its samples j, j + 8, ... (R of them) through both passes:
+// the samples' image gradients, already divided by the projective
+// denominator, stay in registers between the forward pass and the adjoint,
+// which needs only the sums L = sum_i t_i lambda_i and M = sum_i lambda_i
+// per cut (u_ki = (t_i q_k, 1), so sum_i lambda_i u_i^T = [L q_k^T, M]).
+//
+// LOCAL (the refiner's calls): positions are taken relative to (ox, oy), the
+// pixel of the centre.  A float position then errs by ulps of the marker's
+// size instead of the image's (2.5e-4 px at 4000 px; the gradient of 2048
+// markers in a 7360 px mosaic is off by 6e-5 instead of 1.1e-3), and a cut's
+// samples are w(t) = t A_k + H_{:,2} with A_k = H_{:,01} q_k in double, three
+// fused multiply-adds.
+// Otherwise (the identification): image coordinates, each float operation
+// rounded on its own and the adjoint in double, which keeps the identified
+// markers' qualities and homographies as they always were: a descent of 30
+// steps ends where rounding sends it, 3e-4 apart in quality for positions
+// that differ by 1e-4 px.
+//
+// Bound by instruction issue, at 4096 markers.  Before, the forward pass took
+// two double divisions per sample, the adjoint sampled the image again and
+// took three more, and the closed form, the inverse and the score's sum ran
+// on one lane: 20 steps of 4096 markers 4270 us, now 1300; one evaluation of
+// 2048 markers 124 us, now 36.
 template <class T>
 struct EvalShared {
-  double H[9], Hi[9];
-  double v[kMaxCuts][3];       // H^-1 p_k
-  T s[kMaxCuts][kMaxSamples];
-  int oob[kMaxCuts];
-  double S[kMaxSamples];       // sum over valid cuts of s_ki
-  double part[kMaxSamples];
-  double G[kMaxCuts][9];
-  double cost, gH[9];
-  int m, ok;
+  double H[9], Hi[9], det;        // relative to (ox, oy)
+  double dir[2][9];               // dH / d(cx), dH / d(cy)
+  double q[kMaxCuts][2], v[kMaxCuts][3];  // q = v / v2, v = H^-1 (p, 1)
+  double A[kMaxCuts][3];          // H_{:,01} q
+  double S[kMaxSamples];          // sum over the valid cuts of the doubled samples
+  double sum[kMaxGradWaves][11];  // each wavefront's cost and derivatives
+  uint32_t oob;
+  uint32_t plain;                 // cuts whose denominators div2_rn takes
+  int ox, oy;
 };
 
-// Sample i of cut k at the homography (Hs in T): the image position, its
-// half-bilinear value and the value's derivatives along image x and y.
-// False when the position is outside [0, w-1) x [0, h-1).
 template <class T>
-__device__ __forceinline__ bool sample_at(const GradJobDev& J, const T* Hs, T qx, T qy, T t, T& val,
-                                          T& dx, T& dy) {
-  const T ux = t * qx, uy = t * qy;
-  const T w0 = Hs[0] * ux + Hs[1] * uy + Hs[2], w1 = Hs[3] * ux + Hs[4] * uy + Hs[5],
-          w2 = Hs[6] * ux + Hs[7] * uy + Hs[8];
-  const T x = w0 / w2, y = w1 / w2;
-  if (!(x >= (T)0 && x < (T)(J.iw - 1) && y >= (T)0 && y < (T)(J.ih - 1))) return false;
-  const int ix = (int)x, iy = (int)y;
-  const uint32_t q = J.quad[(size_t)iy * J.iw + ix];
-  const T fx = x - (T)ix, fy = y - (T)iy;
-  const T a = (T)(q & 255u), b = (T)((q >> 8) & 255u), c = (T)((q >> 16) & 255u), d = (T)(q >> 24);
-  val = (a * ((T)1 - fx) * ((T)1 - fy) + b * fx * ((T)1 - fy) + c * ((T)1 - fx) * fy + d * fx * fy) / (T)2;
-  dx = ((b - a) * ((T)1 - fy) + (d - c) * fy) / (T)2;
-  dy = ((c - a) * ((T)1 - fx) + (d - b) * fx) / (T)2;
-  return true;
+__device__ __forceinline__ T recip(T w);
+template <>
+__device__ __forceinline__ double recip(double w) {
+  return 1.0 / w;
+}
+template <>
+__device__ __forceinline__ float recip(float w) {  // within 1 ulp
+  const float r = __builtin_amdgcn_rcpf(w);
+  return __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
+}
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Wavefront 0: the cuts' constants from the homography E.H (E.ox, E.oy set).
+template <class T>
+__device__ __forceinline__ void lay_out_cuts(const GradJobDev& J, EvalShared<T>& E) {
+  const int k = threadIdx.x;
+  double H[9], Hi[9];
+  for (int e = 0; e < 9; ++e) H[e] = E.H[e];
+  for (int r = 0; r < 3; ++r)
+    for (int c = 0; c < 3; ++c) Hi[r * 3 + c] = adjugate(H, r, c);
+  const double det = H[0] * Hi[0] + H[1] * Hi[3] + H[2] * Hi[6], id = 1.0 / det;
+  for (int e = 0; e < 9; ++e) Hi[e] *= id;
+  if (k == 0) {
+    for (int e = 0; e < 9; ++e) E.Hi[e] = Hi[e];
+    E.det = det;
+    E.oob = 0;
+  }
+  bool plain = false;
+  if (k < J.n_cuts) {
+    const double px = (double)J.stops[k].x - E.ox, py = (double)J.stops[k].y - E.oy;
+    double v[3];
+    for (int r = 0; r < 3; ++r) v[r] = Hi[r * 3] * px + Hi[r * 3 + 1] * py + Hi[r * 3 + 2];
+    const double qx = v[0] / v[2], qy = v[1] / v[2];
+    E.q[k][0] = qx;
+    E.q[k][1] = qy;
+    for (int r = 0; r < 3; ++r) {
+      E.v[k][r] = v[r];
+      E.A[k][r] = H[r * 3] * qx + H[r * 3 + 1] * qy;
+    }
+    const double a = J.begin_sig * E.A[k][2] + H[8], b = J.end_sig * E.A[k][2] + H[8];
+    plain = (a > 0.0) == (b > 0.0) && fmin(fabs(a), fabs(b)) > 0x1p-60 &&
+            fmax(fabs(a), fabs(b)) < 0x1p60;
+  }
+  const uint32_t p = (uint32_t)__ballot(plain);
+  if (k == 0) E.plain = p;
 }
 
-// Forward (and with `grad`, adjoint) pass of one marker at the homography
-// in E.H; the whole block takes part.  E.cost is DBL_MAX and E.ok 0 when
-// fewer than two cuts are valid or H is singular.
-template <class T>
-__device__ void eval_marker(const GradJobDev& J, int n_samples, bool grad, EvalShared<T>& E) {
-  const int tid = threadIdx.x;
-  const int nc = J.n_cuts;
-  if (tid == 0) E.ok = inverse3d(E.H, E.Hi) ? 1 : 0;
-  if (tid < kMaxCuts) E.oob[tid] = 0;
-  __syncthreads();
-  if (!E.ok) {
-    if (tid == 0) E.cost = DBL_MAX;
-    __syncthreads();
-    return;
-  }
-  if (tid < nc) {
-    const double px = J.stops[tid].x, py = J.stops[tid].y;
-    for (int r = 0; r < 3; ++r) E.v[tid][r] = E.Hi[r * 3 + 0] * px + E.Hi[r * 3 + 1] * py + E.Hi[r * 3 + 2];
-  }
-  __syncthreads();
-  T Hs[9];
-  for (int e = 0; e < 9; ++e) Hs[e] = (T)E.H[e];
+// Score and, per lane, the derivative sums of its cut at E.H (laid out, after
+// a barrier).  False when fewer than two cuts are valid or H is singular;
+// otherwise every lane of a valid cut holds the cut's L and M (scaled to
+// dC/dw) and E.sum[wave][0] its wavefront's share of the score, to be read
+// after a barrier.  sig: n_cuts x n_samples.
+template <class T, int R, bool LOCAL>
+__device__ __forceinline__ bool eval_marker(const GradJobDev& J, int n_samples, EvalShared<T>& E, T* sig,
+                                            double* L, double* M) {
+  const int tid = threadIdx.x, nc = J.n_cuts;
+  const int k = tid / kLanesPerCut, j = tid % kLanesPerCut;
+  const bool on = k < nc;
   const T b = (T)J.begin_sig, step = ((T)J.end_sig - (T)J.begin_sig) / (T)(n_samples - 1);
-  for (int q = tid; q < nc * n_samples; q += kGradBlock) {
-    const int k = q / n_samples, i = q - k * n_samples;
-    const T qx = (T)(E.v[k][0] / E.v[k][2]), qy = (T)(E.v[k][1] / E.v[k][2]);
-    T val, dx, dy;
-    if (sample_at<T>(J, Hs, qx, qy, b + (T)i * step, val, dx, dy)) {
-      E.s[k][i] = val;
-    } else {
-      E.s[k][i] = (T)0;
-      atomicOr(&E.oob[k], 1);
+  // per sample the doubled sample's derivatives along x and y (LOCAL: over
+  // the denominator, and the adjoint's third component)
+  T gx[R], gy[R], gz[LOCAL ? R : 1];
+  if (on) {
+    const T xlo = (T)(-E.ox), xhi = (T)(J.iw - 1 - E.ox), ylo = (T)(-E.oy), yhi = (T)(J.ih - 1 - E.oy);
+    const int base = E.oy * J.iw + E.ox;
+    T H[9];
+    for (int e = 0; e < 9; ++e) H[e] = (T)E.H[e];
+    const T a0 = (T)E.A[k][0], a1 = (T)E.A[k][1], a2 = (T)E.A[k][2];
+    const T qx = (T)E.q[k][0], qy = (T)E.q[k][1];
+    const bool plain = (E.plain >> k) & 1u;
+    bool out = false;
+    constexpr int kBatch = 7;  // samples whose image reads are in flight together
+#pragma unroll
+    for (int t0 = 0; t0 < R; t0 += kBatch) {
+      T x[kBatch], y[kBatch], r[kBatch];
+      uint32_t q[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (t0 + u >= R) continue;
+        const int i = j + (t0 + u) * kLanesPerCut;
+        const T t = b + (T)i * step;
+        if constexpr (LOCAL) {
+          r[u] = recip<T>(fused(t, a2, H[8]));
+          x[u] = fused(t, a0, H[2]) * r[u];
+          y[u] = fused(t, a1, H[5]) * r[u];
+        } else {
+          const T ux = t * qx, uy = t * qy;
+          const T w0 = H[0] * ux + H[1] * uy + H[2], w1 = H[3] * ux + H[4] * uy + H[5],
+                  w2 = H[6] * ux + H[7] * uy + H[8];
+          if (plain) {
+            div2_rn(w0, w1, w2, x[u], y[u]);
+          } else {
+            x[u] = w0 / w2;
+            y[u] = w1 / w2;
+          }
+        }
+        const bool in = x[u] >= xlo && x[u] < xhi && y[u] >= ylo && y[u] < yhi;
+        out |= i < n_samples && !in;
+        const int at = in && i < n_samples ? base + (int)floor(y[u]) * J.iw + (int)floor(x[u]) : 0;
+        q[u] = J.quad[(uint32_t)at];
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (t0 + u >= R) continue;
+        const int i = j + (t0 + u) * kLanesPerCut;
+        const T fx = x[u] - floor(x[u]), fy = y[u] - floor(y[u]);
+        const T p00 = (T)(q[u] & 255u), p10 = (T)((q[u] >> 8) & 255u), p01 = (T)((q[u] >> 16) & 255u),
+                p11 = (T)(q[u] >> 24);
+        const T d0 = p10 - p00, d1 = p11 - p01;
+        T val;
+        if constexpr (LOCAL) {
+          const T top = fused(fx, d0, p00), dy = fused(fx, d1, p01) - top;
+          const T dx = fused(fy, d1 - d0, d0);
+          val = fused(fy, dy, top);
+          gx[t0 + u] = dx * r[u];
+          gy[t0 + u] = dy * r[u];
+          gz[t0 + u] = -(gx[t0 + u] * x[u] + gy[t0 + u] * y[u]);
+        } else {
+          const T fx1 = (T)1 - fx, fy1 = (T)1 - fy;
+          val = p00 * fx1 * fy1 + p10 * fx * fy1 + p01 * fx1 * fy + p11 * fx * fy;
+          gx[t0 + u] = d0 * fy1 + d1 * fy;
+          gy[t0 + u] = (p01 - p00) * fx1 + (p11 - p10) * fx;
+        }
+        if (i < n_samples) sig[k * n_samples + i] = val;
+      }
     }
+    if (out) atomicOr(&E.oob, 1u << k);
   }
   __syncthreads();
-  if (tid == 0) {
-    int m = 0;
-    for (int k = 0; k < nc; ++k) m += E.oob[k] == 0;
-    E.m = m;
+  const uint32_t valid = ~E.oob & (nc >= 32 ? ~0u : (1u << nc) - 1u);
+  const int m = __popc(valid);
+  for (int i = tid; i < n_samples; i += blockDim.x) {
+    double s = 0.0;
+    constexpr int kRead = 8;  // reads in flight together
+    for (int k0 = 0; k0 < nc; k0 += kRead) {
+      T v[kRead];
+#pragma unroll
+      for (int u = 0; u < kRead; ++u) v[u] = sig[min(k0 + u, nc - 1) * n_samples + i];
+#pragma unroll
+      for (int u = 0; u < kRead; ++u)
+        if (k0 + u < nc && ((valid >> (k0 + u)) & 1u)) s += (double)v[u];
+    }
+    E.S[i] = s;
   }
   __syncthreads();
-  const int m = E.m;
-  if (m < 2) {
-    if (tid == 0) {
-      E.cost = DBL_MAX;
-      E.ok = 0;
-    }
-    __syncthreads();
-    return;
-  }
   const double pairs = 0.5 * (double)m * (double)(m - 1);
-  for (int i = tid; i < n_samples; i += kGradBlock) {
-    double s1 = 0.0, s2 = 0.0;
-    for (int k = 0; k < nc; ++k)
-      if (!E.oob[k]) {
-        const double v = (double)E.s[k][i];
-        s1 += v;
-        s2 += v * v;
-      }
-    E.S[i] = s1;
-    E.part[i] = (double)m * s2 - s1 * s1;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double acc = 0.0;
-    for (int i = 0; i < n_samples; ++i) acc += E.part[i];
-    E.cost = acc / pairs;
-  }
-  if (!grad) {
-    __syncthreads();
-    return;
-  }
-  // adjoint: lanes k*8 .. k*8+7 sum cut k's samples
-  {
-    const int k = tid / kLanesPerCut, j = tid - k * kLanesPerCut;
-    double A[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, L[3] = {0, 0, 0};
-    if (k < nc && !E.oob[k]) {
-      const double vx = E.v[k][0] / E.v[k][2], vy = E.v[k][1] / E.v[k][2];
-      const T qx = (T)vx, qy = (T)vy;
-      for (int i = j; i < n_samples; i += kLanesPerCut) {
-        const T tt = b + (T)i * step;
-        T val, dsx, dsy;
-        sample_at<T>(J, Hs, qx, qy, tt, val, dsx, dsy);
-        const double a = 2.0 * ((double)m * (double)E.s[k][i] - E.S[i]) / pairs;
-        const double gx = a * (double)dsx, gy = a * (double)dsy;
-        const double t = (double)tt;
-        const double u0 = t * vx, u1 = t * vy;
-        const double w0 = E.H[0] * u0 + E.H[1] * u1 + E.H[2];
-        const double w1 = E.H[3] * u0 + E.H[4] * u1 + E.H[5];
-        const double w2 = E.H[6] * u0 + E.H[7] * u1 + E.H[8];
-        const double l0 = gx / w2, l1 = gy / w2, l2 = -(gx * w0 + gy * w1) / (w2 * w2);
-        const double lam[3] = {l0, l1, l2}, u[3] = {u0, u1, 1.0};
+  double cost = 0.0;  // sum over the cut of (m s - S)^2, s and S doubled
+  for (int r = 0; r < 3; ++r) L[r] = M[r] = 0.0;
+  if (on && ((valid >> k) & 1u)) {
+    const double dm = (double)m, A[3] = {E.A[k][0], E.A[k][1], E.A[k][2]};
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int i = j + t * kLanesPerCut;
+      if (i < n_samples) {
+        const double d = dm * (double)sig[k * n_samples + i] - E.S[i];
+        const double tt = (double)(b + (T)i * step);
+        cost = __builtin_fma(d, d, cost);
+        double g[3] = {(double)gx[t], (double)gy[t], 0.0};
+        if constexpr (LOCAL) {
+          g[2] = (double)gz[t];
+        } else {
+          const double rw = recip<double>(__builtin_fma(tt, A[2], E.H[8]));
+          g[0] *= rw;
+          g[1] *= rw;
+          g[2] = -(g[0] * __builtin_fma(tt, A[0], E.H[2]) + g[1] * __builtin_fma(tt, A[1], E.H[5])) * rw;
+        }
+#pragma unroll
         for (int r = 0; r < 3; ++r) {
-          for (int c = 0; c < 3; ++c) A[r * 3 + c] += lam[r] * u[c];
-          L[r] += t * lam[r];
-        }
-      }
-    }
-    for (int o = kLanesPerCut / 2; o > 0; o >>= 1) {
-      for (int e = 0; e < 9; ++e) A[e] += __shfl_down(A[e], o, kLanesPerCut);
-      for (int e = 0; e < 3; ++e) L[e] += __shfl_down(L[e], o, kLanesPerCut);
-    }
-    if (j == 0 && k < nc) {
-      if (E.oob[k]) {
-        for (int e = 0; e < 9; ++e) E.G[k][e] = 0.0;
-      } else {
-        const double* H = E.H;
-        const double* v = E.v[k];
-        const double z0 = H[0] * L[0] + H[3] * L[1] + H[6] * L[2];
-        const double z1 = H[1] * L[0] + H[4] * L[1] + H[7] * L[2];
-        const double nu[3] = {z0 / v[2], z1 / v[2], -(z0 * v[0] + z1 * v[1]) / (v[2] * v[2])};
-        for (int a = 0; a < 3; ++a) {
-          const double rho = E.Hi[0 * 3 + a] * nu[0] + E.Hi[1 * 3 + a] * nu[1] + E.Hi[2 * 3 + a] * nu[2];
-          for (int c = 0; c < 3; ++c) E.G[k][a * 3 + c] = A[a * 3 + c] - rho * v[c];
+          const double dg = d * g[r];
+          M[r] += dg;
+          L[r] = __builtin_fma(tt, dg, L[r]);
         }
       }
     }
   }
-  __syncthreads();
-  if (tid < 9) {
-    double acc = 0.0;
-    for (int k = 0; k < nc; ++k) acc += E.G[k][tid];
-    E.gH[tid] = acc;
+  // the cut's sums over its lanes, the score over the wavefront
+  for (int o = 1; o < kLanesPerCut; o <<= 1)
+    for (int r = 0; r < 3; ++r) {
+      L[r] += __shfl_xor(L[r], o, 64);
+      M[r] += __shfl_xor(M[r], o, 64);
+    }
+  for (int o = 1; o < 64; o <<= 1) cost += __shfl_xor(cost, o, 64);
+  // sum_k (m s_k - S)^2 = m (m S2 - S^2); ds = dV / 2
+  const double scale = 1.0 / (2.0 * pairs);
+  for (int r = 0; r < 3; ++r) {
+    L[r] *= scale;
+    M[r] *= scale;
   }
-  __syncthreads();
+  if ((tid & 63) == 0) E.sum[tid >> 6][0] = cost / (4.0 * (double)m * pairs);
+  return m >= 2 && E.det != 0.0 && isfinite(E.det);
 }
 
+// A cut's share of the score's derivative along dH = D (relative to the
+// origin as E.H): lambda . (D u) summed over its samples, and through the
+// cut's direction q, dq = J_pi(v) dv, dv = -H^-1 D v.
 template <class T>
-__global__ __launch_bounds__(kGradBlock) void k_grad_eval(const GradJobDev* __restrict__ jobs,
-                                                          const float* __restrict__ Hin, int n_samples,
-                                                          double* __restrict__ cost,
-                                                          double* __restrict__ grad) {
+__device__ __forceinline__ double along(const EvalShared<T>& E, int k, const double* D, const double* L,
+                                        const double* M) {
+  const double qx = E.q[k][0], qy = E.q[k][1];
+  double acc = 0.0, e[3];
+  for (int r = 0; r < 3; ++r) {
+    acc += (D[r * 3] * qx + D[r * 3 + 1] * qy) * L[r] + D[r * 3 + 2] * M[r];
+    e[r] = D[r * 3] * E.v[k][0] + D[r * 3 + 1] * E.v[k][1] + D[r * 3 + 2] * E.v[k][2];
+  }
+  double f[3];
+  for (int r = 0; r < 3; ++r)
+    f[r] = E.Hi[r * 3] * e[0] + E.Hi[r * 3 + 1] * e[1] + E.Hi[r * 3 + 2] * e[2];
+  const double z0 = E.H[0] * L[0] + E.H[3] * L[1] + E.H[6] * L[2];
+  const double z1 = E.H[1] * L[0] + E.H[4] * L[1] + E.H[7] * L[2];
+  return acc - (z0 * (f[0] - qx * f[2]) + z1 * (f[1] - qy * f[2])) / E.v[k][2];
+}
+
+// Lane j of every cut adds its value over the wavefront's cuts (the same
+// lane of each 8-lane group).
+__device__ __forceinline__ double over_cuts(double v) {
+  for (int o = kLanesPerCut; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// Score and gradient at given homographies, one block per marker.
+template <class T, int R>
+__global__ __launch_bounds__(kMaxGradBlock, sizeof(T) == 4 ? 4 : 1) void k_grad_eval(const GradJobDev* __restrict__ jobs,
+                                                             const float* __restrict__ Hin, int n_samples,
+                                                             double* __restrict__ cost,
+                                                             double* __restrict__ grad) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char grad_lds[];
+  T* sig = reinterpret_cast<T*>(grad_lds);
   __shared__ EvalShared<T> E;
-  const int m = blockIdx.x;
+  const int m = blockIdx.x, tid = threadIdx.x, waves = blockDim.x >> 6;
   const GradJobDev& J = jobs[m];
-  if (threadIdx.x < 9) E.H[threadIdx.x] = (double)Hin[m * 9 + threadIdx.x];
-  __syncthreads();
-  eval_marker<T>(J, n_samples, grad != nullptr, E);
-  if (threadIdx.x == 0) {
-    cost[m] = E.cost;
-    if (grad) {
-      if (!E.ok) {
-        for (int e = 0; e < 10; ++e) grad[m * 10 + e] = 0.0;
-      } else {
-        for (int e = 0; e < 8; ++e) grad[m * 10 + e] = E.gH[e];
-        // marker-plane translation of the centre: H' = H [1 0 dx; 0 1 dy; 0 0 1]
-        grad[m * 10 + 8] = E.gH[2] * E.H[0] + E.gH[5] * E.H[3] + E.gH[8] * E.H[6];
-        grad[m * 10 + 9] = E.gH[2] * E.H[1] + E.gH[5] * E.H[4] + E.gH[8] * E.H[7];
-      }
+  const int nc = J.n_cuts;
+  double L[3], M[3];
+  // the origin: the pixel of the homography's centre, kept inside the image
+  if (tid < 64) {
+    const float* h = Hin + m * 9;
+    const double w = h[8];
+    const double cx = (double)h[2] / w, cy = (double)h[5] / w;
+    const int ox = cx > 0.0 && cx < J.iw ? (int)cx : 0, oy = cy > 0.0 && cy < J.ih ? (int)cy : 0;
+    if (tid < 9) {
+      const double o = tid < 3 ? ox : tid < 6 ? oy : 0;
+      E.H[tid] = (double)h[tid] - o * (double)h[6 + tid % 3];
     }
+    if (tid == 0) {
+      E.ox = ox;
+      E.oy = oy;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  if (tid < 64) lay_out_cuts(J, E);
+  __syncthreads();
+  const bool ok = eval_marker<T, R, true>(J, n_samples, E, sig, L, M);
+  if (grad) {
+    // directions 0..7: H's free entries (an entry of the last row moves the
+    // relative rows above it too); 8, 9: the marker-plane shift of the centre
+    // along x and y, H' = H [1 0 x; 0 1 y; 0 0 1]
+    const int k = tid / kLanesPerCut, j = tid % kLanesPerCut;
+    for (int d = j; d < 10; d += kLanesPerCut) {
+      double D[9];
+      for (int e = 0; e < 9; ++e) {
+        const int r = e / 3, c = e % 3;
+        if (d >= 8) D[e] = c == 2 ? E.H[r * 3 + d - 8] : 0.0;
+        else if (c != d % 3) D[e] = 0.0;
+        else if (d < 6) D[e] = e == d ? 1.0 : 0.0;
+        else D[e] = r == 2 ? 1.0 : r == 0 ? -(double)E.ox : -(double)E.oy;
+      }
+      const double v = over_cuts(ok && k < nc ? along(E, k, D, L, M) : 0.0);
+      if ((tid & 63) < kLanesPerCut) E.sum[tid >> 6][1 + d] = v;
+    }
+  }
+  __syncthreads();
+  if (tid < (grad ? 11 : 1)) {
+    double v = 0.0;
+    for (int w = 0; w < waves; ++w) v += E.sum[w][tid];
+    if (tid == 0) cost[m] = ok ? v : DBL_MAX;
+    else grad[m * 10 + tid - 1] = ok ? v : 0.0;
   }
 }
 
 __global__ __launch_bounds__(256) void k_grad_homography(const GradJobDev* __restrict__ jobs, int n,
                                                          const float* __restrict__ centers,
                                                          float* __restrict__ H) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, m = i / 9, e = i - m * 9;
   if (m >= n) return;
-  D2 h[9];
-  closed_form(jobs[m], centers[2 * m], centers[2 * m + 1], h);
-  for (int e = 0; e < 9; ++e) H[m * 9 + e] = (float)h[e].v;
+  H[i] = (float)closed_form(jobs[m], centers[2 * m], centers[2 * m + 1], e / 3, e % 3, false, 0.0, 0.0).v;
 }
 
 // `steps` evaluations per marker, each one forward + adjoint pass at H(c):
 // a step that lowers the score is kept and the step length grows by 1.5,
 // otherwise the centre returns to the best one and the length halves; the
-// next centre moves the best one by the length along -dC/dc.
-template <class T>
-__global__ __launch_bounds__(kGradBlock) void k_grad_descend(const GradJobDev* __restrict__ jobs,
-                                                             int steps, int n_samples,
-                                                             const float* __restrict__ start,
-                                                             float* __restrict__ centers,
-                                                             double* __restrict__ cost) {
+// next centre moves the best one by the length along -dC/dc.  Every lane of
+// wavefront 0 keeps the descent's state; its lanes 0..17 take the closed
+// form's entries and derivatives.
+template <class T, int R, bool LOCAL>
+__global__ __launch_bounds__(kMaxGradBlock, sizeof(T) == 4 ? 4 : 1) void k_grad_descend(const GradJobDev* __restrict__ jobs,
+                                                                int steps, int n_samples,
+                                                                const float* __restrict__ start,
+                                                                float* __restrict__ centers,
+                                                                double* __restrict__ cost) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char grad_lds[];
+  T* sig = reinterpret_cast<T*>(grad_lds);
   __shared__ EvalShared<T> E;
-  __shared__ double dH[9][2];
-  __shared__ double cx, cy, best_x, best_y, best_cost, gbx, gby, alpha;
   __shared__ int stop;
-  const int m = blockIdx.x, tid = threadIdx.x;
+  const int m = blockIdx.x, tid = threadIdx.x, waves = blockDim.x >> 6;
   const GradJobDev& J = jobs[m];
-  if (tid == 0) {
-    cx = start ? start[2 * m] : J.c0x;
-    cy = start ? start[2 * m + 1] : J.c0y;
-    best_x = cx;
-    best_y = cy;
-    best_cost = DBL_MAX;
-    gbx = gby = 0.0;
-    alpha = J.alpha0;
-    stop = 0;
-  }
-  __syncthreads();
+  const int nc = J.n_cuts;
+  double cx = start ? start[2 * m] : J.c0x, cy = start ? start[2 * m + 1] : J.c0y;
+  double best_x = cx, best_y = cy, best_cost = DBL_MAX, gbx = 0.0, gby = 0.0, alpha = J.alpha0;
+  double L[3], M[3];
   for (int it = 0; it < steps; ++it) {
-    if (tid == 0) {
-      D2 h[9];
-      closed_form(J, cx, cy, h);
-      for (int e = 0; e < 9; ++e) {
-        E.H[e] = h[e].v;
-        dH[e][0] = h[e].dx;
-        dH[e][1] = h[e].dy;
+    if (tid < 64) {
+      const int ox = LOCAL && cx > 0.0 && cx < J.iw ? (int)cx : 0;
+      const int oy = LOCAL && cy > 0.0 && cy < J.ih ? (int)cy : 0;
+      const int e = min(tid >> 1, 8), s = tid & 1;
+      const D1 h = closed_form(J, cx, cy, e / 3, e % 3, s, ox, oy);
+      if (tid < 18) {
+        if (s == 0) E.H[e] = h.v;
+        E.dir[s][e] = h.d;
+      }
+      if (tid == 0) {
+        E.ox = ox;
+        E.oy = oy;
+        stop = 0;
       }
     }
     __syncthreads();
-    eval_marker<T>(J, n_samples, true, E);
-    if (tid == 0) {
-      const bool better = E.ok && E.cost < best_cost;
-      if (better) {
-        double gx = 0.0, gy = 0.0;
-        for (int e = 0; e < 9; ++e) {
-          gx += E.gH[e] * dH[e][0];
-          gy += E.gH[e] * dH[e][1];
-        }
+    if (tid < 64) lay_out_cuts(J, E);
+    __syncthreads();
+    const bool ok = eval_marker<T, R, LOCAL>(J, n_samples, E, sig, L, M);
+    {
+      const int k = tid / kLanesPerCut, s = tid & 1;
+      const double v = over_cuts(ok && k < nc ? along(E, k, E.dir[s], L, M) : 0.0);
+      if ((tid & 63) < 2) E.sum[tid >> 6][1 + s] = v;
+    }
+    __syncthreads();
+    if (tid < 64) {
+      double sum[3] = {0.0, 0.0, 0.0};
+      for (int w = 0; w < waves; ++w)
+        for (int r = 0; r < 3; ++r) sum[r] += E.sum[w][r];
+      if (ok && sum[0] < best_cost) {
         if (it > 0) alpha *= 1.5;
         best_x = cx;
         best_y = cy;
-        best_cost = E.cost;
-        gbx = gx;
-        gby = gy;
+        best_cost = sum[0];
+        gbx = sum[1];
+        gby = sum[2];
       } else {
         alpha *= 0.5;
       }
       const double gn = sqrt(gbx * gbx + gby * gby);
       if (!(gn > 0.0) || !isfinite(gn) || best_cost == DBL_MAX) {
-        stop = 1;
+        if (tid == 0) stop = 1;
       } else {
         cx = best_x - alpha * gbx / gn;
         cy = best_y - alpha * gby / gn;
@@ -399,6 +548,42 @@ __global__ __launch_bounds__(256) void k_quads(const uint8_t* __restrict__ img, 
             (uint32_t)r0[dy + dx] << 24;
 }
 
+// A block's shape: kLanesPerCut lanes per cut; kSamplesPerLane samples of a
+// lane are kept in registers (13 cover 104 samples, 16 kMaxSamples).
+struct GradShape {
+  int block;
+  size_t lds;
+};
+template <class T>
+GradShape grad_shape(int max_cuts, int n_samples) {
+  const int cuts = std::min(std::max(max_cuts, 1), kMaxCuts);
+  return GradShape{(cuts * kLanesPerCut + 63) / 64 * 64, sizeof(T) * cuts * n_samples};
+}
+constexpr int kFewSamples = 13, kAllSamples = 16;
+static_assert(kAllSamples * kLanesPerCut >= kMaxSamples, "every sample has a lane");
+
+template <class T>
+void eval_launch(const GradJobDev* jobs, int n, const float* H, int max_cuts, int n_samples,
+                 double* cost, double* grad, hipStream_t s) {
+  const GradShape sh = grad_shape<T>(max_cuts, n_samples);
+  if (n_samples <= kFewSamples * kLanesPerCut)
+    k_grad_eval<T, kFewSamples><<<n, sh.block, sh.lds, s>>>(jobs, H, n_samples, cost, grad);
+  else
+    k_grad_eval<T, kAllSamples><<<n, sh.block, sh.lds, s>>>(jobs, H, n_samples, cost, grad);
+}
+
+template <class T, bool LOCAL>
+void descend_launch(const GradJobDev* jobs, int n, int steps, int max_cuts, int n_samples,
+                    const float* start, float* centers, double* cost, hipStream_t s) {
+  const GradShape sh = grad_shape<T>(max_cuts, n_samples);
+  if (n_samples <= kFewSamples * kLanesPerCut)
+    k_grad_descend<T, kFewSamples, LOCAL><<<n, sh.block, sh.lds, s>>>(jobs, steps, n_samples, start,
+                                                                      centers, cost);
+  else
+    k_grad_descend<T, kAllSamples, LOCAL><<<n, sh.block, sh.lds, s>>>(jobs, steps, n_samples, start,
+                                                                      centers, cost);
+}
+
 }  // namespace
 
 int launch_quads(const uint8_t* img, int w, int h, uint32_t* quad, hipStream_t s) {
@@ -414,28 +599,31 @@ int launch_grad_start(const GradJobDev* jobs, int n, const int* coarse_of, const
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_grad_eval(const GradJobDev* jobs, int n, const float* H, int n_samples, bool fp64,
-                     double* cost, double* grad, hipStream_t s) {
+int launch_grad_eval(const GradJobDev* jobs, int n, const float* H, int max_cuts, int n_samples,
+                     bool fp64, double* cost, double* grad, hipStream_t s) {
   if (n <= 0) return 0;
-  if (fp64) k_grad_eval<double><<<n, kGradBlock, 0, s>>>(jobs, H, n_samples, cost, grad);
-  else k_grad_eval<float><<<n, kGradBlock, 0, s>>>(jobs, H, n_samples, cost, grad);
+  if (fp64) eval_launch<double>(jobs, n, H, max_cuts, n_samples, cost, grad, s);
+  else eval_launch<float>(jobs, n, H, max_cuts, n_samples, cost, grad, s);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 int launch_grad_homography(const GradJobDev* jobs, int n, const float* centers, float* H,
                            hipStream_t s) {
   if (n <= 0) return 0;
-  k_grad_homography<<<(n + 255) / 256, 256, 0, s>>>(jobs, n, centers, H);
+  k_grad_homography<<<(9 * n + 255) / 256, 256, 0, s>>>(jobs, n, centers, H);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int launch_grad_descend(const GradJobDev* jobs, int n, int steps, int n_samples, bool fp64,
-                        const float* start, float* centers, double* cost, hipStream_t s) {
+int launch_grad_descend(const GradJobDev* jobs, int n, int steps, int max_cuts, int n_samples,
+                        GradSampling sampling, const float* start, float* centers, double* cost,
+                        hipStream_t s) {
   if (n <= 0) return 0;
-  if (fp64)
-    k_grad_descend<double><<<n, kGradBlock, 0, s>>>(jobs, steps, n_samples, start, centers, cost);
+  if (sampling == GradSampling::fp64)
+    descend_launch<double, true>(jobs, n, steps, max_cuts, n_samples, start, centers, cost, s);
+  else if (sampling == GradSampling::local)
+    descend_launch<float, true>(jobs, n, steps, max_cuts, n_samples, start, centers, cost, s);
   else
-    k_grad_descend<float><<<n, kGradBlock, 0, s>>>(jobs, steps, n_samples, start, centers, cost);
+    descend_launch<float, false>(jobs, n, steps, max_cuts, n_samples, start, centers, cost, s);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

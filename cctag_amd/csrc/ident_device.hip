@@ -263,7 +263,8 @@ void GpuIdentBackend::refine_gradient(const std::vector<RefineJob>& jobs, const 
   const int ns = k_.n_samples;
   if (launch_refine_coarse(d_ref_jobs_, n, most_cuts(jobs), ns, p.imaged_center_n_grid_sample, d_work_,
                            d_coarse_.as<float>(), s) != 0 ||
-      launch_grad_descend(d_grad_jobs_.as<GradJobDev>(), n, grad_steps_, ns, false,
+      launch_grad_descend(d_grad_jobs_.as<GradJobDev>(), n, grad_steps_, most_cuts(jobs), ns,
+                          GradSampling::image,
                           d_coarse_.as<float>(), d_gcenters_.as<float>(), d_gcost_.as<double>(),
                           s) != 0 ||
       launch_grad_homography(d_grad_jobs_.as<GradJobDev>(), n, d_gcenters_.as<float>(),
