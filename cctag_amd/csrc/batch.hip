@@ -36,7 +36,7 @@ struct cctagx_batch {
   hipStream_t stream = nullptr;
   FrontEndDevice fe;
   GpuIdentBackend ident;
-  std::unique_ptr<TaskPool> pool;
+  PoolPlace pool;  // host workers, leased by each call
   LevelStager stager;
   std::vector<LevelEdges> views;
   std::vector<std::vector<Marker>> cand, found;
@@ -174,8 +174,7 @@ int cctagx_batch_create(const cctagx_params* params, int n_frames, const int32_t
     for (const PlaneDesc& d : b->fe.planes().planes)
       if (d.level == 0) images.push_back(DeviceImage{b->fe.buffers().quad + d.pix, d.w, d.h});
     b->ident.set_images(images);
-    const int threads = TaskPool::default_threads();
-    if (threads > 1) b->pool = std::make_unique<TaskPool>(threads);
+    b->pool.set(TaskPool::default_threads());
   } catch (const std::exception& e) {
     set_error(e.what());
     return CCTAGX_ERR_HIP;
@@ -208,7 +207,8 @@ int cctagx_batch_load(cctagx_batch* b, int frame, const uint8_t* gray, int width
     set_error("frame size differs from the one given at cctagx_batch_create");
     return CCTAGX_ERR_ARG;
   }
-  if (int rc = b->fe.upload(frame, gray, stride, b->stream, b->pool.get())) return rc;
+  const PoolLease pool(b->pool);
+  if (int rc = b->fe.upload(frame, gray, stride, b->stream, pool.get())) return rc;
   b->loaded[frame] = true;
   return CCTAGX_OK;
 }
@@ -262,6 +262,7 @@ int cctagx_batch_detect(cctagx_batch* b, cctagx_marker* out, int max_out, int32_
   b->stats.stage_us = (float)(ms_since(t) * 1000.0);
   try {
     t = Clock::now();
+    const PoolLease pool(b->pool);
     const int nl = b->n_levels;
     // frames in parallel, each frame's tasks serial on its worker; the
     // largest frames are handed out first (their candidate stages are the
@@ -272,7 +273,7 @@ int cctagx_batch_detect(cctagx_batch* b, cctagx_marker* out, int max_out, int32_
       return (long long)b->sizes[a].first * b->sizes[a].second >
              (long long)b->sizes[c].first * b->sizes[c].second;
     });
-    parallel_for(b->pool.get(), b->n_frames, [&](int k) {
+    parallel_for(pool.get(), b->n_frames, [&](int k) {
       const int f = order[k];
       std::vector<LevelEdges> lv(b->views.begin() + (size_t)f * nl,
                                  b->views.begin() + (size_t)(f + 1) * nl);
@@ -287,9 +288,9 @@ int cctagx_batch_detect(cctagx_batch* b, cctagx_marker* out, int max_out, int32_
         frames[f].markers = &b->cand[f];
         frames[f].image = f;
       }
-      identify_frames(frames, b->host, b->bank, b->ident, b->pool.get());
+      identify_frames(frames, b->host, b->bank, b->ident, pool.get());
     }
-    parallel_for(b->pool.get(), b->n_frames,
+    parallel_for(pool.get(), b->n_frames,
                  [&](int f) { finish_markers(b->cand[f], b->found[f]); });
     b->stats.ident_us = (float)(ms_since(t) * 1000.0);
     b->stats.select_us = b->ident.last_select_us();

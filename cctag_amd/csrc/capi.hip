@@ -59,7 +59,7 @@ struct cctagx_handle {
   std::vector<LevelEdges> views;  // candidate-stage inputs of the last detection
   GpuIdentBackend ident;
   std::vector<Marker> markers;
-  std::unique_ptr<TaskPool> pool;  // host candidate-stage workers
+  PoolPlace pool;  // host candidate-stage workers, leased by each call
   double host_ms = 0;  // last detection: host wall time after the front end
   double stage_ms = 0; // last detection: wall time of the level staging copies
   bool staged_two_step = false;  // last detection: the levels did not fit the one-step gather
@@ -149,8 +149,7 @@ int cctagx_create(const cctagx_params* params, int width, int height, cctagx_han
   h->bank = marker_bank(params->n_crowns);
   try {
     if (int rc = h->ident.init(h->bank, h->host, h->stream)) return rc;
-    const int threads = TaskPool::default_threads();
-    if (threads > 1) h->pool = std::make_unique<TaskPool>(threads);
+    h->pool.set(TaskPool::default_threads());
   } catch (const std::exception& e) {
     set_error(e.what());
     return CCTAGX_ERR_HIP;
@@ -179,7 +178,8 @@ static int check_frame(const cctagx_handle* h, const uint8_t* gray, int width, i
 
 int cctagx_load(cctagx_handle* h, const uint8_t* gray, int width, int height, size_t stride) {
   if (int rc = check_frame(h, gray, width, height, stride)) return rc;
-  if (int rc = h->fe.upload(0, gray, stride, h->stream, h->pool.get())) return rc;
+  const PoolLease pool(h->pool);
+  if (int rc = h->fe.upload(0, gray, stride, h->stream, pool.get())) return rc;
   h->have_frame = true;
   h->have_front_end = false;
   return CCTAGX_OK;
@@ -200,7 +200,8 @@ int cctagx_load_bgr(cctagx_handle* h, const uint8_t* bgr, int width, int height,
   }
   // stride / channels >= width exactly when a row of width pixels fits
   if (int rc = check_frame(h, bgr, width, height, stride / channels)) return rc;
-  if (int rc = h->fe.upload_color(0, bgr, stride, channels, h->stream, h->pool.get())) return rc;
+  const PoolLease pool(h->pool);
+  if (int rc = h->fe.upload_color(0, bgr, stride, channels, h->stream, pool.get())) return rc;
   h->have_frame = true;
   h->have_front_end = false;
   return CCTAGX_OK;
@@ -268,7 +269,8 @@ int cctagx_identify(cctagx_handle* h, const cctagx_ident_marker* in, int n,
     const PlaneDesc& d0 = h->fe.planes().planes[0];
     h->ident.set_image(h->fe.buffers().quad + d0.pix, d0.w, d0.h);
     h->ident.clear_stats();
-    identify_markers(markers, h->host, h->bank, h->ident, h->pool.get(), nullptr);
+    const PoolLease pool(h->pool);
+    identify_markers(markers, h->host, h->bank, h->ident, pool.get(), nullptr);
   } catch (const std::exception& e) {
     set_error(e.what());
     return CCTAGX_ERR_HIP;
@@ -357,7 +359,8 @@ int cctagx_detect_loaded(cctagx_handle* h, uint64_t frame, cctagx_marker* out, i
     const PlaneDesc& d0 = h->fe.planes().planes[0];
     h->ident.set_image(h->fe.buffers().quad + d0.pix, d0.w, d0.h);
     h->host_times = HostTimes();
-    detect_markers(h->views, h->host, h->bank, &h->ident, h->markers, h->pool.get(),
+    const PoolLease pool(h->pool);
+    detect_markers(h->views, h->host, h->bank, &h->ident, h->markers, pool.get(),
                    &h->host_times, &h->workspace);
   } catch (const std::exception& e) {
     set_error(e.what());
@@ -398,8 +401,7 @@ int cctagx_set_host_threads(cctagx_handle* h, int threads) {
   if (!h || threads < 0) return CCTAGX_ERR_ARG;
   if (threads == 0) threads = TaskPool::default_threads();
   try {
-    h->pool.reset();
-    if (threads > 1) h->pool = std::make_unique<TaskPool>(threads);
+    h->pool.set(threads);
   } catch (const std::exception& e) {
     set_error(e.what());
     return CCTAGX_ERR_ARG;
@@ -409,7 +411,7 @@ int cctagx_set_host_threads(cctagx_handle* h, int threads) {
 
 int cctagx_get_host_threads(cctagx_handle* h) {
   if (!h) return CCTAGX_ERR_ARG;
-  return h->pool ? h->pool->threads() : 1;
+  return h->pool.threads();
 }
 
 int cctagx_get_detect_stats(cctagx_handle* h, cctagx_detect_stats* st) {
@@ -460,7 +462,8 @@ int cctagx_destroy(cctagx_handle* h) {
 int cctagx_front_end(cctagx_handle* h, const uint8_t* gray, int width, int height,
                      size_t stride) {
   if (int rc = check_frame(h, gray, width, height, stride)) return rc;
-  if (int rc = h->fe.upload(0, gray, stride, h->stream, h->pool.get())) return rc;
+  const PoolLease pool(h->pool);
+  if (int rc = h->fe.upload(0, gray, stride, h->stream, pool.get())) return rc;
   h->have_frame = true;
   h->timer.reset();
   if (int rc = h->fe.run(h->stream, &h->timer)) return rc;

@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdlib>
+#include <map>
+#include <memory>
 
 namespace cctagx {
 namespace {
@@ -122,6 +124,81 @@ void TaskPool::run(int n, const std::function<void(int)>& fn) {
     error_ = nullptr;
   }
   if (err) std::rethrow_exception(err);
+}
+
+namespace {
+struct PoolShelf {
+  int places = 0, pools = 0;          // pools: leased and idle
+  std::vector<std::unique_ptr<TaskPool>> idle;  // the last one was used last
+};
+struct PoolShelves {
+  std::mutex m;
+  std::map<int, PoolShelf> of;  // by thread count
+};
+// (never destroyed: handles may outlive static destruction)
+PoolShelves& shelves() {
+  static PoolShelves* s = new PoolShelves;
+  return *s;
+}
+}  // namespace
+
+void PoolPlace::set(int threads) {
+  if (threads < 1) threads = 1;
+  if (threads == threads_) return;
+  std::unique_ptr<TaskPool> ended;  // joined outside the lock
+  {
+    PoolShelves& all = shelves();
+    std::lock_guard<std::mutex> lk(all.m);
+    if (threads > 1) ++all.of[threads].places;
+    if (threads_ > 1) {
+      PoolShelf& s = all.of[threads_];
+      --s.places;
+      if (s.pools > s.places && !s.idle.empty()) {
+        ended = std::move(s.idle.front());
+        s.idle.erase(s.idle.begin());
+        --s.pools;
+      }
+    }
+  }
+  threads_ = threads;
+}
+
+PoolLease::PoolLease(const PoolPlace& place) {
+  const int threads = place.threads();
+  if (threads <= 1) return;
+  PoolShelves& all = shelves();
+  {
+    std::lock_guard<std::mutex> lk(all.m);
+    PoolShelf& s = all.of[threads];
+    if (!s.idle.empty()) {
+      pool_ = s.idle.back().release();
+      s.idle.pop_back();
+      return;
+    }
+    ++s.pools;
+  }
+  try {
+    pool_ = new TaskPool(threads);
+  } catch (const std::exception&) {
+    std::lock_guard<std::mutex> lk(all.m);
+    --all.of[threads].pools;
+  }
+}
+
+PoolLease::~PoolLease() {
+  if (!pool_) return;
+  std::unique_ptr<TaskPool> pool(pool_);  // (joined outside the lock when its place has gone)
+  PoolShelves& all = shelves();
+  std::lock_guard<std::mutex> lk(all.m);
+  PoolShelf& s = all.of[pool->threads()];
+  if (s.pools > s.places) --s.pools;
+  else s.idle.push_back(std::move(pool));
+}
+
+int pools_alive(int threads) {
+  PoolShelves& all = shelves();
+  std::lock_guard<std::mutex> lk(all.m);
+  return all.of[threads].pools;
 }
 
 void parallel_for(TaskPool* pool, int n, const std::function<void(int)>& fn) {

@@ -10,9 +10,11 @@
 #include <cstring>
 #include <string>
 #include <algorithm>
+#include <atomic>
 #include <exception>
 #include <stdexcept>
 #include <memory>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -487,6 +489,45 @@ int oracle_detect(const cctagx_params* params, const uint8_t* img, int w, int h,
 // g[5i .. 5i+4] = (gx_front, gy_front, gx_back, gy_back, dir): the number of
 // cases in which any of the three decisions differs.  The first neighbour
 // direction is compared modulo 8, the only way the linking uses it.
+// The process's shared worker pools: `users` threads, each with a place of its
+// own, lease a pool `rounds` times and sum 0..n-1 on it, after the same users
+// have taken turns on one thread.  Returns 0, or the number of the first
+// property that failed: a wrong sum (1), more than one pool among users that
+// take turns (2), more pools than places (3), pools left without places (4).
+int oracle_pool_places(int users, int threads, int rounds) {
+  using namespace cctagx;
+  constexpr int n = 200;
+  auto work = [&](const PoolPlace& place) {
+    const PoolLease pool(place);
+    std::atomic<int> sum{0};
+    parallel_for(pool.get(), n, [&](int i) { sum += i; });
+    return sum.load() == n * (n - 1) / 2;
+  };
+  std::atomic<int> wrong{0}, over{0};
+  {
+    std::vector<std::unique_ptr<PoolPlace>> places;
+    for (int u = 0; u < users; ++u) places.push_back(std::make_unique<PoolPlace>(threads));
+    for (int r = 0; r < rounds; ++r)
+      for (auto& p : places) wrong += !work(*p);
+    if (pools_alive(threads) > 1) return 2;
+    std::vector<std::thread> ts;
+    for (auto& p : places)
+      ts.emplace_back([&, place = p.get()] {
+        for (int r = 0; r < rounds; ++r) {
+          wrong += !work(*place);
+          over += pools_alive(threads) > users;
+        }
+      });
+    for (std::thread& t : ts) t.join();
+    if (wrong) return 1;
+    if (over) return 3;
+    places.pop_back();  // a place that goes takes a pool with it, the others' stay
+    if (pools_alive(threads) > users - 1) return 3;
+    if (users > 1 && !work(*places[0])) return 1;
+  }
+  return pools_alive(threads) == 0 ? 0 : 4;
+}
+
 int oracle_linking_mismatches(const float* g, int n) {
   const float pi = 3.14159265358979323846f;
   auto angle = [&](float gx, float gy) { return std::fmod(std::atan2(gy, gx) + 2.0f * pi, 2.0f * pi); };
