@@ -28,7 +28,7 @@ struct cctagx_refiner {
   int max_markers = 0, n = 0;
   int max_cuts = 0;  // most cuts of a marker set
   int w = 0, h = 0;
-  DeviceBuffer img, quad, jobs, H, cost, grad, centers, coarse, start, coarse_of;
+  DeviceBuffer img, quad, jobs, H, cost, centers, coarse, start, coarse_of;
   PinnedBuffer h_jobs, h_io;
   GpuIdentBackend ident;
   std::vector<RefineJob> rjobs;
@@ -99,8 +99,8 @@ int cctagx_refiner_create(const cctagx_params* params, int max_markers, cctagx_r
   }
   if (r->jobs.ensure(sizeof(GradJobDev) * max_markers) ||
       r->h_jobs.ensure(sizeof(GradJobDev) * max_markers) ||
-      r->H.ensure(sizeof(float) * 9 * max_markers) || r->cost.ensure(sizeof(double) * max_markers) ||
-      r->grad.ensure(sizeof(double) * 10 * max_markers) ||
+      r->H.ensure(sizeof(float) * 9 * max_markers) ||
+      r->cost.ensure(sizeof(double) * 11 * max_markers) ||  // scores, then gradients
       r->centers.ensure(sizeof(float) * 2 * max_markers))
     return CCTAGX_ERR_HIP;
   *out = r.release();
@@ -123,9 +123,10 @@ int cctagx_refiner_set_image(cctagx_refiner* r, const uint8_t* gray, int width, 
   if ((size_t)width * height > (size_t)INT32_MAX / 4) return CCTAGX_ERR_ARG;
   if (r->img.ensure((size_t)width * height) || r->quad.ensure(4 * (size_t)width * height))
     return CCTAGX_ERR_HIP;
-  CCTAGX_HIP(hipMemcpy2DAsync(r->img.as<uint8_t>(), width, gray, stride, width, height,
-                              hipMemcpyHostToDevice, r->stream));
-  if (launch_quads(r->img.as<uint8_t>(), width, height, r->quad.as<uint32_t>(), r->stream))
+  size_t pitch = 0;
+  CCTAGX_HIP(upload_rows(r->img.as<uint8_t>(), (size_t)width * height, gray, width, height, stride,
+                         r->stream, &pitch));
+  if (launch_quads(r->img.as<uint8_t>(), width, height, pitch, r->quad.as<uint32_t>(), r->stream))
     return CCTAGX_ERR_HIP;
   CCTAGX_HIP(hipStreamSynchronize(r->stream));
   r->w = width;
@@ -202,13 +203,21 @@ int cctagx_refiner_cost_grad(cctagx_refiner* r, const float* H, int fp64, double
                              double* grad) {
   if (!r || !H || !cost) return CCTAGX_ERR_ARG;
   if (!r->n) return CCTAGX_ERR_STATE;
-  if (int rc = to_device(r, r->H, H, (size_t)9 * r->n)) return rc;
-  if (launch_grad_eval(r->jobs.as<GradJobDev>(), r->n, r->H.as<float>(), r->max_cuts, r->kc.n_samples, fp64 != 0,
-                       r->cost.as<double>(), grad ? r->grad.as<double>() : nullptr, r->stream))
+  // homographies in and results out through one pinned buffer, one wait
+  const size_t n = (size_t)r->n, in = 9 * n * sizeof(float), out = (grad ? 11 : 1) * n * sizeof(double);
+  const size_t at = (in + 255) & ~size_t(255);
+  if (r->h_io.ensure(at + out)) return CCTAGX_ERR_HIP;
+  uint8_t* io = r->h_io.as<uint8_t>();
+  std::memcpy(io, H, in);
+  CCTAGX_HIP(hipMemcpyAsync(r->H.as<void>(), io, in, hipMemcpyHostToDevice, r->stream));
+  double* d_cost = r->cost.as<double>();
+  if (launch_grad_eval(r->jobs.as<GradJobDev>(), r->n, r->H.as<float>(), r->max_cuts, r->kc.n_samples,
+                       fp64 != 0, d_cost, grad ? d_cost + n : nullptr, r->stream))
     return CCTAGX_ERR_HIP;
-  if (int rc = to_host(r, cost, r->cost, r->n)) return rc;
-  if (grad)
-    if (int rc = to_host(r, grad, r->grad, (size_t)10 * r->n)) return rc;
+  CCTAGX_HIP(hipMemcpyAsync(io + at, d_cost, out, hipMemcpyDeviceToHost, r->stream));
+  CCTAGX_HIP(stream_wait(r->stream));
+  std::memcpy(cost, io + at, n * sizeof(double));
+  if (grad) std::memcpy(grad, io + at + n * sizeof(double), 10 * n * sizeof(double));
   return CCTAGX_OK;
 }
 
@@ -269,9 +278,10 @@ int cctagx_refiner_refine(cctagx_refiner* r, int steps, int fp64, float* centers
 int cctagx_refiner_grid(cctagx_refiner* r, float* centers, int32_t* ok) {
   if (!r || !centers || !ok) return CCTAGX_ERR_ARG;
   if (!r->n) return CCTAGX_ERR_STATE;
-  std::vector<RefineResult> res;
+  std::vector<Pt2> c;
+  std::vector<uint8_t> found;
   try {
-    r->ident.refine(r->rjobs, r->host, res);
+    r->ident.search_centers(r->rjobs, r->host, c, found);
   } catch (const std::exception& e) {
     set_error(e.what());
     return CCTAGX_ERR_HIP;
@@ -279,9 +289,9 @@ int cctagx_refiner_grid(cctagx_refiner* r, float* centers, int32_t* ok) {
   r->grid_us = r->ident.last_refine_us();
   for (int i = 0; i < r->n; ++i) {
     const int j = r->rjob_of[i];
-    ok[i] = j >= 0 && res[j].ok;
-    centers[2 * i] = ok[i] ? res[j].center.x : 0.f;
-    centers[2 * i + 1] = ok[i] ? res[j].center.y : 0.f;
+    ok[i] = j >= 0 && found[j];
+    centers[2 * i] = ok[i] ? c[j].x : 0.f;
+    centers[2 * i + 1] = ok[i] ? c[j].y : 0.f;
   }
   return CCTAGX_OK;
 }

@@ -22,8 +22,15 @@ struct GradJobDev {
   float2 stops[kMaxCuts];
 };
 
-// The quads of a w x h image (w, h >= 2) into quad (w * h words).
-int launch_quads(const uint8_t* img, int w, int h, uint32_t* quad, hipStream_t s);
+// The rows of a host image to the device (room for `capacity` bytes, at least
+// width * height): as they lie, one transfer, when they fit with their stride,
+// else packed row by row (a 2-D copy from pageable memory takes about 9 us a
+// row).  *pitch: the device rows' distance.
+hipError_t upload_rows(uint8_t* dst, size_t capacity, const uint8_t* src, int width, int height,
+                       size_t stride, hipStream_t s, size_t* pitch);
+// The quads of a w x h image (w, h >= 2, rows `pitch` bytes apart) into quad
+// (w * h words).
+int launch_quads(const uint8_t* img, int w, int h, size_t pitch, uint32_t* quad, hipStream_t s);
 // max_cuts: the most cuts of a job.
 int launch_grad_eval(const GradJobDev* jobs, int n, const float* H, int max_cuts, int n_samples,
                      bool fp64, double* cost, double* grad, hipStream_t s);

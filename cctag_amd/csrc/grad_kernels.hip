@@ -538,14 +538,14 @@ __global__ __launch_bounds__(256) void k_grad_start(const GradJobDev* __restrict
 
 // One word per pixel: its 2x2 neighbourhood, indices clamped to the image.
 __global__ __launch_bounds__(256) void k_quads(const uint8_t* __restrict__ img, int w, int h,
-                                               uint32_t* __restrict__ quad) {
+                                               size_t pitch, uint32_t* __restrict__ quad) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= w * h) return;
   const int y = i / w, x = i - y * w;
-  const uint8_t* r0 = img + i;
-  const int dx = x + 1 < w ? 1 : 0, dy = y + 1 < h ? w : 0;
-  quad[i] = (uint32_t)r0[0] | (uint32_t)r0[dx] << 8 | (uint32_t)r0[dy] << 16 |
-            (uint32_t)r0[dy + dx] << 24;
+  const uint8_t* r0 = img + (size_t)y * pitch + x;
+  const uint8_t* r1 = y + 1 < h ? r0 + pitch : r0;
+  const int dx = x + 1 < w ? 1 : 0;
+  quad[i] = (uint32_t)r0[0] | (uint32_t)r0[dx] << 8 | (uint32_t)r1[0] << 16 | (uint32_t)r1[dx] << 24;
 }
 
 // A block's shape: kLanesPerCut lanes per cut; kSamplesPerLane samples of a
@@ -586,9 +586,20 @@ void descend_launch(const GradJobDev* jobs, int n, int steps, int max_cuts, int 
 
 }  // namespace
 
-int launch_quads(const uint8_t* img, int w, int h, uint32_t* quad, hipStream_t s) {
+hipError_t upload_rows(uint8_t* dst, size_t capacity, const uint8_t* src, int width, int height,
+                       size_t stride, hipStream_t s, size_t* pitch) {
+  const size_t span = (size_t)(height - 1) * stride + width;
+  if (span <= capacity) {
+    *pitch = stride;
+    return hipMemcpyAsync(dst, src, span, hipMemcpyHostToDevice, s);
+  }
+  *pitch = width;
+  return hipMemcpy2DAsync(dst, width, src, stride, width, height, hipMemcpyHostToDevice, s);
+}
+
+int launch_quads(const uint8_t* img, int w, int h, size_t pitch, uint32_t* quad, hipStream_t s) {
   if (w < 2 || h < 2) return -1;
-  k_quads<<<(w * h + 255) / 256, 256, 0, s>>>(img, w, h, quad);
+  k_quads<<<(w * h + 255) / 256, 256, 0, s>>>(img, w, h, pitch, quad);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -87,19 +87,21 @@ struct RefineWork {
   RefineHomDev* hom;       // n_jobs x kMaxGrid^2
 };
 
-// out: one header per job; dist: per job n_cuts x bank_rows distances from
-// its dist_offset on (invalid cuts' rows are not written).
-// The grid search's first iteration only: per job the centre it moves to
-// (centers: 2 per job, device memory).
-int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int max_cuts, int n_samples,
-                         int grid_n, const RefineWork& work, float* centers, hipStream_t s);
+// The search alone, at most `iters` iterations (1: the coarse step): per job
+// the centre it reaches (its start when it finds none) and, with `found`,
+// whether it found one.  max_cuts: the most cuts of a job.
+int launch_refine_centers(const RefineJobDev* jobs, int n_jobs, int iters, int max_cuts,
+                          int n_samples, int grid_n, const RefineWork& work, float2* centers,
+                          int* found, hipStream_t s);
 // The read-out of launch_refine's last kernel at given homographies (9 per
 // job), centres (2 per job) and scores instead of the grid search's choice.
 int launch_refine_readout(const RefineJobDev* jobs, int n_jobs, int n_samples, const float* H,
                           const float* centers, const double* cost, const float* inv_ratio,
                           int bank_rows, int bank_cols, const RefineWork& work, RefineOutDev* out,
                           float* dist, hipStream_t s);
-// max_iter, max_cuts: the most iterations and cuts of a job.
+// The search and its read-out (max_iter, max_cuts: the most iterations and cuts
+// of a job).  out: one header per job; dist: per job n_cuts x bank_rows
+// distances from its dist_offset on (invalid cuts' rows are not written).
 int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int max_cuts, int n_samples,
                   int grid_n, const float* inv_ratio, int bank_rows, int bank_cols, const RefineWork& work,
                   RefineOutDev* out, float* dist, hipStream_t s);
@@ -145,6 +147,10 @@ class GpuIdentBackend : public IdentBackend {
   // The centres after the grid search's first iteration, into device memory
   // (2 floats per job), on the backend's stream without synchronizing.
   void coarse_centers(const std::vector<RefineJob>& jobs, const HostParams& p, float* d_centers);
+  // The grid search without its read-out: per job the centre and whether one
+  // was found.
+  void search_centers(const std::vector<RefineJob>& jobs, const HostParams& p,
+                      std::vector<Pt2>& centers, std::vector<uint8_t>& found);
   // Device time of the last select / refine launches, microseconds.
   float last_select_us() const { return select_us_; }
   float last_refine_us() const { return refine_us_; }
@@ -191,7 +197,9 @@ class GpuIdentBackend : public IdentBackend {
   bool jobs_in_flight_ = false;
   int grad_steps_ = 0;
   void refine_gradient(const std::vector<RefineJob>& jobs, const HostParams& p);
-  PinnedBuffer h_grad_jobs_;
+  void send_refine_jobs(const std::vector<RefineJob>& jobs);
+  void count_refine_work(const std::vector<RefineJob>& jobs, const HostParams& p);
+  PinnedBuffer h_grad_jobs_, h_centers_;
   DeviceBuffer d_grad_jobs_, d_coarse_, d_gcenters_, d_gcost_, d_gH_;
   float select_us_ = 0, refine_us_ = 0;
   int select_jobs_ = 0, refine_jobs_ = 0;

@@ -700,6 +700,13 @@ __device__ void state_at(const RefineJobDev& J, int it, int n_samples, int grid_
   __syncthreads();
 }
 
+// A marker's centre, its job's start when no grid point was readable.
+__device__ __forceinline__ void put_center(const RefineJobDev& J, bool found, const RefineStateDev& S,
+                                           int m, float2* centers, int* found_out) {
+  centers[m] = found ? make_float2(S.cx, S.cy) : make_float2(J.c0x, J.c0y);
+  if (found_out) found_out[m] = found ? 1 : 0;
+}
+
 // Two kernels run the search, with the same results: k_refine_iter, one
 // launch per iteration, spreads few markers over the chip; k_refine_search,
 // a block per marker, does the least work for many.
@@ -868,8 +875,8 @@ __global__ __launch_bounds__(kMaxRefineBlock) void k_refine_iter(
         RefinePointDev{center[tid].x, center[tid].y, flags(tid), 0u};
 }
 
-// The whole search in one block per marker (at most `iters` iterations; the
-// coarse step is one, its centres go to `centers`).  A lane owns one chunk of
+// The whole search in one block per marker (at most `iters` iterations; with
+// `centers`, the centre reached is all that is kept).  A lane owns one chunk of
 // kSumChunk samples at one grid point, the grid points side by side as in
 // k_refine_iter, and keeps the sums over the cuts in registers, so no sample
 // goes through LDS; B >= grid_n^2 * sum chunks.  The cuts' running sums are
@@ -879,7 +886,7 @@ constexpr int kSearchCuts = 6;
 template <int B>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_refine_search(
     const RefineJobDev* __restrict__ jobs, Samples ns, int grid_n, int iters, RefineWork W,
-    float* __restrict__ centers) {
+    float2* __restrict__ centers, int* __restrict__ found) {
   __shared__ float2 start[kSearchCuts][kMaxSumChunks][G2MAX], step[kSearchCuts][G2MAX];
   __shared__ double part[G2MAX][kMaxSumChunks];
   __shared__ float gH[G2MAX][9], gHi[G2MAX][9];
@@ -997,11 +1004,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_r
     if (!S.ok) break;
   }
   if (centers) {
-    if (tid == 0) {
-      const bool moved = n_iter >= 1 && S.ok;
-      centers[2 * m] = moved ? S.cx : J.c0x;
-      centers[2 * m + 1] = moved ? S.cy : J.c0y;
-    }
+    if (tid == 0) put_center(J, n_iter >= 1 && S.ok, S, m, centers, found);
     return;
   }
   if (tid == 0) W.state[(size_t)(J.n_iter & 1) * n_jobs + m] = S;
@@ -1288,25 +1291,20 @@ __global__ __launch_bounds__(64) void k_take_stops(const RefineJobDev* __restric
   }
 }
 
-// The centre the grid search moves to after its first iteration (the job's
-// start when that iteration found no readable grid point), a wavefront per
-// marker.
-__global__ __launch_bounds__(64) void k_refine_coarse_out(const RefineJobDev* __restrict__ jobs,
-                                                          int n_samples, int grid_n,
-                                                          RefineWork W,
-                                                          float* __restrict__ centers) {
+// The centre each marker has reached after at most `iters` launches of
+// k_refine_iter, a wavefront per marker.
+__global__ __launch_bounds__(64) void k_refine_centers(const RefineJobDev* __restrict__ jobs,
+                                                       int iters, int n_samples, int grid_n,
+                                                       RefineWork W, float2* __restrict__ centers,
+                                                       int* __restrict__ found) {
   __shared__ RefineStateDev S;
   const int m = blockIdx.x;
   const RefineJobDev& J = jobs[m];
-  const bool searched = J.n_iter >= 1;
+  const int it = min(J.n_iter, iters);
   PointRecord rec;
-  load_records(searched ? 1 : 0, m, gridDim.x, n_samples, grid_n, W, rec);
-  state_at(J, searched ? 1 : 0, n_samples, grid_n, rec, S);
-  if (threadIdx.x == 0) {
-    const bool moved = searched && S.ok;
-    centers[2 * m] = moved ? S.cx : J.c0x;
-    centers[2 * m + 1] = moved ? S.cy : J.c0y;
-  }
+  load_records(it, m, gridDim.x, n_samples, grid_n, W, rec);
+  state_at(J, it, n_samples, grid_n, rec, S);
+  if (threadIdx.x == 0) put_center(J, it >= 1 && S.ok, S, m, centers, found);
 }
 
 Samples samples(int n) { return Samples{n, 1.0 / (double)(n - 1)}; }
@@ -1350,27 +1348,34 @@ constexpr int kSearchBlock = 512, kSearchBlockWide = 704;
 static_assert(G2MAX * kMaxSumChunks <= kSearchBlockWide, "a lane per grid point and chunk");
 
 void launch_search(const RefineJobDev* jobs, int n_jobs, int n_samples, int grid_n, int iters,
-                   const RefineWork& work, float* centers, hipStream_t s) {
+                   const RefineWork& work, float2* centers, int* found, hipStream_t s) {
   const Samples ns = samples(n_samples);
   if (grid_n * grid_n * sum_chunks_of(n_samples) <= kSearchBlock)
     k_refine_search<kSearchBlock><<<n_jobs, kSearchBlock, 0, s>>>(jobs, ns, grid_n, iters, work,
-                                                                  centers);
+                                                                  centers, found);
   else
     k_refine_search<kSearchBlockWide><<<n_jobs, kSearchBlockWide, 0, s>>>(jobs, ns, grid_n, iters,
-                                                                          work, centers);
+                                                                          work, centers, found);
+}
+
+void launch_iterations(const RefineJobDev* jobs, int n_jobs, int iters, int max_cuts, int n_samples,
+                       int grid_n, const RefineWork& work, hipStream_t s) {
+  const SearchShape sh = search_shape(max_cuts, grid_n, chunks_per_block(n_jobs, n_samples));
+  for (int it = 0; it < iters; ++it)
+    launch_iteration(jobs, n_jobs, it, sh, n_samples, grid_n, work, s);
 }
 
 }  // namespace
 
-int launch_refine_coarse(const RefineJobDev* jobs, int n_jobs, int max_cuts, int n_samples,
-                         int grid_n, const RefineWork& work, float* centers, hipStream_t s) {
+int launch_refine_centers(const RefineJobDev* jobs, int n_jobs, int iters, int max_cuts,
+                          int n_samples, int grid_n, const RefineWork& work, float2* centers,
+                          int* found, hipStream_t s) {
   if (n_jobs <= 0) return 0;
   if (n_jobs >= kSearchMinJobs) {
-    launch_search(jobs, n_jobs, n_samples, grid_n, 1, work, centers, s);
+    launch_search(jobs, n_jobs, n_samples, grid_n, iters, work, centers, found, s);
   } else {
-    const SearchShape sh = search_shape(max_cuts, grid_n, chunks_per_block(n_jobs, n_samples));
-    launch_iteration(jobs, n_jobs, 0, sh, n_samples, grid_n, work, s);
-    k_refine_coarse_out<<<n_jobs, 64, 0, s>>>(jobs, n_samples, grid_n, work, centers);
+    launch_iterations(jobs, n_jobs, iters, max_cuts, n_samples, grid_n, work, s);
+    k_refine_centers<<<n_jobs, 64, 0, s>>>(jobs, iters, n_samples, grid_n, work, centers, found);
   }
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
@@ -1404,13 +1409,8 @@ int launch_refine(const RefineJobDev* jobs, int n_jobs, int max_iter, int max_cu
                   RefineOutDev* out, float* dist, hipStream_t s) {
   if (n_jobs <= 0) return 0;
   const int searched = n_jobs >= kSearchMinJobs;
-  if (searched) {
-    launch_search(jobs, n_jobs, n_samples, grid_n, max_iter, work, nullptr, s);
-  } else {
-    const SearchShape sh = search_shape(max_cuts, grid_n, chunks_per_block(n_jobs, n_samples));
-    for (int it = 0; it < max_iter; ++it)
-      launch_iteration(jobs, n_jobs, it, sh, n_samples, grid_n, work, s);
-  }
+  if (searched) launch_search(jobs, n_jobs, n_samples, grid_n, max_iter, work, nullptr, nullptr, s);
+  else launch_iterations(jobs, n_jobs, max_iter, max_cuts, n_samples, grid_n, work, s);
   k_refine_final<<<n_jobs, kFinalBlock, 0, s>>>(jobs, samples(n_samples), grid_n, inv_ratio, bank_rows,
                                                  bank_cols, work, nullptr, nullptr, nullptr,
                                                  searched, out, dist);

@@ -1,7 +1,7 @@
 // The grid search of cctagx_refiner_grid as one call that allocates nothing
 // (include/cctag_amd.h, cctagx_refine_grid_static).  Every device buffer the
 // call needs -- the frame, its quad image, the jobs, the grid search's
-// per-marker state, grid records and homographies, the read-out's outputs
+// per-marker state, grid records and homographies, the centres
 // -- lives in `scratch`, a fixed array of device memory that each GPU holds
 // from the library's load until the process ends.  Host code reaches it
 // through the address hipGetSymbolAddress returns on that device; the
@@ -27,6 +27,11 @@ constexpr size_t kMaxPixels = CCTAGX_STATIC_MAX_PIXELS;
 constexpr int kMaxMarkers = CCTAGX_STATIC_MAX_MARKERS;
 constexpr int kG2 = kMaxGrid * kMaxGrid;
 
+struct Centers {
+  float2 center[kMaxMarkers];
+  int found[kMaxMarkers];
+};
+
 constexpr size_t up256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Byte offsets of the buffers inside the array.
@@ -38,8 +43,7 @@ constexpr size_t kPoints = up256(kState + sizeof(RefineStateDev) * 2 * kMaxMarke
 constexpr size_t kPart = up256(kPoints + sizeof(RefinePointDev) * 2 * kMaxMarkers * kG2);
 constexpr size_t kHom = up256(kPart + sizeof(double) * 2 * kMaxMarkers * kG2 * kMaxRefineSums);
 constexpr size_t kOut = up256(kHom + sizeof(RefineHomDev) * kMaxMarkers * kG2);
-constexpr size_t kDist = up256(kOut + sizeof(RefineOutDev) * kMaxMarkers);
-constexpr size_t kScratchBytes = up256(kDist + sizeof(float));
+constexpr size_t kScratchBytes = up256(kOut + sizeof(Centers));
 static_assert(kScratchBytes <= 11400000, "the size the C ABI documents (11.4 MB)");
 
 constexpr int kMaxDevices = 64;
@@ -111,8 +115,7 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
   work.points = reinterpret_cast<RefinePointDev*>(base + kPoints);
   work.part = reinterpret_cast<double*>(base + kPart);
   work.hom = reinterpret_cast<RefineHomDev*>(base + kHom);
-  RefineOutDev* d_out = reinterpret_cast<RefineOutDev*>(base + kOut);
-  float* d_dist = reinterpret_cast<float*>(base + kDist);
+  float2* d_out = reinterpret_cast<float2*>(base + kOut);
 
   // per-marker constants on the host, as cctagx_refiner_set_markers makes
   // them (the first marker's (a+b)/2 conditions every marker)
@@ -153,7 +156,7 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
       d.n_cuts = m.n_cuts;
       d.c0x = m.center0[0];
       d.c0y = m.center0[1];
-      d.dist_offset = 0;  // no bank rows: the read-out writes no distances
+      d.dist_offset = 0;
       d.sel_index = -1;
       for (int k = 0; k < m.n_cuts; ++k) d.stops[k] = make_float2(m.stops[k][0], m.stops[k][1]);
       max_iter = std::max(max_iter, r.n_iter);
@@ -166,22 +169,24 @@ int cctagx_refine_grid_static(const cctagx_params* params, const uint8_t* gray, 
   }
 
   hipStream_t s = nullptr;  // the current device's null stream
-  CCTAGX_HIP(hipMemcpy2DAsync(d_img, width, gray, stride, width, height, hipMemcpyHostToDevice, s));
-  if (launch_quads(d_img, width, height, d_quad, s)) return CCTAGX_ERR_HIP;
-  RefineOutDev out[kMaxMarkers];
+  size_t pitch = 0;
+  CCTAGX_HIP(upload_rows(d_img, kMaxPixels, gray, width, height, stride, s, &pitch));
+  if (launch_quads(d_img, width, height, pitch, d_quad, s)) return CCTAGX_ERR_HIP;
+  Centers out;
   if (n_jobs > 0) {
     CCTAGX_HIP(hipMemcpyAsync(d_jobs, jobs, sizeof(RefineJobDev) * n_jobs, hipMemcpyHostToDevice, s));
-    if (launch_refine(d_jobs, n_jobs, max_iter, max_cuts, kc.n_samples, hp.imaged_center_n_grid_sample,
-                      nullptr, 0, 0, work, d_out, d_dist, s))
+    if (launch_refine_centers(d_jobs, n_jobs, max_iter, max_cuts, kc.n_samples,
+                              hp.imaged_center_n_grid_sample, work, d_out,
+                              reinterpret_cast<int*>(d_out + kMaxMarkers), s))
       return CCTAGX_ERR_HIP;
-    CCTAGX_HIP(hipMemcpyAsync(out, d_out, sizeof(RefineOutDev) * n_jobs, hipMemcpyDeviceToHost, s));
+    CCTAGX_HIP(hipMemcpyAsync(&out, d_out, sizeof(out), hipMemcpyDeviceToHost, s));
   }
   CCTAGX_HIP(hipStreamSynchronize(s));
   for (int i = 0; i < n; ++i) {
     const int j = job_of[i];
-    ok[i] = j >= 0 && out[j].ok;
-    centers[2 * i] = ok[i] ? out[j].cx : 0.f;
-    centers[2 * i + 1] = ok[i] ? out[j].cy : 0.f;
+    ok[i] = j >= 0 && out.found[j];
+    centers[2 * i] = ok[i] ? out.center[j].x : 0.f;
+    centers[2 * i + 1] = ok[i] ? out.center[j].y : 0.f;
   }
   return CCTAGX_OK;
 }
