@@ -93,7 +93,6 @@ __device__ __forceinline__ void condition(float& x, float& y, const float* T) {
   y = c1 / c2;
 }
 
-// boost::accumulators immediate mean and variance, one sample at a time.
 // x / n, correctly rounded, for a float x and an integer 1 <= n <=
 // kMaxSamples, from inv_n = 1/n rounded to double: the double product is
 // within 2^-52 (relative) of x/n; x/n, a 24-bit significand over an
@@ -104,115 +103,201 @@ __device__ __forceinline__ void condition(float& x, float& y, const float* T) {
 __device__ __forceinline__ double div_n_product(float x, double inv_n) { return (double)x * inv_n; }
 __device__ __forceinline__ bool div_n_tiny(double p) { return p != 0.0 && fabs(p) < 0x1p-126; }
 
-// 1/n in double for n = 1 .. kMaxSamples (entry 0 unused), by the block.
-__device__ __forceinline__ void fill_inv(double* inv) {
-  for (int q = threadIdx.x; q <= kMaxSamples; q += blockDim.x) inv[q] = 1.0 / (double)q;
-}
+// n in float and 1/n in double for n = 0 .. kMaxSamples (1/0 unused).  Every
+// lane is at the same count, so these are scalar loads, a batch at a time.
+struct CountTable {
+  double inv[kMaxSamples + 1];
+  float n[kMaxSamples + 1];
+  constexpr CountTable() : inv{}, n{} {
+    for (int q = 0; q <= kMaxSamples; ++q) {
+      inv[q] = q ? 1.0 / (double)q : 0.0;
+      n[q] = (float)q;
+    }
+  }
+};
+__constant__ const CountTable kCount;
 
-// Running mean and variance, one value at a time (at most kMaxSamples).
-// The reciprocals a step needs are read from fill_inv's table one step
-// ahead, so the table's latency stays off the chain of products.  With
-// EXACT false a product in the subnormal range (where it need not round to
-// the quotient) is only recorded in `tiny`, keeping branches off the chain:
-// the caller then runs the same values through MeanVar<true>, which divides
-// there, so the result is always the division's.
+// boost::accumulators immediate mean and variance, one non-negative value at
+// a time (at most kMaxSamples; cnt, the same in every lane, counts this one).
+// With EXACT false every quotient is a double product.  That is the division
+// while no nonzero value or squared deviation is below 2^-100 (the mean and
+// the variance then stay above 2^-120 or zero); `low` remembers the smallest
+// of them (their bits less one, so that zero is the largest), and the caller
+// runs the values again through the dividing form where it was too small:
+// the chain itself has no test and no branch.
 template <bool EXACT>
 struct MeanVar {
   float mean = 0.f, var = 0.f;
-  unsigned cnt = 0;
-  bool tiny = false;
-  const double* inv;
-  double inv_cnt, inv_prev;  // 1/(cnt + 1) and 1/cnt for the next add
-  __device__ explicit MeanVar(const double* table) : inv(table), inv_cnt(table[1]), inv_prev(0.0) {}
-  __device__ __forceinline__ void add(float v) {
-    ++cnt;
-    const double inv_next = inv[min(cnt + 1, (unsigned)kMaxSamples)];
-    const float before = (float)(cnt - 1);
+  uint32_t low = ~0u;
+  __device__ __forceinline__ bool tiny() const { return low < 0x0d800000u; }  // 2^-100
+  __device__ __forceinline__ void add(float v, int cnt) {
+    const float before = kCount.n[cnt - 1];
     const float xm = mean * before + v;
-    const double pm = div_n_product(xm, inv_cnt);
-    mean = (float)pm;
-    if (EXACT) {
-      if (div_n_tiny(pm)) mean = xm / (float)cnt;
-    } else {
-      tiny |= div_n_tiny(pm);
-    }
+    if (EXACT) mean = xm / (float)cnt;
+    else mean = (float)div_n_product(xm, kCount.inv[cnt]);
     if (cnt > 1) {
       const float t = v - mean;
       const float xa = var * before, xb = t * t;
-      const double pa = div_n_product(xa, inv_cnt), pb = div_n_product(xb, inv_prev);
-      float a = (float)pa, b = (float)pb;
       if (EXACT) {
-        if (div_n_tiny(pa)) a = xa / (float)cnt;
-        if (div_n_tiny(pb)) b = xb / before;
+        var = xa / (float)cnt + xb / before;
       } else {
-        tiny |= div_n_tiny(pa) | div_n_tiny(pb);
+        var = (float)div_n_product(xa, kCount.inv[cnt]) + (float)div_n_product(xb, kCount.inv[cnt - 1]);
+        low = min(low, min(__float_as_uint(xb) - 1u, __float_as_uint(v) - 1u));
       }
-      var = a + b;
+    } else if (!EXACT) {
+      low = min(low, __float_as_uint(v) - 1u);
     }
-    inv_prev = inv_cnt;
-    inv_cnt = inv_next;
   }
 };
 
-// Identification.cpp:396-459 for a cut whose signal is only consumed
-// sample by sample; returns false when a sample falls outside the image
-// (the caller then discards what f saw).  Sample positions follow the
-// reference's running sums; the image reads of kWalkBatch samples are issued
-// together so their latencies overlap (a sample past the end re-reads the
-// batch's first one, which is inside).
+// Identification.cpp:396-459: the n samples of a cut, kWalkBatch at a time.
+// Positions follow the reference's running sums, which are monotone in x and
+// in y: a batch lies inside the image when its last sample (and the cut's
+// first) does.  The image reads of a batch are issued together.
 constexpr int kWalkBatch = 20;
-
-template <class F>
-__device__ bool cut_walk(const Img& im, float sx, float sy, float ex, float ey, float begin, float end,
-                         int n, F&& f) {
-  float xs, ys, xe, ye;
-  const float diffX = ex - sx, diffY = ey - sy;
-  if (begin != 0.f) {
-    xs = sx + diffX * begin;
-    ys = sy + diffY * begin;
-  } else {
-    xs = sx;
-    ys = sy;
+struct WalkBatch {
+  float fx[kWalkBatch], fy[kWalkBatch];
+  uint32_t q[kWalkBatch];
+  __device__ __forceinline__ float value(int t) const { return bilinear2(fx[t], fy[t], q[t]) / 2; }
+};
+struct CutWalk {
+  float x, y, stepX, stepY;
+  bool inside;  // every sample so far
+  __device__ __forceinline__ CutWalk(const Img& im, float sx, float sy, float ex, float ey, float begin,
+                                     float end, int n) {
+    float xe, ye;
+    const float diffX = ex - sx, diffY = ey - sy;
+    if (begin != 0.f) {
+      x = sx + diffX * begin;
+      y = sy + diffY * begin;
+    } else {
+      x = sx;
+      y = sy;
+    }
+    if (end != 1.f) {
+      xe = sx + diffX * end;
+      ye = sy + diffY * end;
+    } else {
+      xe = ex;
+      ye = ey;
+    }
+    stepX = (xe - x) / ((float)n - 1.f);
+    stepY = (ye - y) / ((float)n - 1.f);
+    inside = in(im, x, y);
   }
-  if (end != 1.f) {
-    xe = sx + diffX * end;
-    ye = sy + diffY * end;
-  } else {
-    xe = ex;
-    ye = ey;
+  static __device__ __forceinline__ bool in(const Img& im, float x, float y) {
+    return x >= 1.f && x < (float)(im.w - 1) && y >= 1.f && y < (float)(im.h - 1);
   }
-  const float stepX = (xe - xs) / ((float)n - 1.f), stepY = (ye - ys) / ((float)n - 1.f);
-  const float xmax = (float)(im.w - 1), ymax = (float)(im.h - 1);
-  float x = xs, y = ys;
-  for (int i0 = 0; i0 < n; i0 += kWalkBatch) {
+  // The next `live` samples (1 <= live <= kWalkBatch, the same in every
+  // lane); nothing is read once a sample was outside.
+  __device__ __forceinline__ void fetch(const Img& im, int live, WalkBatch& b) {
     float px[kWalkBatch], py[kWalkBatch];
-    bool inside = true;
+    float lx = x, ly = y;
 #pragma unroll
     for (int t = 0; t < kWalkBatch; ++t) {
-      px[t] = x;
-      py[t] = y;
-      if (i0 + t < n) inside &= (x >= 1.f && x < xmax && y >= 1.f && y < ymax);
+      px[t] = t < live ? x : px[0];
+      py[t] = t < live ? y : py[0];
+      lx = t < live ? x : lx;
+      ly = t < live ? y : ly;
       x += stepX;
       y += stepY;
     }
-    if (!inside) return false;
-    uint32_t qd[kWalkBatch];
+    inside = inside && in(im, lx, ly);
+    if (!inside) return;
 #pragma unroll
     for (int t = 0; t < kWalkBatch; ++t) {
-      const bool live = i0 + t < n;
-      qd[t] = im.quad((int)(live ? px[t] : px[0]), (int)(live ? py[t] : py[0]));
+      b.q[t] = im.quad24((uint32_t)(int)px[t], (uint32_t)(int)py[t]);
+      b.fx[t] = __builtin_amdgcn_fractf(px[t]);
+      b.fy[t] = __builtin_amdgcn_fractf(py[t]);
     }
-#pragma unroll
-    for (int t = 0; t < kWalkBatch; ++t)
-      if (i0 + t < n) f(i0 + t, bilinear_of(px[t], py[t], qd[t]));
   }
-  return true;
+};
+
+// The mean and variance of a cut's samples, the next batch's reads in flight
+// while one is added up.  False when a sample falls outside the image.
+template <bool EXACT>
+__device__ __forceinline__ bool cut_stats(const Img& im, float cx, float cy, float sx, float sy,
+                                          float begin, int n, MeanVar<EXACT>& mv) {
+  CutWalk walk(im, cx, cy, sx, sy, begin, 1.f, n);
+  WalkBatch a, b;
+  auto take = [&](const WalkBatch& w, int i0) {
+    if (i0 + kWalkBatch <= n) {
+#pragma unroll
+      for (int t = 0; t < kWalkBatch; ++t) mv.add(w.value(t), i0 + t + 1);
+    } else {
+#pragma unroll
+      for (int t = 0; t < kWalkBatch; ++t)
+        if (i0 + t < n) mv.add(w.value(t), i0 + t + 1);
+    }
+  };
+  walk.fetch(im, min(kWalkBatch, n), a);
+  for (int i0 = 0; i0 < n && walk.inside; i0 += 2 * kWalkBatch) {
+    if (i0 + kWalkBatch < n) walk.fetch(im, min(kWalkBatch, n - i0 - kWalkBatch), b);
+    if (!walk.inside) return false;
+    take(a, i0);
+    if (i0 + kWalkBatch >= n) break;
+    if (i0 + 2 * kWalkBatch < n) walk.fetch(im, min(kWalkBatch, n - i0 - 2 * kWalkBatch), a);
+    if (!walk.inside) return false;
+    take(b, i0 + kWalkBatch);
+  }
+  return walk.inside;
 }
 
-__constant__ float kRefineKernels[3][9] = {
+constexpr float kRefineKernels[3][9] = {
     {-0.0000f, -0.0003f, -0.1065f, -0.7863f, .0f, 0.7863f, 0.1065f, 0.0003f, 0.0000f},
     {-0.0044f, -0.0540f, -0.2376f, -0.3450f, .0f, 0.3450f, 0.2376f, 0.0540f, 0.0044f},
     {-0.0366f, -0.1113f, -0.1801f, -0.1594f, .0f, 0.1594f, 0.1801f, 0.1113f, 0.0366f}};
+
+// The strongest response of each refinement kernel along a signal of N
+// samples (value(i); beyond the ends its first and last), and where
+// (Identification.cpp:630-657).  A tap of weight zero adds nothing to a sum
+// and is left out.
+template <int N, class F>
+__device__ __forceinline__ void edge_responses(const F& value, float* key, float* loc) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    float best = 0.f;
+    int bi = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float tmp = 0;
+#pragma unroll
+      for (int j = 0; j < 9; ++j)
+        if (kRefineKernels[k][j] != 0.f) {
+          const int r = i - 4 + j;
+          tmp += value(r < 0 ? 0 : r >= N ? N - 1 : r) * kRefineKernels[k][j];
+        }
+      if (i == 0 || tmp > best) {
+        best = tmp;
+        bi = i;
+      }
+    }
+    key[k] = best;
+    loc[k] = (float)bi;
+  }
+}
+
+// (the same for any n, in a loop)
+template <class F>
+__device__ __forceinline__ void edge_responses_any(int n, const F& value, float* key, float* loc) {
+  for (int k = 0; k < 3; ++k) {
+    float best = 0.f;
+    int bi = 0;
+    for (int i = 0; i < n; ++i) {
+      float tmp = 0;
+      for (int j = 0; j < 9; ++j) {
+        const int r = i - 4 + j;
+        tmp += value(r < 0 ? 0 : r >= n ? n - 1 : r) * kRefineKernels[k][j];
+      }
+      if (i == 0 || tmp > best) {
+        best = tmp;
+        bi = i;
+      }
+    }
+    key[k] = best;
+    loc[k] = (float)bi;
+  }
+}
 
 // One thread per outer point (n <= kMaxOuterPoints = blockDim.x).  The
 // counts, the maximum variance and the candidates' ranks come from block
@@ -232,9 +317,6 @@ __global__ __launch_bounds__(kSelectBlock) void k_select_cuts(const SelectJobDev
   __shared__ int w_cnt[NW], w_cand[NW];
   __shared__ float w_max[NW];
   __shared__ float ref_sig[kMaxRefineSamples][kSelectBlock];  // the thread's refinement cut
-  __shared__ double inv[kMaxSamples + 1];
-  fill_inv(inv);
-  __syncthreads();
   const SelectJobDev J = jobs[blockIdx.x];
   const Img im{J.quad, J.iw, J.ih};
   const int n = J.n_outer;
@@ -244,14 +326,12 @@ __global__ __launch_bounds__(kSelectBlock) void k_select_cuts(const SelectJobDev
   float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
   if (t < n) {
     s = pts[J.pt_offset + t];
-    MeanVar<false> mv(inv);
-    valid = cut_walk(im, J.cx, J.cy, s.x, s.y, start_sig, 1.f, n_samples,
-                     [&](int, float v) { mv.add(v); });
+    MeanVar<false> mv;
+    valid = cut_stats(im, J.cx, J.cy, s.x, s.y, start_sig, n_samples, mv);
     var = mv.var;
-    if (valid && mv.tiny) {  // the same walk again, dividing where a product was subnormal
-      MeanVar<true> me(inv);
-      cut_walk(im, J.cx, J.cy, s.x, s.y, start_sig, 1.f, n_samples,
-               [&](int, float v) { me.add(v); });
+    if (valid && mv.tiny()) {  // the same walk again, dividing
+      MeanVar<true> me;
+      cut_stats(im, J.cx, J.cy, s.x, s.y, start_sig, n_samples, me);
       var = me.var;
     }
   }
@@ -296,29 +376,30 @@ __global__ __launch_bounds__(kSelectBlock) void k_select_cuts(const SelectJobDev
     const float hx = half * gdx, hy = half * gdy;
     const float psx = s.x - hx, psy = s.y - hy;
     const float pex = s.x + half * gdx, pey = s.y + half * gdy;
-    float (*sig)[kSelectBlock] = ref_sig;
-    const bool ok =
-        cut_walk(im, psx, psy, pex, pey, 0.f, 1.f, n_ref, [&](int i, float v) { sig[i][t] = v; });
-    if (ok) {
-      float key[3], loc[3];
-      for (int k = 0; k < 3; ++k) {
-        float best = 0.f;
-        int bi = 0;
-        for (int i = 0; i < n_ref; ++i) {
-          float tmp = 0;
-          for (int j = 0; j < 9; ++j) {
-            const int r = i - 4 + j;
-            const float v = r < 0 ? sig[0][t] : (r >= n_ref ? sig[n_ref - 1][t] : sig[r][t]);
-            tmp += v * kRefineKernels[k][j];
-          }
-          if (i == 0 || tmp > best) {
-            best = tmp;
-            bi = i;
-          }
-        }
-        key[k] = best;
-        loc[k] = (float)bi;
+    CutWalk walk(im, psx, psy, pex, pey, 0.f, 1.f, n_ref);
+    float key[3], loc[3];
+    if (n_ref == kWalkBatch) {
+      // (the default: the signal stays in registers)
+      WalkBatch w;
+      walk.fetch(im, kWalkBatch, w);
+      if (walk.inside) {
+        float v[kWalkBatch];
+#pragma unroll
+        for (int i = 0; i < kWalkBatch; ++i) v[i] = w.value(i);
+        edge_responses<kWalkBatch>([&](int i) { return v[i]; }, key, loc);
       }
+    } else {
+      for (int i0 = 0; i0 < n_ref && walk.inside; i0 += kWalkBatch) {
+        WalkBatch w;
+        walk.fetch(im, min(kWalkBatch, n_ref - i0), w);
+        if (!walk.inside) break;
+#pragma unroll
+        for (int i = 0; i < kWalkBatch; ++i)
+          if (i0 + i < n_ref) ref_sig[i0 + i][t] = w.value(i);
+      }
+      if (walk.inside) edge_responses_any(n_ref, [&](int i) { return ref_sig[i][t]; }, key, loc);
+    }
+    if (walk.inside) {
       // std::map<float,float> insert (first of equal keys kept), then the largest key
       int b = 0;
       for (int k = 1; k < 3; ++k)
@@ -1045,7 +1126,6 @@ __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
   // a sample's term of the distance, for each ring parity
   __shared__ float term[2][kMaxCuts][kMaxSamples + 1];
   __shared__ RefineStateDev S;
-  __shared__ double inv[kMaxSamples + 1];
   const int m = blockIdx.x, tid = threadIdx.x, n_jobs = gridDim.x;
   const RefineJobDev& J = jobs[m];
   RefineOutDev& O = out[m];
@@ -1055,7 +1135,6 @@ __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
     return;
   }
   for (int q = tid; q < bank_rows * kMaxRatios; q += kFinalBlock) ratio[q] = inv_ratio[q];
-  fill_inv(inv);
   const int nc = J.n_cuts;
   if (given) {
     if (tid == 0) {
@@ -1122,23 +1201,24 @@ __global__ __launch_bounds__(kFinalBlock) void k_refine_final(
   }
   // orazioDistanceRobust statistics per valid cut (Identification.cpp:88-121)
   if (tid < nc && !((sticky >> tid) & 1u)) {
-    // the signal is read kStatBatch samples at a time (indices clamped,
-    // so the reads are in flight together), then consumed in order
-    constexpr int kStatBatch = 8;
+    // the signal is read kStatBatch samples at a time, so the reads are in
+    // flight together, then consumed in order
+    constexpr int kStatBatch = 10;
     const float* sg = sig[tid];
-    MeanVar<false> mv(inv);
-    for (int i0 = 30; i0 < n_samples; i0 += kStatBatch) {
+    MeanVar<false> mv;
+    int i0 = 30;
+    for (; i0 + kStatBatch <= n_samples; i0 += kStatBatch) {
       float v[kStatBatch];
 #pragma unroll
-      for (int j = 0; j < kStatBatch; ++j) v[j] = sg[min(i0 + j, n_samples - 1)];
+      for (int j = 0; j < kStatBatch; ++j) v[j] = sg[i0 + j];
 #pragma unroll
-      for (int j = 0; j < kStatBatch; ++j)
-        if (i0 + j < n_samples) mv.add(v[j]);
+      for (int j = 0; j < kStatBatch; ++j) mv.add(v[j], i0 - 30 + j + 1);
     }
+    for (; i0 < n_samples; ++i0) mv.add(sg[i0], i0 - 30 + 1);
     float s_mean = mv.mean, s_var = mv.var;
-    if (mv.tiny) {  // again, dividing where a product was subnormal
-      MeanVar<true> me(inv);
-      for (int i = 30; i < n_samples; ++i) me.add(sg[i]);
+    if (mv.tiny()) {  // again, dividing
+      MeanVar<true> me;
+      for (int i = 30; i < n_samples; ++i) me.add(sg[i], i - 30 + 1);
       s_mean = me.mean;
       s_var = me.var;
     }
