@@ -103,6 +103,30 @@ def test_identify_does_not_depend_on_a_failing_first_marker():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_ref,n_samples", [(9, 100), (19, 31), (20, 45), (21, 60), (32, 128)])
+def test_identify_sample_counts(n_ref, n_samples):
+    """Cuts read in batches of 20: the shortest and longest accepted lengths,
+    whole batches and remainders, and edge refinements of fewer and more
+    samples than one batch (20 has its own path).  The bounds do not depend
+    on the counts: a cut's statistics are the oracle's float sequence, and a
+    sum of fewer samples rounds less."""
+    p = _lib.default_params()
+    p.num_samples_outer_edge_points_refinement = n_ref
+    p.sample_cut_length = n_samples
+    img, gts = frames.config_frame(1)
+    border, border_gts = frames.border_frame(7000)
+    for im, gs in ((img, gts), (border, border_gts)):
+        markers = [frames.ident_input(g.H) for g in gs]
+        print("sample counts", n_ref, n_samples, im.shape, len(markers), flush=True)
+        ref = oracle_lib.identify_given(im, markers, p)
+        h, w = im.shape
+        with Detector(w, h, params=p) as det:
+            det.front_end(im)
+            got = det.identify(markers)
+        compare(got, ref, (n_ref, n_samples))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("seed", [7000, 7003])
 def test_detect_border_frames_match_oracle(seed):
     from tests.test_detect_gpu import match
