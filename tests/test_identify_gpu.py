@@ -79,6 +79,18 @@ def test_identify_border_markers(seed):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dw,dh", [(0, 1), (1, 0), (2, 3), (3, 2), (4, 5), (8, 4)])
+def test_identify_frame_remainders(dw, dh):
+    """The sampling words are built four pixels at a time where the width is
+    a multiple of four and one by one elsewhere: markers cut by the last
+    column and row of frames of either kind."""
+    img, gts = frames.border_frame(7003)
+    h, w = img.shape
+    crop = np.ascontiguousarray(img[:h - dh, :w - dw])
+    identify_both(crop, [frames.ident_input(g.H) for g in gts], "crop %d %d" % (dw, dh))
+
+
+@pytest.mark.gpu
 def test_identify_clean_and_faded_markers():
     for k in range(4):
         img, _, m = frames.clean_marker(100 + k)
