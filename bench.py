@@ -88,7 +88,6 @@ def frontend_bytes(name, lv):
             "cc_flatten": N + 4 * N + 4 * N + N,           # cls, labels in/out, root flag
             "thin": N + 4 * N + N + N,                     # cls, labels, roots in; thinned map out
             "compact_count": N,                            # thinned map
-            "compact_scan": 0,
             "compact_write": N + 4 * E + 4 * N + 12 * E + 4 * E,  # map, grads at edges; emap, list, flags
             "descent": 8 * E + 8 * E,                      # list in, before/after out
             "vote": 16 * E + 12 * E,                       # list + links in; chosen, dist, counts out

@@ -38,9 +38,12 @@ struct PlaneCounts {
   int32_t pad;
 };
 
-// Blocks per plane of the two-pass scans over edge points (voter offsets,
+// Blocks per plane of the scans over edge points (voter offsets,
 // seed compaction); each block scans one contiguous range.
 constexpr int kScanBlocks = 64;
+// Words from one range's count to the next: a memory line each, since the
+// atomics of eight XCDs on one line queue behind each other.
+constexpr int kPartStride = 64;
 
 // Tile geometry shared by host launch code and kernels.
 constexpr int kFilterTileW = 64, kFilterTileH = 32;
@@ -92,7 +95,8 @@ struct FrontEndBuffers {
   int32_t* ismax;
   int32_t* seedmark;   // voter index -> point that reached min votes with it
   int32_t* seeds;
-  int32_t* scan_part;  // nplanes x kScanBlocks partial sums of the two-pass scans
+  int32_t* vote_part;  // nplanes x kScanBlocks x kPartStride: votes per scan range
+  int32_t* seed_part;  // nplanes x kScanBlocks x kPartStride: seeds per scan range
   PlaneCounts* counts; // nplanes
 };
 

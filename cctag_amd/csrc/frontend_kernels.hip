@@ -759,52 +759,29 @@ __global__ __launch_bounds__(256) void k_compact_count(const PlaneDesc* __restri
   if (threadIdx.x == 0) tcount[blockIdx.x] = total;
 }
 
-// Per-plane exclusive scan of chunk counts (one 1024-thread block per plane).
-__global__ __launch_bounds__(1024) void k_compact_scan(const PlaneDesc* __restrict__ P, int np,
-                                                        int32_t* __restrict__ tcount,
-                                                        PlaneCounts* __restrict__ counts) {
-  __shared__ int wsum[16];
-  __shared__ int carry;
-  const int p = blockIdx.x;
-  const PlaneDesc d = P[p];
-  const int nchunks = (d.w * d.h + kChunk - 1) / kChunk;
-  int32_t* a = tcount + d.tile_c;
-  if (threadIdx.x == 0) carry = 0;
+// Sum of v over the block (256 threads), in every thread.
+__device__ __forceinline__ int block_sum(int v) {
+  __shared__ int wsum[4];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
   __syncthreads();
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int base = 0; base < nchunks; base += 1024) {
-    const int i = base + threadIdx.x;
-    const int v = i < nchunks ? a[i] : 0;
-    int incl = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int n = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += n;
-    }
-    if (lane == 63) wsum[wid] = incl;
-    __syncthreads();
-    int wb = 0, tot = 0;
-    for (int w = 0; w < 16; ++w) {
-      if (w < wid) wb += wsum[w];
-      tot += wsum[w];
-    }
-    if (i < nchunks) a[i] = carry + wb + incl - v;
-    __syncthreads();
-    if (threadIdx.x == 0) carry += tot;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) counts[p].n_edges = carry;
+  return wsum[0] + wsum[1] + wsum[2] + wsum[3];
 }
 
 // Writes the edge list and, per 32-pixel mask word, the index of its first
 // edge pixel (a point's index is then that plus the edges before it in the
-// word).
+// word).  A block adds up the chunk counts before its own itself, at most
+// 2025 of them at 3840x2160, eight per thread (1.3 us more), instead of
+// waiting 4.8 for a launch that scans them.  The first block of a plane also clears the sums
+// that the vote and the seeds are counted into (scan_range).
 __global__ __launch_bounds__(256) void k_compact_write(
     const PlaneDesc* __restrict__ P, int np, const uint8_t* __restrict__ edges,
     const int16_t* __restrict__ dx, const int16_t* __restrict__ dy,
-    const int32_t* __restrict__ tcount, int32_t* __restrict__ erank, int16_t* __restrict__ ex,
+    const int32_t* __restrict__ tcount, PlaneCounts* __restrict__ counts,
+    int32_t* __restrict__ erank, int16_t* __restrict__ ex,
     int16_t* __restrict__ ey, int16_t* __restrict__ egx, int16_t* __restrict__ egy,
-    int32_t* __restrict__ vcount, int32_t* __restrict__ seedmark) {
+    int32_t* __restrict__ vcount, int32_t* __restrict__ seedmark, int32_t* __restrict__ vote_part,
+    int32_t* __restrict__ seed_part) {
   const int p = plane_of<F_TILE_C>(P, np, blockIdx.x);
   const PlaneDesc d = P[p];
   const int c = blockIdx.x - d.tile_c;
@@ -817,8 +794,16 @@ __global__ __launch_bounds__(256) void k_compact_write(
     e[k] = (b + k < n) ? edges[d.pix + b + k] : 0;
     cnt += e[k] == 255;
   }
+  int before = 0;
+  for (int k = threadIdx.x; k < c; k += 256) before += tcount[d.tile_c + k];
+  before = block_sum(before);
   int total;
-  int idx = tcount[blockIdx.x] + block_exclusive_scan(cnt, &total);
+  int idx = before + block_exclusive_scan(cnt, &total);
+  if (c == 0 && threadIdx.x < kScanBlocks) {
+    vote_part[(p * kScanBlocks + threadIdx.x) * kPartStride] = 0;
+    seed_part[(p * kScanBlocks + threadIdx.x) * kPartStride] = 0;
+  }
+  if ((c + 1) * kChunk >= n && threadIdx.x == 0) counts[p].n_edges = before + total;
   // even lanes start a 32-pixel word
   if ((threadIdx.x & 1) == 0 && b < n) erank[(d.pix >> 5) + (b >> 5)] = idx;
 #pragma unroll
@@ -992,6 +977,48 @@ __global__ __launch_bounds__(256) void k_descent(const PlaneDesc* __restrict__ P
 }
 
 // ---------------------------------------------------------------------------
+// Scans over a plane's edge points (voter offsets, seeds): kScanBlocks blocks
+// per plane, block b owning one contiguous range of whole kScanStep-point
+// steps.  The kernel that produces what is scanned also counts it per range
+// (in LDS, then one atomic per range that the block met), so a scan block
+// has the sum of the ranges before its own without a launch that adds them
+// up; such a launch took 4.6 us at 1920x1080, most of it the launch.  The
+// counts lie a memory line apart (kPartStride): side by side, the atomics of
+// 2048 blocks took k_vote from 56 to 67 us at 3840x2160 and k_voters_finish
+// from 16 to 28; a line apart they are 59 and 18.  From the compaction to the
+// seeds the kernels concerned take 35, 45 and 158 us at 640x480, 1920x1080
+// and 3840x2160, against 46, 56 and 165 with launches of their own for the
+// three sums.
+constexpr int kScanStep = 1024;  // threads of a scan block = points per step
+
+__device__ __forceinline__ int scan_steps(int n) {  // steps per range
+  const int per = (n + kScanBlocks - 1) / kScanBlocks;
+  return (per + kScanStep - 1) / kScanStep;
+}
+__device__ __forceinline__ void scan_range(int n, int& lo, int& hi) {
+  const int chunk = scan_steps(n) * kScanStep;
+  lo = min(n, (int)blockIdx.x * chunk);
+  hi = min(n, lo + chunk);
+}
+
+// A block's counts per range of n points; every thread of the block calls
+// the constructor and flush.
+struct RangeCounts {
+  int* lds;  // kScanBlocks
+  int steps;
+  __device__ RangeCounts(int* lds_, int n) : lds(lds_), steps(max(scan_steps(n), 1)) {
+    for (int t = threadIdx.x; t < kScanBlocks; t += blockDim.x) lds[t] = 0;
+    __syncthreads();
+  }
+  __device__ void count(int point) { atomicAdd(lds + (point / kScanStep) / steps, 1); }
+  __device__ void flush(int32_t* part) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < kScanBlocks; t += blockDim.x)
+      if (lds[t]) atomicAdd(part + t * kPartStride, lds[t]);
+  }
+};
+
+// ---------------------------------------------------------------------------
 // a9: vote chain walk (Vote.cpp:101-243).  Gradients are small integers, so
 // the dot products are exact; distances are sqrt of exact integer sums.
 __device__ __forceinline__ float neg_dot(const int16_t* gx, const int16_t* gy, int a, int b) {
@@ -1013,9 +1040,12 @@ __global__ __launch_bounds__(256) void k_vote(const PlaneDesc* __restrict__ P,
                                                float ratio, float angle,
                                                int32_t* __restrict__ chosen,
                                                float* __restrict__ tdist,
-                                               int32_t* __restrict__ vcount) {
+                                               int32_t* __restrict__ vcount,
+                                               int32_t* __restrict__ part) {
+  __shared__ int range_votes[kScanBlocks];
   const PlaneDesc d = P[blockIdx.y];
   const int n = counts[blockIdx.y].n_edges;
+  RangeCounts votes(range_votes, n);
   const int16_t* X = ex + d.pix;
   const int16_t* Y = ey + d.pix;
   const int16_t* GX = egx + d.pix;
@@ -1062,8 +1092,12 @@ __global__ __launch_bounds__(256) void k_vote(const PlaneDesc* __restrict__ P,
     }
     chosen[d.pix + ip] = choosen;
     tdist[d.pix + ip] = total;
-    if (choosen >= 0) atomicAdd(vcount + d.pix + choosen, 1);
+    if (choosen >= 0) {
+      atomicAdd(vcount + d.pix + choosen, 1);
+      votes.count(choosen);
+    }
   }
+  votes.flush(part + blockIdx.y * kScanBlocks * kPartStride);
 }
 
 // ---------------------------------------------------------------------------
@@ -1072,19 +1106,6 @@ __global__ __launch_bounds__(256) void k_vote(const PlaneDesc* __restrict__ P,
 // filled with atomics, then each list sorted ascending (the CPU pushes voters
 // in index order), flow length accumulated in that order, and the point's
 // seed key (the voter that brought it to min votes) recorded.
-// Two-pass scans over a plane's edge points: kScanBlocks blocks per plane,
-// block b owning one contiguous range of whole 1024-point steps.  Pass one
-// stores each block's sum, pass two adds the sums of the blocks before it
-// and scans its range.
-constexpr int kScanStep = 1024;  // threads of a scan block = points per step
-
-__device__ __forceinline__ void scan_range(int n, int& lo, int& hi) {
-  const int per = (n + kScanBlocks - 1) / kScanBlocks;
-  const int chunk = (per + kScanStep - 1) / kScanStep * kScanStep;
-  lo = min(n, (int)blockIdx.x * chunk);
-  hi = min(n, lo + chunk);
-}
-
 // Block-wide inclusive scan of v (1024 threads); *total gets the block sum.
 __device__ __forceinline__ int block_incl_scan(int v, int* wsum, int* total) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -1106,11 +1127,11 @@ __device__ __forceinline__ int block_incl_scan(int v, int* wsum, int* total) {
   return wb + incl;
 }
 
-// Sum of the blocks before this one (pass two's offset).
+// Sum of the ranges before this block's.
 __device__ __forceinline__ int prior_parts(const int32_t* part) {
   __shared__ int off;
   if (threadIdx.x < 64) {
-    int v = (int)threadIdx.x < (int)blockIdx.x ? part[threadIdx.x] : 0;
+    int v = threadIdx.x < blockIdx.x ? part[threadIdx.x * kPartStride] : 0;
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if (threadIdx.x == 0) off = v;
   }
@@ -1123,22 +1144,6 @@ __device__ __forceinline__ int prior_parts(const int32_t* part) {
 // filled with atomics, then each list sorted ascending (the CPU pushes voters
 // in index order), flow length accumulated in that order, and the point's
 // seed key (the voter that brought it to min votes) recorded.
-__global__ __launch_bounds__(kScanStep) void k_voters_sum(const PlaneDesc* __restrict__ P,
-                                                          const PlaneCounts* __restrict__ counts,
-                                                          const int32_t* __restrict__ vcount,
-                                                          int32_t* __restrict__ part) {
-  __shared__ int wsum[kScanStep / 64];
-  const int p = blockIdx.y;
-  const int32_t* a = vcount + P[p].pix;
-  int lo, hi;
-  scan_range(counts[p].n_edges, lo, hi);
-  int acc = 0;
-  for (int i = lo + threadIdx.x; i < hi; i += kScanStep) acc += a[i];
-  int tot;
-  block_incl_scan(acc, wsum, &tot);
-  if (threadIdx.x == 0) part[p * kScanBlocks + blockIdx.x] = tot;
-}
-
 __global__ __launch_bounds__(kScanStep) void k_voters_scan(const PlaneDesc* __restrict__ P,
                                                            PlaneCounts* __restrict__ counts,
                                                            const int32_t* __restrict__ vcount,
@@ -1153,7 +1158,7 @@ __global__ __launch_bounds__(kScanStep) void k_voters_scan(const PlaneDesc* __re
   int32_t* o = vindex + d.pix + p;
   int lo, hi;
   scan_range(n, lo, hi);
-  int carry = prior_parts(part + p * kScanBlocks);
+  int carry = prior_parts(part + p * kScanBlocks * kPartStride);
   for (int base = lo; base < hi; base += kScanStep) {
     const int i = base + threadIdx.x;
     const int v = i < hi ? a[i] : 0;
@@ -1204,15 +1209,18 @@ __global__ __launch_bounds__(kFinishBlock) void k_voters_finish(const PlaneDesc*
                                                                 int32_t* __restrict__ vlist,
                                                                 float* __restrict__ flow,
                                                                 int32_t* __restrict__ ismax,
-                                                                int32_t* __restrict__ seedmark) {
+                                                                int32_t* __restrict__ seedmark,
+                                                                int32_t* __restrict__ part) {
   __shared__ int32_t stage_in[kFinishStage];
   __shared__ int32_t stage_out[kFinishStage];
   __shared__ float dist_s[kFinishStage];
   __shared__ uint8_t owner[kFinishStage];
   __shared__ int seg_b[kFinishBlock], seg_e[kFinishBlock];
+  __shared__ int range_seeds[kScanBlocks];
   const int p = blockIdx.y;
   const PlaneDesc d = P[p];
   const int n = counts[p].n_edges;
+  RangeCounts seeds(range_seeds, n);
   const int32_t* vi = vindex + d.pix + p;
   int32_t* vl = vlist + d.pix;
   const float* td = tdist + d.pix;
@@ -1267,30 +1275,19 @@ __global__ __launch_bounds__(kFinishBlock) void k_voters_finish(const PlaneDesc*
       }
       flow[d.pix + c] = fl;
       ismax[d.pix + c] = nv >= min_votes ? nv : -1;
-      if (nv >= min_votes)
-        seedmark[d.pix + (staged ? stage_out[b - run_b + min_votes - 1] : vl[b + min_votes - 1])] = c;
+      if (nv >= min_votes) {
+        // (a voter is in one list only, so no seed is marked twice)
+        const int key = staged ? stage_out[b - run_b + min_votes - 1] : vl[b + min_votes - 1];
+        seedmark[d.pix + key] = c;
+        seeds.count(key);
+      }
     }
     __syncthreads();
   }
+  seeds.flush(part + p * kScanBlocks * kPartStride);
 }
 
 // Seeds in the order they reached min votes = ascending key voter index.
-__global__ __launch_bounds__(kScanStep) void k_seeds_sum(const PlaneDesc* __restrict__ P,
-                                                         const PlaneCounts* __restrict__ counts,
-                                                         const int32_t* __restrict__ seedmark,
-                                                         int32_t* __restrict__ part) {
-  __shared__ int wsum[kScanStep / 64];
-  const int p = blockIdx.y;
-  const int32_t* a = seedmark + P[p].pix;
-  int lo, hi;
-  scan_range(counts[p].n_edges, lo, hi);
-  int acc = 0;
-  for (int i = lo + threadIdx.x; i < hi; i += kScanStep) acc += a[i] >= 0;
-  int tot;
-  block_incl_scan(acc, wsum, &tot);
-  if (threadIdx.x == 0) part[p * kScanBlocks + blockIdx.x] = tot;
-}
-
 __global__ __launch_bounds__(kScanStep) void k_seeds(const PlaneDesc* __restrict__ P,
                                                      PlaneCounts* __restrict__ counts,
                                                      const int32_t* __restrict__ seedmark,
@@ -1301,7 +1298,7 @@ __global__ __launch_bounds__(kScanStep) void k_seeds(const PlaneDesc* __restrict
   const PlaneDesc d = P[p];
   int lo, hi;
   scan_range(counts[p].n_edges, lo, hi);
-  int carry = prior_parts(part + p * kScanBlocks);
+  int carry = prior_parts(part + p * kScanBlocks * kPartStride);
   for (int base = lo; base < hi; base += kScanStep) {
     const int i = base + threadIdx.x;
     const int s = i < hi ? seedmark[d.pix + i] : -1;
@@ -1359,10 +1356,9 @@ int launch_front_end(const FrontEndLaunch& L, hipStream_t s, StageTimer* timer) 
   mark("thin");
   k_compact_count<<<L.n_tiles_c, 256, 0, s>>>(P, np, b.edges, b.tcount, b.ebits);
   mark("compact_count");
-  k_compact_scan<<<np, 1024, 0, s>>>(P, np, b.tcount, b.counts);
-  mark("compact_scan");
-  k_compact_write<<<L.n_tiles_c, 256, 0, s>>>(P, np, b.edges, b.dx, b.dy, b.tcount, b.erank,
-                                               b.ex, b.ey, b.egx, b.egy, b.vcount, b.seedmark);
+  k_compact_write<<<L.n_tiles_c, 256, 0, s>>>(P, np, b.edges, b.dx, b.dy, b.tcount, b.counts,
+                                               b.erank, b.ex, b.ey, b.egx, b.egy, b.vcount,
+                                               b.seedmark, b.vote_part, b.seed_part);
   mark("compact_write");
   const dim3 g(L.edge_blocks, np);
   k_descent<<<g, 256, 0, s>>>(P, b.counts, b.ebits, b.erank, b.ex, b.ey, b.egx, b.egy,
@@ -1370,19 +1366,17 @@ int launch_front_end(const FrontEndLaunch& L, hipStream_t s, StageTimer* timer) 
   mark("descent");
   k_vote<<<g, 256, 0, s>>>(P, b.counts, b.ex, b.ey, b.egx, b.egy, b.before, b.after,
                            L.prm.n_crowns, L.prm.ratio_voting, L.prm.angle_voting, b.chosen,
-                           b.tdist, b.vcount);
+                           b.tdist, b.vcount, b.vote_part);
   mark("vote");
   const dim3 gs(kScanBlocks, np);
-  k_voters_sum<<<gs, kScanStep, 0, s>>>(P, b.counts, b.vcount, b.scan_part);
-  k_voters_scan<<<gs, kScanStep, 0, s>>>(P, b.counts, b.vcount, b.scan_part, b.vindex, b.ismax);
+  k_voters_scan<<<gs, kScanStep, 0, s>>>(P, b.counts, b.vcount, b.vote_part, b.vindex, b.ismax);
   mark("voters_scan");
   k_voters_fill<<<g, 256, 0, s>>>(P, b.counts, b.chosen, b.ismax, b.vlist);
   mark("voters_fill");
   k_voters_finish<<<g, kFinishBlock, 0, s>>>(P, b.counts, b.vindex, b.tdist, L.prm.min_votes,
-                                              b.vlist, b.flow, b.ismax, b.seedmark);
+                                              b.vlist, b.flow, b.ismax, b.seedmark, b.seed_part);
   mark("voters_finish");
-  k_seeds_sum<<<gs, kScanStep, 0, s>>>(P, b.counts, b.seedmark, b.scan_part);
-  k_seeds<<<gs, kScanStep, 0, s>>>(P, b.counts, b.seedmark, b.scan_part, b.seeds);
+  k_seeds<<<gs, kScanStep, 0, s>>>(P, b.counts, b.seedmark, b.seed_part, b.seeds);
   mark("seeds", true);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }

@@ -88,6 +88,21 @@ def test_front_end_parity_edge_cases(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("w,h", [(64, 64), (512, 128), (1024, 1024), (1024, 1028), (1536, 1024)])
+def test_front_end_parity_many_edges(w, h):
+    """Rings side by side: edge points everywhere that vote for each other.
+    One chunk of pixels up to 256, 257 and more (a thread adds up more than
+    one), and scan ranges of one, three and five steps of 1024 points."""
+    y, x = np.mgrid[0:h, 0:w]
+    r = np.hypot(x % 64 - 31.5, y % 64 - 31.5)
+    noise = np.random.default_rng(5).normal(0, 4, (h, w))
+    img = np.clip(128 + 90 * np.sign(np.sin(r * (2 * np.pi / 10))) + noise, 0, 255).astype(np.uint8)
+    print("front-end parity many edges", img.shape, flush=True)
+    ref = run_parity(img)
+    assert ref[0]["n_edges"] > 0.15 * w * h and len(ref[0]["seeds"]) > 0.01 * w * h
+
+
+@pytest.mark.gpu
 def test_front_end_repeatable():
     """Two runs on one handle give identical results (union-find and atomics
     leave no trace in the outputs)."""
