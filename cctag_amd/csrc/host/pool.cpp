@@ -35,10 +35,17 @@ bool spin_until(F&& done, int micros) {
 }  // namespace
 
 TaskPool::TaskPool(int threads) {
-  for (int i = 1; i < threads; ++i) workers_.emplace_back([this] { worker(); });
+  try {
+    for (int i = 1; i < threads; ++i) workers_.emplace_back([this] { worker(); });
+  } catch (...) {  // those started end before the exception goes on
+    end();
+    throw;
+  }
 }
 
-TaskPool::~TaskPool() {
+TaskPool::~TaskPool() { end(); }
+
+void TaskPool::end() {
   {
     std::lock_guard<std::mutex> lk(m_);
     stop_.store(true);
@@ -140,16 +147,35 @@ PoolShelves& shelves() {
   static PoolShelves* s = new PoolShelves;
   return *s;
 }
+
+// A pool already counted on its shelf; null (and no longer counted) when its
+// threads cannot be started.
+std::unique_ptr<TaskPool> start_pool(int threads) {
+  try {
+    return std::make_unique<TaskPool>(threads);
+  } catch (const std::exception&) {
+    PoolShelves& all = shelves();
+    std::lock_guard<std::mutex> lk(all.m);
+    --all.of[threads].pools;
+    return nullptr;
+  }
+}
 }  // namespace
 
 void PoolPlace::set(int threads) {
   if (threads < 1) threads = 1;
   if (threads == threads_) return;
   std::unique_ptr<TaskPool> ended;  // joined outside the lock
+  PoolShelves& all = shelves();
+  bool first = false;  // no pool of this size: start one with the place
   {
-    PoolShelves& all = shelves();
     std::lock_guard<std::mutex> lk(all.m);
-    if (threads > 1) ++all.of[threads].places;
+    if (threads > 1) {
+      PoolShelf& s = all.of[threads];
+      ++s.places;
+      first = s.pools == 0;
+      if (first) ++s.pools;
+    }
     if (threads_ > 1) {
       PoolShelf& s = all.of[threads_];
       --s.places;
@@ -161,6 +187,11 @@ void PoolPlace::set(int threads) {
     }
   }
   threads_ = threads;
+  if (!first) return;
+  std::unique_ptr<TaskPool> pool = start_pool(threads);
+  if (!pool) return;
+  std::lock_guard<std::mutex> lk(all.m);
+  all.of[threads].idle.push_back(std::move(pool));
 }
 
 PoolLease::PoolLease(const PoolPlace& place) {
@@ -177,12 +208,7 @@ PoolLease::PoolLease(const PoolPlace& place) {
     }
     ++s.pools;
   }
-  try {
-    pool_ = new TaskPool(threads);
-  } catch (const std::exception&) {
-    std::lock_guard<std::mutex> lk(all.m);
-    --all.of[threads].pools;
-  }
+  pool_ = start_pool(threads).release();
 }
 
 PoolLease::~PoolLease() {

@@ -42,6 +42,7 @@ class TaskPool {
 
  private:
   void worker();
+  void end();  // stops and joins the workers
   void drain(const std::function<void(int)>& fn, int n);
 
   // A worker joins a job by raising busy_ and then reading fn_; run()
@@ -66,8 +67,9 @@ class TaskPool {
 // one's: three 1080p handles on 16 cores took 4.9 ms per detection, one alone
 // 2.3.  So a handle owns no pool but a place (threads at a time), and a call
 // leases one: the pool given back last, whose workers are still awake, or a
-// new one when calls overlap.  There are never more pools than places of
-// their size, and they end with the places.
+// new one when calls overlap.  The first place starts the first pool (left to
+// the first call it cost that call 0.2 ms).  There are never more pools than
+// places of their size, and they end with the places.
 class PoolPlace {
  public:
   explicit PoolPlace(int threads = 1) { set(threads); }
