@@ -139,10 +139,11 @@ int cctagx_refiner_set_image(cctagx_refiner* r, const uint8_t* gray, int width, 
 int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* markers, int n) {
   if (!r || (n > 0 && !markers) || n < 0 || n > r->max_markers) return CCTAGX_ERR_ARG;
   if (!r->w) return CCTAGX_ERR_STATE;
+  // a refused set leaves the one before it in force, whole
   GradJobDev* hj = r->h_jobs.as<GradJobDev>();
-  r->rjobs.clear();
-  r->rjob_of.assign(n, -1);
-  r->max_cuts = 0;
+  std::vector<RefineJob> rjobs;
+  std::vector<int> rjob_of(n, -1);
+  int max_cuts = 0;
   bool have_mean_ab = false;
   float mean_ab = 0.f;
   for (int i = 0; i < n; ++i) {
@@ -167,7 +168,7 @@ int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* ma
       // a quarter of the grid search's first neighbourhood
       d.alpha0 = 0.25f * r->host.imaged_center_neighbour_size * std::max(e.a(), e.b());
       d.n_cuts = m.n_cuts;
-      r->max_cuts = std::max(r->max_cuts, m.n_cuts);
+      max_cuts = std::max(max_cuts, m.n_cuts);
       d.c0x = m.center0[0];
       d.c0y = m.center0[1];
       std::vector<Pt2> stops;
@@ -181,21 +182,25 @@ int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* ma
       }
       RefineJob rj;
       if (make_refine_job(e, Pt2(m.center0[0], m.center0[1]), stops, r->host, r->kc, mean_ab, rj)) {
-        r->rjob_of[i] = (int)r->rjobs.size();
-        r->rjobs.push_back(std::move(rj));
+        rjob_of[i] = (int)rjobs.size();
+        rjobs.push_back(std::move(rj));
       }
     } catch (const std::exception& ex) {
       set_error(std::string("marker ") + std::to_string(i) + ": " + ex.what());
       return CCTAGX_ERR_ARG;
     }
   }
-  r->n = n;
+  r->n = 0;
   if (n > 0) {
     CCTAGX_HIP(hipMemcpyAsync(r->jobs.as<void>(), hj, sizeof(GradJobDev) * n, hipMemcpyHostToDevice,
                               r->stream));
     CCTAGX_HIP(hipStreamSynchronize(r->stream));
-    if (int rc = to_device(r, r->coarse_of, r->rjob_of.data(), (size_t)n)) return rc;
+    if (int rc = to_device(r, r->coarse_of, rjob_of.data(), (size_t)n)) return rc;
   }
+  r->rjobs = std::move(rjobs);
+  r->rjob_of = std::move(rjob_of);
+  r->max_cuts = max_cuts;
+  r->n = n;
   return CCTAGX_OK;
 }
 

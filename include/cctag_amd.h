@@ -354,6 +354,7 @@ int cctagx_refiner_destroy(cctagx_refiner* r);
 /* The image every marker is sampled in (row-major 8-bit, stride in bytes). */
 int cctagx_refiner_set_image(cctagx_refiner* r, const uint8_t* gray, int width, int height,
                              size_t stride);
+/* A set that is refused (CCTAGX_ERR_ARG) leaves the one before it in force. */
 int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* markers, int n);
 /* Forward + adjoint at given homographies (n x 9, row-major): score (n) and
  * gradient (n x 10: d/dh00 .. d/dh21 with h22 held, then d/d of a
