@@ -204,12 +204,12 @@ __device__ __forceinline__ void lay_out_cuts(const GradJobDev& J, EvalShared<T>&
 }
 
 // Score and, per lane, the derivative sums of its cut at E.H (laid out, after
-// a barrier).  False when fewer than two cuts are valid or H is singular;
-// otherwise every lane of a valid cut holds the cut's L and M (scaled to
+// a barrier).  Returns the valid cuts, none when there are fewer than two or
+// H is singular; every lane of a valid cut holds the cut's L and M (scaled to
 // dC/dw) and E.sum[wave][0] its wavefront's share of the score, to be read
 // after a barrier.  sig: n_cuts x n_samples.
 template <class T, int R, bool LOCAL>
-__device__ __forceinline__ bool eval_marker(const GradJobDev& J, int n_samples, EvalShared<T>& E, T* sig,
+__device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_samples, EvalShared<T>& E, T* sig,
                                             double* L, double* M) {
   const int tid = threadIdx.x, nc = J.n_cuts;
   const int k = tid / kLanesPerCut, j = tid % kLanesPerCut;
@@ -345,11 +345,12 @@ __device__ __forceinline__ bool eval_marker(const GradJobDev& J, int n_samples, 
     M[r] *= scale;
   }
   if ((tid & 63) == 0) E.sum[tid >> 6][0] = cost / (4.0 * (double)m * pairs);
-  return m >= 2 && E.det != 0.0 && isfinite(E.det);
+  return m >= 2 && E.det != 0.0 && isfinite(E.det) ? valid : 0u;
 }
 
-// A cut's share of the score's derivative along dH = D (relative to the
-// origin as E.H): lambda . (D u) summed over its samples, and through the
+// A valid cut's share of the score's derivative along dH = D (relative to the
+// origin as E.H; a cut left out may have no finite direction, and 0 * inf is
+// not 0): lambda . (D u) summed over its samples, and through the
 // cut's direction q, dq = J_pi(v) dv, dv = -H^-1 D v.
 template <class T>
 __device__ __forceinline__ double along(const EvalShared<T>& E, int k, const double* D, const double* L,
@@ -407,7 +408,8 @@ __global__ __launch_bounds__(kMaxGradBlock, sizeof(T) == 4 ? 4 : 1) void k_grad_
   __syncthreads();
   if (tid < 64) lay_out_cuts(J, E);
   __syncthreads();
-  const bool ok = eval_marker<T, R, true>(J, n_samples, E, sig, L, M);
+  const uint32_t valid = eval_marker<T, R, true>(J, n_samples, E, sig, L, M);
+  const bool ok = valid != 0;
   if (grad) {
     // directions 0..7: H's free entries (an entry of the last row moves the
     // relative rows above it too); 8, 9: the marker-plane shift of the centre
@@ -422,7 +424,7 @@ __global__ __launch_bounds__(kMaxGradBlock, sizeof(T) == 4 ? 4 : 1) void k_grad_
         else if (d < 6) D[e] = e == d ? 1.0 : 0.0;
         else D[e] = r == 2 ? 1.0 : r == 0 ? -(double)E.ox : -(double)E.oy;
       }
-      const double v = over_cuts(ok && k < nc ? along(E, k, D, L, M) : 0.0);
+      const double v = over_cuts((valid >> k) & 1u ? along(E, k, D, L, M) : 0.0);
       if ((tid & 63) < kLanesPerCut) E.sum[tid >> 6][1 + d] = v;
     }
   }
@@ -484,10 +486,11 @@ __global__ __launch_bounds__(kMaxGradBlock, sizeof(T) == 4 ? 4 : 1) void k_grad_
     __syncthreads();
     if (tid < 64) lay_out_cuts(J, E);
     __syncthreads();
-    const bool ok = eval_marker<T, R, LOCAL>(J, n_samples, E, sig, L, M);
+    const uint32_t valid = eval_marker<T, R, LOCAL>(J, n_samples, E, sig, L, M);
+    const bool ok = valid != 0;
     {
       const int k = tid / kLanesPerCut, s = tid & 1;
-      const double v = over_cuts(ok && k < nc ? along(E, k, E.dir[s], L, M) : 0.0);
+      const double v = over_cuts((valid >> k) & 1u ? along(E, k, E.dir[s], L, M) : 0.0);
       if ((tid & 63) < 2) E.sum[tid >> 6][1 + s] = v;
     }
     __syncthreads();
