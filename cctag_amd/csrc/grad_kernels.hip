@@ -24,8 +24,8 @@
 // derivatives along directions of H: its free entries, or dH/dc of the closed
 // form (evaluated in forward mode with dual numbers) for the centre; each is
 // contracted cut by cut, without forming dC/dH.  Sample positions and
-// interpolation run in T (float in production, double for checking); every
-// sum is in double.
+// interpolation run in T (float in production, double for checking); lambda
+// and every sum are in double.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -119,17 +119,21 @@ constexpr int kMaxGradWaves = kMaxGradBlock / 64;
 
 // One marker's evaluation, by a block of kLanesPerCut lanes per cut.  Lane j
 // of a cut takes its samples j, j + 8, ... (R of them) through both passes:
-// the samples' image gradients, already divided by the projective
-// denominator, stay in registers between the forward pass and the adjoint,
-// which needs only the sums L = sum_i t_i lambda_i and M = sum_i lambda_i
-// per cut (u_ki = (t_i q_k, 1), so sum_i lambda_i u_i^T = [L q_k^T, M]).
+// the samples' image gradients stay in registers between the forward pass and
+// the adjoint (in double), which needs only the sums L = sum_i t_i lambda_i
+// and M = sum_i lambda_i per cut (u_ki = (t_i q_k, 1), so sum_i lambda_i u_i^T
+// = [L q_k^T, M]).
 //
 // LOCAL (the refiner's calls): positions are taken relative to (ox, oy), the
 // pixel of the centre.  A float position then errs by ulps of the marker's
-// size instead of the image's (2.5e-4 px at 4000 px; the gradient of 2048
-// markers in a 7360 px mosaic is off by 6e-5 instead of 1.1e-3), and a cut's
-// samples are w(t) = t A_k + H_{:,2} with A_k = H_{:,01} q_k in double, three
-// fused multiply-adds.
+// size instead of the image's (2.5e-4 px at 4000 px; score and gradient of
+// 2048 markers in a 7360 px mosaic are off by 1.7e-5 instead of 8.3e-4, and 20
+// descent steps of 4096 markers end 2e-5 px from those with positions in
+// double, not 4e-3), and a cut's samples are w(t) = t A_k + H_{:,2} with
+// A_k = H_{:,01} q_k in double, three fused multiply-adds.  The quotients are
+// correctly rounded; a rounded reciprocal in their place and in the adjoint,
+// with a third value per sample kept between the passes, took longer (20
+// steps 1300 us).
 // Otherwise (the identification): image coordinates, each float operation
 // rounded on its own and the adjoint in double, which keeps the identified
 // markers' qualities and homographies as they always were: a descent of 30
@@ -139,7 +143,7 @@ constexpr int kMaxGradWaves = kMaxGradBlock / 64;
 // Bound by instruction issue, at 4096 markers.  Before, the forward pass took
 // two double divisions per sample, the adjoint sampled the image again and
 // took three more, and the closed form, the inverse and the score's sum ran
-// on one lane: 20 steps of 4096 markers 4270 us, now 1300; one evaluation of
+// on one lane: 20 steps of 4096 markers 4270 us, now 1000; one evaluation of
 // 2048 markers 124 us, now 36.
 template <class T>
 struct EvalShared {
@@ -154,16 +158,18 @@ struct EvalShared {
   int ox, oy;
 };
 
-template <class T>
-__device__ __forceinline__ T recip(T w);
-template <>
-__device__ __forceinline__ double recip(double w) {
-  return 1.0 / w;
+// u / w and v / w, correctly rounded; `plain`: w is in div2_rn's range.
+__device__ __forceinline__ void quotients(float u, float v, float w, bool plain, float& x, float& y) {
+  if (plain) {
+    div2_rn(u, v, w, x, y);
+  } else {
+    x = u / w;
+    y = v / w;
+  }
 }
-template <>
-__device__ __forceinline__ float recip(float w) {  // within 1 ulp
-  const float r = __builtin_amdgcn_rcpf(w);
-  return __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
+__device__ __forceinline__ void quotients(double u, double v, double w, bool, double& x, double& y) {
+  x = u / w;
+  y = v / w;
 }
 __device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
@@ -215,9 +221,7 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
   const int k = tid / kLanesPerCut, j = tid % kLanesPerCut;
   const bool on = k < nc;
   const T b = (T)J.begin_sig, step = ((T)J.end_sig - (T)J.begin_sig) / (T)(n_samples - 1);
-  // per sample the doubled sample's derivatives along x and y (LOCAL: over
-  // the denominator, and the adjoint's third component)
-  T gx[R], gy[R], gz[LOCAL ? R : 1];
+  T gx[R], gy[R];  // per sample the doubled sample's derivatives along x and y
   if (on) {
     const T xlo = (T)(-E.ox), xhi = (T)(J.iw - 1 - E.ox), ylo = (T)(-E.oy), yhi = (T)(J.ih - 1 - E.oy);
     const int base = E.oy * J.iw + E.ox;
@@ -230,7 +234,7 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
     constexpr int kBatch = 7;  // samples whose image reads are in flight together
 #pragma unroll
     for (int t0 = 0; t0 < R; t0 += kBatch) {
-      T x[kBatch], y[kBatch], r[kBatch];
+      T x[kBatch], y[kBatch];
       uint32_t q[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
@@ -238,19 +242,12 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
         const int i = j + (t0 + u) * kLanesPerCut;
         const T t = b + (T)i * step;
         if constexpr (LOCAL) {
-          r[u] = recip<T>(fused(t, a2, H[8]));
-          x[u] = fused(t, a0, H[2]) * r[u];
-          y[u] = fused(t, a1, H[5]) * r[u];
+          quotients(fused(t, a0, H[2]), fused(t, a1, H[5]), fused(t, a2, H[8]), plain, x[u], y[u]);
         } else {
           const T ux = t * qx, uy = t * qy;
           const T w0 = H[0] * ux + H[1] * uy + H[2], w1 = H[3] * ux + H[4] * uy + H[5],
                   w2 = H[6] * ux + H[7] * uy + H[8];
-          if (plain) {
-            div2_rn(w0, w1, w2, x[u], y[u]);
-          } else {
-            x[u] = w0 / w2;
-            y[u] = w1 / w2;
-          }
+          quotients(w0, w1, w2, plain, x[u], y[u]);
         }
         const bool in = x[u] >= xlo && x[u] < xhi && y[u] >= ylo && y[u] < yhi;
         out |= i < n_samples && !in;
@@ -268,11 +265,9 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
         T val;
         if constexpr (LOCAL) {
           const T top = fused(fx, d0, p00), dy = fused(fx, d1, p01) - top;
-          const T dx = fused(fy, d1 - d0, d0);
           val = fused(fy, dy, top);
-          gx[t0 + u] = dx * r[u];
-          gy[t0 + u] = dy * r[u];
-          gz[t0 + u] = -(gx[t0 + u] * x[u] + gy[t0 + u] * y[u]);
+          gx[t0 + u] = fused(fy, d1 - d0, d0);
+          gy[t0 + u] = dy;
         } else {
           const T fx1 = (T)1 - fx, fy1 = (T)1 - fy;
           val = p00 * fx1 * fy1 + p10 * fx * fy1 + p01 * fx1 * fy + p11 * fx * fy;
@@ -313,15 +308,9 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
         const double d = dm * (double)sig[k * n_samples + i] - E.S[i];
         const double tt = (double)(b + (T)i * step);
         cost = __builtin_fma(d, d, cost);
-        double g[3] = {(double)gx[t], (double)gy[t], 0.0};
-        if constexpr (LOCAL) {
-          g[2] = (double)gz[t];
-        } else {
-          const double rw = recip<double>(__builtin_fma(tt, A[2], E.H[8]));
-          g[0] *= rw;
-          g[1] *= rw;
-          g[2] = -(g[0] * __builtin_fma(tt, A[0], E.H[2]) + g[1] * __builtin_fma(tt, A[1], E.H[5])) * rw;
-        }
+        const double rw = 1.0 / __builtin_fma(tt, A[2], E.H[8]);
+        double g[3] = {(double)gx[t] * rw, (double)gy[t] * rw, 0.0};
+        g[2] = -(g[0] * __builtin_fma(tt, A[0], E.H[2]) + g[1] * __builtin_fma(tt, A[1], E.H[5])) * rw;
 #pragma unroll
         for (int r = 0; r < 3; ++r) {
           const double dg = d * g[r];
