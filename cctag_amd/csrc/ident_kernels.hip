@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cfloat>
 
+#include "cut_place.hpp"
 #include "ident_device.hpp"
 
 namespace cctagx {
@@ -552,48 +553,6 @@ __device__ __forceinline__ void cut_walk_begin(const float* Hi, float2 stop, flo
   first = make_float2(xs, ys);
 }
 
-// Where the samples of a cut lie at a grid point (homography H, inverse Hi),
-// decided from the two ends of the cut.  The samples are, up to rounding,
-// the images of the marker-plane segment t * b, t in [begin, end], b the stop
-// back-projected (homogeneous b = Hi (stop, 1)).  When the projective
-// denominator keeps its sign between the ends (it is linear in t) the image
-// is the straight segment between the ends' images, so two ends 2 px inside
-// the image keep every sample in [0, w-1) x [0, h-1), and one end 2 px
-// outside puts its own sample outside.  The positions compared here and the
-// samples' own differ by their rounding: a relative 2^-22 or so of the terms'
-// magnitudes over the denominator, below 0.1 px where `steady` holds.  The
-// window on the denominator keeps div2_rn away from the ends of the float
-// range.  Anything else is kUnsure and gets its samples tested.
-enum CutPlace { kInside, kOutside, kUnsure };
-__device__ __forceinline__ CutPlace cut_place(const float* H, const float* Hi, float2 stop,
-                                              float begin_sig, float end_sig, int w, int h) {
-  const float b0 = Hi[0] * stop.x + Hi[1] * stop.y + Hi[2];
-  const float b1 = Hi[3] * stop.x + Hi[4] * stop.y + Hi[5];
-  const float b2 = Hi[6] * stop.x + Hi[7] * stop.y + Hi[8];
-  bool all_in = true, out = false;
-  float den[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const float t = e ? end_sig : begin_sig, p0 = t * b0, p1 = t * b1;
-    const float d = H[6] * p0 + H[7] * p1 + H[8] * b2, ad = fabsf(d);
-    const float s = d < 0.f ? -1.f : 1.f;
-    const float x = s * (H[0] * p0 + H[1] * p1 + H[2] * b2);  // times |d|: the position
-    const float y = s * (H[3] * p0 + H[4] * p1 + H[5] * b2);
-    const float mag = fmaxf(fabsf(H[0] * p0) + fabsf(H[1] * p1) + fabsf(H[2] * b2),
-                            fabsf(H[3] * p0) + fabsf(H[4] * p1) + fabsf(H[5] * b2));
-    const float dmag = fabsf(H[6] * p0) + fabsf(H[7] * p1) + fabsf(H[8] * b2);
-    const bool steady = ad > 0.05f * dmag && mag < 65536.f * ad && ad > 0x1p-60f * fabsf(b2) &&
-                        ad < 0x1p60f * fabsf(b2);
-    den[e] = d;
-    all_in &= steady && x >= 2.f * ad && x <= (float)(w - 3) * ad && y >= 2.f * ad &&
-              y <= (float)(h - 3) * ad;
-    out |= steady && (x < -2.f * ad || x > (float)(w + 1) * ad || y < -2.f * ad ||
-                      y > (float)(h + 1) * ad);
-  }
-  if (out) return kOutside;
-  return all_in && (den[0] > 0.f) == (den[1] > 0.f) ? kInside : kUnsure;
-}
-
 // u / w and v / w, each correctly rounded: the reciprocal refined by one
 // Newton step, a quotient and two remainder corrections (Markstein, IBM J.
 // Res. Dev. 1990), which is the division's own sequence without its scaling
@@ -880,7 +839,7 @@ __global__ __launch_bounds__(kMaxRefineBlock) void k_refine_iter(
       H[r] = gH[g][r];
       Hi[r] = gHi[g][r];
     }
-    CutPlace at = cut_place(H, Hi, stop, J.begin_sig, J.end_sig, J.iw, J.ih);
+    CutPlace at = cut_place(H, Hi, stop.x, stop.y, J.begin_sig, J.end_sig, J.iw, J.ih);
     inside = at == kInside;
     if (at == kUnsure && samples_leave(im, H, Hi, stop, J.begin_sig, J.end_sig, ns)) at = kOutside;
     if (at == kOutside) {
@@ -1007,7 +966,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_r
     __syncthreads();
     for (int p = tid; p < G2 * nc; p += B) {
       const int k = p / G2, gp = p - k * G2;
-      const CutPlace at = cut_place(gH[gp], gHi[gp], J.stops[k], J.begin_sig, J.end_sig, J.iw, J.ih);
+      const float2 stop = J.stops[k];
+      const CutPlace at =
+          cut_place(gH[gp], gHi[gp], stop.x, stop.y, J.begin_sig, J.end_sig, J.iw, J.ih);
       if (at == kUnsure) {
         atomicOr(&unsure[gp], 1u << k);
         any_unsure = 1;

@@ -137,6 +137,7 @@ double oracle_time_front_end(const uint8_t* img, int w, int h, int n_levels, int
 // Full CPU detection: the oracle front end, candidate stage, identification
 // and de-duplication.  The library's host candidate stage (pipeline.hpp) is
 // linked only as the thing under test of oracle_candidate_mismatch.
+#include "../cctag_amd/csrc/cut_place.hpp"
 #include "../cctag_amd/csrc/host/cabi.hpp"
 #include "../cctag_amd/csrc/host/pipeline.hpp"
 #include "oracle_cand.hpp"
@@ -446,6 +447,29 @@ int oracle_sample_cut(const uint8_t* img, int w, int h, const float* H, const fl
                       float begin, float end, int n, int homography, float* sig) {
   const oracle::DPt p{stop[0], stop[1], 0.f, 0.f};
   return oracle::sample_cut(img, w, h, H, p, begin, end, n, homography != 0, sig) ? 1 : 0;
+}
+// The library's cut_place for n cases (H 9 and stop 2 floats each) in a w x h
+// image, and the extent (min x, max x, min y, max y) of the positions the
+// cut's samples are read at, NaN positions as +inf.
+void oracle_cut_places(int n, const float* H, const float* stop, float begin, float end, int samples,
+                       int w, int h, int* place, float* extent) {
+  std::vector<float> xy(2 * (size_t)samples);
+  for (int c = 0; c < n; ++c) {
+    float Hi[9];
+    const float* s = stop + 2 * c;
+    oracle::cut_positions(H + 9 * c, s[0], s[1], begin, end, samples, Hi, xy.data());
+    place[c] = (int)cctagx::cut_place(H + 9 * c, Hi, s[0], s[1], begin, end, w, h);
+    for (int a = 0; a < 2; ++a) {
+      float lo = INFINITY, hi = -INFINITY;
+      for (int i = 0; i < samples; ++i) {
+        const float v = std::isnan(xy[2 * i + a]) ? INFINITY : xy[2 * i + a];
+        lo = std::min(lo, v);
+        hi = std::max(hi, v);
+      }
+      extent[4 * c + 2 * a] = lo;
+      extent[4 * c + 2 * a + 1] = hi;
+    }
+  }
 }
 int oracle_cut_distances(int n_crowns, const float* sig, int n, float begin, float end,
                          float* out) {

@@ -735,6 +735,25 @@ bool sample_cut(const uint8_t* img, int w, int h, const float* H, const DPt& sto
   return c.oob;
 }
 
+void cut_positions(const float* H, float sx, float sy, float begin, float end, int n, float* Hinv,
+                   float* xy) {
+  M3 M;
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) M.m[i][j] = H[i * 3 + j];
+  const M3 Mi = inverse(M);
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) Hinv[i * 3 + j] = Mi.m[i][j];
+  float bx, by;
+  apply_h(bx, by, Mi, sx, sy);
+  float x = bx * begin, y = by * begin;
+  const float stepX = (bx * end - x) / (n - 1.f), stepY = (by * end - y) / (n - 1.f);
+  for (int i = 0; i < n; ++i) {
+    apply_h(xy[2 * i], xy[2 * i + 1], M, x, y);
+    x += stepX;
+    y += stepY;
+  }
+}
+
 bool refine_stop(const uint8_t* img, int w, int h, DPt& stop, float scale, int n_ref) {
   Cut c;
   c.stop = stop;

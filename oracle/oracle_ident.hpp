@@ -80,6 +80,10 @@ void cut_distances(const std::vector<float>& sig, float begin, float end,
 // (Identification.cpp:1221-1235).
 float start_signal(int n_crowns);
 
+// The positions (n x 2) at which extract_signal samples a cut, and the
+// inverse it takes (0 < begin).
+void cut_positions(const float* H, float sx, float sy, float begin, float end, int n, float* Hinv,
+                   float* xy);
 // One cut's signal: with `homography`, extractSignalUsingHomography
 // (Identification.cpp:216-280) through the 3x3 row-major H (marker plane ->
 // image) towards `stop`; else cutInterpolated (:396-459) from the start

@@ -62,6 +62,9 @@ def load():
     o.oracle_homography_from_center.restype = None
     o.oracle_conditioner.argtypes = [ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                      ctypes.c_float, vp]
+    o.oracle_cut_places.argtypes = [ctypes.c_int, vp, vp, ctypes.c_float, ctypes.c_float, ctypes.c_int,
+                                    ctypes.c_int, ctypes.c_int, vp, vp]
+    o.oracle_cut_places.restype = None
     o.oracle_sample_cut.argtypes = [vp, ctypes.c_int, ctypes.c_int, vp, vp, ctypes.c_float,
                                     ctypes.c_float, ctypes.c_int, ctypes.c_int, vp]
     o.oracle_conditioner.restype = None
@@ -319,6 +322,19 @@ def conditioner(cx: float, cy: float, a: float, b: float) -> np.ndarray:
     T = np.zeros(9, np.float32)
     load().oracle_conditioner(cx, cy, a, b, T.ctypes.data)
     return T.reshape(3, 3)
+
+
+def cut_places(H, stops, n_samples: int, w: int, h: int, begin: float = 0.25, end: float = 1.0):
+    """The library's decision for each (homography, stop) -- 0 inside, 1
+    outside, 2 unsure -- and the extent (n x 4: min x, max x, min y, max y) of
+    the positions at which the cut's samples are read."""
+    H = np.ascontiguousarray(np.asarray(H, np.float32).reshape(-1, 9))
+    st = np.ascontiguousarray(np.asarray(stops, np.float32).reshape(-1, 2))
+    place = np.zeros(len(H), np.int32)
+    ext = np.zeros((len(H), 4), np.float32)
+    load().oracle_cut_places(len(H), H.ctypes.data, st.ctypes.data, begin, end, n_samples, w, h,
+                             place.ctypes.data, ext.ctypes.data)
+    return place, ext
 
 
 def sample_cut(img: np.ndarray, stop, begin: float, end: float, n: int, H=None, start=None):
