@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cstdlib>
 #include <map>
 #include <memory>
@@ -136,6 +137,7 @@ void TaskPool::run(int n, const std::function<void(int)>& fn) {
 namespace {
 struct PoolShelf {
   int places = 0, pools = 0;          // pools: leased and idle
+  int most = INT_MAX;                 // pools that could be started when it was last tried
   std::vector<std::unique_ptr<TaskPool>> idle;  // the last one was used last
 };
 struct PoolShelves {
@@ -148,67 +150,79 @@ PoolShelves& shelves() {
   return *s;
 }
 
-// A pool already counted on its shelf; null (and no longer counted) when its
-// threads cannot be started.
-std::unique_ptr<TaskPool> start_pool(int threads) {
+// Threads may have become free, or scarce: starting one is worth a try again.
+void try_again(PoolShelves& all) {
+  for (auto& s : all.of) s.second.most = INT_MAX;
+}
+
+// A place more for pools of `threads`, and its first pool when there is none.
+// Throws, with nothing changed, when the pool's threads cannot be started.
+void enter(int threads) {
+  PoolShelves& all = shelves();
+  std::unique_lock<std::mutex> lk(all.m);
+  PoolShelf& s = all.of[threads];
+  s.idle.reserve(s.places + 1);  // a lease's end allocates nothing
+  ++s.places;
+  try_again(all);
+  if (s.pools > 0) return;
+  ++s.pools;
+  lk.unlock();
+  std::unique_ptr<TaskPool> pool;
   try {
-    return std::make_unique<TaskPool>(threads);
-  } catch (const std::exception&) {
-    PoolShelves& all = shelves();
-    std::lock_guard<std::mutex> lk(all.m);
-    --all.of[threads].pools;
-    return nullptr;
+    pool = std::make_unique<TaskPool>(threads);
+  } catch (...) {
+    lk.lock();
+    --s.pools;
+    --s.places;
+    throw;
   }
+  lk.lock();
+  s.idle.push_back(std::move(pool));
+}
+
+void leave(int threads) {
+  std::unique_ptr<TaskPool> ended;  // joined outside the lock
+  PoolShelves& all = shelves();
+  std::lock_guard<std::mutex> lk(all.m);
+  PoolShelf& s = all.of[threads];
+  --s.places;
+  if (s.pools > s.places && !s.idle.empty()) {
+    ended = std::move(s.idle.front());
+    s.idle.erase(s.idle.begin());
+    --s.pools;
+  }
+  try_again(all);
 }
 }  // namespace
 
 void PoolPlace::set(int threads) {
   if (threads < 1) threads = 1;
   if (threads == threads_) return;
-  std::unique_ptr<TaskPool> ended;  // joined outside the lock
-  PoolShelves& all = shelves();
-  bool first = false;  // no pool of this size: start one with the place
-  {
-    std::lock_guard<std::mutex> lk(all.m);
-    if (threads > 1) {
-      PoolShelf& s = all.of[threads];
-      ++s.places;
-      first = s.pools == 0;
-      if (first) ++s.pools;
-    }
-    if (threads_ > 1) {
-      PoolShelf& s = all.of[threads_];
-      --s.places;
-      if (s.pools > s.places && !s.idle.empty()) {
-        ended = std::move(s.idle.front());
-        s.idle.erase(s.idle.begin());
-        --s.pools;
-      }
-    }
-  }
+  if (threads > 1) enter(threads);
+  if (threads_ > 1) leave(threads_);
   threads_ = threads;
-  if (!first) return;
-  std::unique_ptr<TaskPool> pool = start_pool(threads);
-  if (!pool) return;
-  std::lock_guard<std::mutex> lk(all.m);
-  all.of[threads].idle.push_back(std::move(pool));
 }
 
 PoolLease::PoolLease(const PoolPlace& place) {
   const int threads = place.threads();
   if (threads <= 1) return;
   PoolShelves& all = shelves();
-  {
-    std::lock_guard<std::mutex> lk(all.m);
-    PoolShelf& s = all.of[threads];
-    if (!s.idle.empty()) {
-      pool_ = s.idle.back().release();
-      s.idle.pop_back();
-      return;
-    }
-    ++s.pools;
+  std::unique_lock<std::mutex> lk(all.m);
+  PoolShelf& s = all.of[threads];
+  if (!s.idle.empty()) {
+    pool_ = s.idle.back().release();
+    s.idle.pop_back();
+    return;
   }
-  pool_ = start_pool(threads).release();
+  if (s.pools >= s.most) return;
+  ++s.pools;
+  lk.unlock();
+  try {
+    pool_ = new TaskPool(threads);
+  } catch (const std::exception&) {
+    lk.lock();
+    s.most = --s.pools;
+  }
 }
 
 PoolLease::~PoolLease() {

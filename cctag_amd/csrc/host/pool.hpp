@@ -68,7 +68,8 @@ class TaskPool {
 // 2.3.  So a handle owns no pool but a place (threads at a time), and a call
 // leases one: the pool given back last, whose workers are still awake, or a
 // new one when calls overlap.  The first place starts the first pool (left to
-// the first call it cost that call 0.2 ms).  There are never more pools than
+// the first call it cost that call 0.2 ms), so a size whose threads cannot be
+// started is refused where it is asked for.  There are never more pools than
 // places of their size, and they end with the places.
 class PoolPlace {
  public:
@@ -76,7 +77,9 @@ class PoolPlace {
   ~PoolPlace() { set(1); }
   PoolPlace(const PoolPlace&) = delete;
   PoolPlace& operator=(const PoolPlace&) = delete;
-  void set(int threads);  // 1: no pool; not while a lease is held
+  // 1: no pool; not while a lease is held.  Throws, the place as it was, when
+  // the threads cannot be started.
+  void set(int threads);
   int threads() const { return threads_; }
 
  private:
@@ -85,7 +88,9 @@ class PoolPlace {
 
 class PoolLease {
  public:
-  // No pool (serial work) for one thread, or when none can be started.
+  // No pool (serial work) for one thread, or when calls overlap and another
+  // pool cannot be started; that is not tried again before a place comes or
+  // goes.
   explicit PoolLease(const PoolPlace& place);
   ~PoolLease();
   PoolLease(const PoolLease&) = delete;

@@ -231,7 +231,11 @@ int cctagx_identify(cctagx_handle* h, const cctagx_ident_marker* in, int n,
 /* Host threads of the candidate stage, the counterpart of the reference's
  * tbb::parallel_for loops (Detection.cpp:616,644,680).  A handle starts with
  * min(16, hardware threads) or $CCTAGX_HOST_THREADS; 0 restores that default,
- * 1 runs the stage on the calling thread.  Results do not depend on it. */
+ * 1 runs the stage on the calling thread.  Results do not depend on it.  The
+ * threads are shared by the handles of the process that ask for as many, a
+ * set per call that runs at a time.  Threads that cannot be started are
+ * refused (CCTAGX_ERR_ARG, the handle as it was); where only the further set
+ * of an overlapping call cannot be started, that call runs on its own thread. */
 int cctagx_set_host_threads(cctagx_handle* h, int threads);
 int cctagx_get_host_threads(cctagx_handle* h);
 

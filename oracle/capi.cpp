@@ -4,10 +4,14 @@
 #include "../include/cctag_amd.h"
 #include "oracle.hpp"
 
+#include <sys/resource.h>
+#include <unistd.h>
+
 #include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <fstream>
 #include <string>
 #include <algorithm>
 #include <atomic>
@@ -513,6 +517,26 @@ int oracle_detect(const cctagx_params* params, const uint8_t* img, int w, int h,
 // g[5i .. 5i+4] = (gx_front, gy_front, gx_back, gy_back, dir): the number of
 // cases in which any of the three decisions differs.  The first neighbour
 // direction is compared modulo 8, the only way the linking uses it.
+int oracle_linking_mismatches(const float* g, int n) {
+  const float pi = 3.14159265358979323846f;
+  auto angle = [&](float gx, float gy) { return std::fmod(std::atan2(gy, gx) + 2.0f * pi, 2.0f * pi); };
+  int bad = 0;
+  for (int i = 0; i < n; ++i) {
+    const float fx = g[5 * i], fy = g[5 * i + 1], bx = g[5 * i + 2], by = g[5 * i + 3];
+    const int dir = g[5 * i + 4] < 0.f ? -1 : 1;
+    const float af = angle(fx, fy), ab = angle(bx, by);
+    const int shifting = (int)std::round(((af + pi / 4.0f) / (2.0f * pi)) * 8.0f) - 1;
+    const bool full = dir * std::sin(ab - af) < 0.0f;
+    const float s = dir * std::sin(ab - af), c = std::cos(ab - af);
+    const bool part = ((s < -0.707f) && (c > 0.f)) || ((s < 0.f) && (c < 0.f));
+    if (cctagx::linking_shift(fx, fy) != ((shifting % 8) + 8) % 8 ||
+        cctagx::convexity_lost(fx, fy, bx, by, dir, true) != full ||
+        cctagx::convexity_lost(fx, fy, bx, by, dir, false) != part)
+      ++bad;
+  }
+  return bad;
+}
+
 // The process's shared worker pools: `users` threads, each with a place of its
 // own, lease a pool `rounds` times and sum 0..n-1 on it, after the same users
 // have taken turns on one thread.  Returns 0, or the number of the first
@@ -553,24 +577,48 @@ int oracle_pool_places(int users, int threads, int rounds) {
   return pools_alive(threads) == 0 ? 0 : 4;
 }
 
-int oracle_linking_mismatches(const float* g, int n) {
-  const float pi = 3.14159265358979323846f;
-  auto angle = [&](float gx, float gy) { return std::fmod(std::atan2(gy, gx) + 2.0f * pi, 2.0f * pi); };
-  int bad = 0;
-  for (int i = 0; i < n; ++i) {
-    const float fx = g[5 * i], fy = g[5 * i + 1], bx = g[5 * i + 2], by = g[5 * i + 3];
-    const int dir = g[5 * i + 4] < 0.f ? -1 : 1;
-    const float af = angle(fx, fy), ab = angle(bx, by);
-    const int shifting = (int)std::round(((af + pi / 4.0f) / (2.0f * pi)) * 8.0f) - 1;
-    const bool full = dir * std::sin(ab - af) < 0.0f;
-    const float s = dir * std::sin(ab - af), c = std::cos(ab - af);
-    const bool part = ((s < -0.707f) && (c > 0.f)) || ((s < 0.f) && (c < 0.f));
-    if (cctagx::linking_shift(fx, fy) != ((shifting % 8) + 8) % 8 ||
-        cctagx::convexity_lost(fx, fy, bx, by, dir, true) != full ||
-        cctagx::convexity_lost(fx, fy, bx, by, dir, false) != part)
-      ++bad;
+// Pools whose threads cannot be started (the process's address space held to
+// what it has): returns 0, or the number of the first property that failed --
+// a place refuses the size and stays as it was (1), leaves no pool behind (2),
+// still takes a size that has one (3); of two overlapping users one has the
+// pool and the other works serially (4), without another try while nothing has
+// changed (5); a place that comes makes it one again (6).
+int oracle_pool_refusal() {
+  using namespace cctagx;
+  PoolPlace a(4), b;
+  rlimit was{};
+  long pages = 0;
+  std::ifstream("/proc/self/statm") >> pages;
+  if (pages <= 0 || getrlimit(RLIMIT_AS, &was)) return -1;
+  rlimit held = was;
+  held.rlim_cur = (rlim_t)pages * sysconf(_SC_PAGESIZE) + (4 << 20);  // less than a thread's stack
+  if (setrlimit(RLIMIT_AS, &held)) return -1;
+  int rc = 0;
+  try {
+    b.set(64);
+    rc = 1;
+  } catch (const std::exception&) {
   }
-  return bad;
+  if (!rc && b.threads() != 1) rc = 1;
+  if (!rc && pools_alive(64) != 0) rc = 2;
+  b.set(4);
+  if (!rc && (b.threads() != 4 || pools_alive(4) != 1)) rc = 3;
+  std::atomic<int> sum{0};
+  {
+    const PoolLease of_a(a);
+    const PoolLease of_b(b);
+    parallel_for(of_b.get(), 100, [&](int i) { sum += i; });
+    if (!rc && (!of_a.get() || of_b.get() || sum != 4950 || pools_alive(4) != 1)) rc = 4;
+  }
+  if (setrlimit(RLIMIT_AS, &was)) return -1;
+  {
+    const PoolLease of_a(a), of_b(b);
+    if (!rc && of_b.get()) rc = 5;
+  }
+  PoolPlace c(4);
+  const PoolLease of_a(a), of_b(b);
+  if (!rc && (!of_b.get() || of_b.get() == of_a.get())) rc = 6;
+  return rc;
 }
 
 // The RANSAC trials' classification of the shared candidate stage
