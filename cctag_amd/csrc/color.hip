@@ -55,12 +55,17 @@ int FrontEndDevice::upload_color(int frame, const uint8_t* bgr, size_t stride, i
     color_in_flight_ = false;
     const void* had = color_pinned_.as<uint8_t>();
     if (color_pinned_.ensure(row * d.h)) return -2;
-    // A new buffer is filled by this thread alone: its pages are mapped as
-    // they are first written, and sixteen threads that fault at once wait for
-    // one lock (first load of a 1366x768 colour frame 1040-1440 us by the
-    // pool, 160 so).
+    // A new buffer's pages are mapped as they are first written.  By one thread
+    // that runs at 2.8 GB/s (2.4 ms at 1920x1080, 9 at 3840x2160, 35 at
+    // 7680x4320, three channels); sixty-four interleaved pieces on sixteen
+    // threads wait for each other's mappings below 16 MB (0.7 to 3.1 ms at
+    // 1920x1080, 2.5 where a freed buffer's pages come again, 0.28 by one
+    // thread), above they take 2.0 and 5.9 ms.  Few whole ranges do in every
+    // case: eight 0.9 ms at 1920x1080 (0.32 on pages that come again), sixteen
+    // 1.8 and 5.6 at the larger sizes, where eight take 2.2 and 7.7.
     const bool fresh = color_pinned_.as<uint8_t>() != had;
-    copy_rows(fresh ? nullptr : pool, color_pinned_.as<uint8_t>(), bgr, row, d.h, stride);
+    const int pieces = !fresh ? 0 : row * d.h < (size_t)16 << 20 ? 8 : 16;
+    copy_rows(pool, color_pinned_.as<uint8_t>(), bgr, row, d.h, stride, pieces);
     CCTAGX_HIP(hipMemcpyAsync(staged, color_pinned_.as<uint8_t>(), row * d.h,
                               hipMemcpyHostToDevice, s));
     CCTAGX_HIP(hipEventRecord(color_sent_, s));

@@ -186,8 +186,9 @@ int FrontEndDevice::init(const PlaneSet& ps, const FrontEndParams& prm) {
 }
 
 void copy_rows(TaskPool* pool, uint8_t* dst, const uint8_t* src, size_t row_bytes, int rows,
-               size_t stride) {
-  const int parts = std::max(1, std::min(rows, 4 * (pool ? pool->threads() : 1)));
+               size_t stride, int pieces) {
+  if (pieces <= 0) pieces = 4 * (pool ? pool->threads() : 1);
+  const int parts = std::max(1, std::min(rows, pieces));
   parallel_for(pool, parts, [&](int k) {
     const int r0 = (int)((long long)rows * k / parts), r1 = (int)((long long)rows * (k + 1) / parts);
     if (stride == row_bytes)

@@ -8,9 +8,10 @@
 namespace cctagx {
 
 // Copies `rows` rows of `row_bytes` bytes (source rows `stride` apart) to
-// the packed destination, the rows shared among the pool's threads.
+// the packed destination, shared among the pool's threads in `pieces` ranges
+// of rows (0: four per thread).
 void copy_rows(TaskPool* pool, uint8_t* dst, const uint8_t* src, size_t row_bytes, int rows,
-               size_t stride);
+               size_t stride, int pieces = 0);
 
 class FrontEndDevice {
  public:

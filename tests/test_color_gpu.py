@@ -73,3 +73,22 @@ def test_color_argument_errors():
         img = np.zeros((48, 64, 3), np.uint8)
         assert lib.cctagx_load_bgr(det._h, img.ctypes.data, 64, 48, 64 * 3 - 1, 3) == -1
         assert lib.cctagx_load_bgr(det._h, img.ctypes.data, 64, 48, 64 * 3, 2) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h,channels", [(40, 3, 4), (2047, 2048, 4), (1365, 4096, 3), (2736, 2048, 3)])
+def test_first_color_load(w, h, channels):
+    """The first load of a handle fills a new upload buffer in 8 ranges of
+    rows, in 16 from 16 MB on, fewer where there are fewer rows; later loads
+    in more and smaller ones: the same gray frame, also from padded rows."""
+    rng = np.random.default_rng(w)
+    img = rng.integers(0, 256, size=(h, w + 3, channels), dtype=np.uint8)[:, :w]
+    want = oracle_lib.bgr_to_gray(img)
+    prm = _lib.default_params(3)
+    prm.number_of_processed_multires_layers = 1
+    prm.canny_thr_low, prm.canny_thr_high = 1000.0, 2000.0  # no edges to look through
+    with Detector(w, h, params=prm) as det:
+        for _ in range(2):
+            det.load_bgr(img)
+            det.detect_loaded()
+            assert np.array_equal(det.level(0)["img"], want)
