@@ -79,6 +79,12 @@ def test_both_kernels_agree_and_match_float64(n_samples, n_cuts):
     many, ok_many = grid(img, ms * 10, p)  # 160 markers
     assert len(ms) * 10 >= FIRST_BLOCK_PER_MARKER
     assert ok_many.all() and np.array_equal(many, np.tile(few, (10, 1)))
+    # 112 and 52 markers: several chunks per block, so two sample buffers (with
+    # 32 cuts the most LDS a block takes) and blocks that end on a partial chunk
+    for n in (112, 52):
+        got, ok = grid(img, (ms * 7)[:n], p)
+        print("split over blocks", n_samples, n_cuts, n, flush=True)
+        assert ok.all() and np.array_equal(got, np.tile(few, (7, 1))[:n])
     if n_cuts >= 7:  # (two cuts leave the minimum undetermined along a line)
         # the centres of two equal searches agree within the pixel tolerance
         # that the detection tests hold (float sampling moves a near tie)
