@@ -32,6 +32,7 @@
 #include <cfloat>
 
 #include "grad_device.hpp"
+#include "host/rows.hpp"
 
 namespace cctagx {
 namespace {
@@ -580,10 +581,9 @@ void descend_launch(const GradJobDev* jobs, int n, int steps, int max_cuts, int 
 
 hipError_t upload_rows(uint8_t* dst, size_t capacity, const uint8_t* src, int width, int height,
                        size_t stride, hipStream_t s, size_t* pitch) {
-  const size_t span = (size_t)(height - 1) * stride + width;
-  if (span <= capacity) {
+  if (rows_fit(capacity, width, height, stride)) {
     *pitch = stride;
-    return hipMemcpyAsync(dst, src, span, hipMemcpyHostToDevice, s);
+    return hipMemcpyAsync(dst, src, (size_t)(height - 1) * stride + width, hipMemcpyHostToDevice, s);
   }
   *pitch = width;
   return hipMemcpy2DAsync(dst, width, src, stride, width, height, hipMemcpyHostToDevice, s);

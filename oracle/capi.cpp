@@ -144,6 +144,7 @@ double oracle_time_front_end(const uint8_t* img, int w, int h, int n_levels, int
 #include "../cctag_amd/csrc/cut_place.hpp"
 #include "../cctag_amd/csrc/host/cabi.hpp"
 #include "../cctag_amd/csrc/host/pipeline.hpp"
+#include "../cctag_amd/csrc/host/rows.hpp"
 #include "oracle_cand.hpp"
 #include "oracle_ident.hpp"
 
@@ -535,6 +536,10 @@ int oracle_linking_mismatches(const float* g, int n) {
       ++bad;
   }
   return bad;
+}
+
+int oracle_rows_fit(size_t capacity, size_t width, size_t height, size_t stride) {
+  return cctagx::rows_fit(capacity, width, height, stride) ? 1 : 0;
 }
 
 // The process's shared worker pools: `users` threads, each with a place of its
