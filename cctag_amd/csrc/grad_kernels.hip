@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cfloat>
 
+#include "division.hpp"
 #include "grad_device.hpp"
 #include "host/rows.hpp"
 
@@ -97,21 +98,6 @@ __device__ D1 closed_form(const GradJobDev& J, double cx, double cy, int row, in
 __device__ __forceinline__ double adjugate(const double* m, int row, int col) {
   const int i1 = (col + 1) % 3, i2 = (col + 2) % 3, j1 = (row + 1) % 3, j2 = (row + 2) % 3;
   return m[i1 * 3 + j1] * m[i2 * 3 + j2] - m[i1 * 3 + j2] * m[i2 * 3 + j1];
-}
-
-// u / w and v / w, correctly rounded, for w and quotients away from the ends
-// of the float range: the division's own sequence (a Newton step on the
-// reciprocal, two remainder corrections of each quotient; Markstein, IBM J.
-// Res. Dev. 1990) without its scaling, the reciprocal shared.
-__device__ __forceinline__ void div2_rn(float u, float v, float w, float& x, float& y) {
-  float r = __builtin_amdgcn_rcpf(w);
-  r = __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
-  float q = u * r;
-  q = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
-  x = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
-  q = v * r;
-  q = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
-  y = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
 }
 
 constexpr int kLanesPerCut = 8;

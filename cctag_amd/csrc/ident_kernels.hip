@@ -22,6 +22,7 @@
 #include <cfloat>
 
 #include "cut_place.hpp"
+#include "division.hpp"
 #include "ident_device.hpp"
 
 namespace cctagx {
@@ -551,22 +552,6 @@ __device__ __forceinline__ void cut_walk_begin(const float* Hi, float2 stop, flo
   step.x = per_step(xe - xs, ns);
   step.y = per_step(ye - ys, ns);
   first = make_float2(xs, ys);
-}
-
-// u / w and v / w, each correctly rounded: the reciprocal refined by one
-// Newton step, a quotient and two remainder corrections (Markstein, IBM J.
-// Res. Dev. 1990), which is the division's own sequence without its scaling
-// of extreme operands -- w and the quotients are far from the ends of the
-// float range here (cut_place) -- and with the reciprocal shared.
-__device__ __forceinline__ void div2_rn(float u, float v, float w, float& x, float& y) {
-  float r = __builtin_amdgcn_rcpf(w);
-  r = __builtin_fmaf(__builtin_fmaf(-w, r, 1.f), r, r);
-  float q = u * r;
-  q = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
-  x = __builtin_fmaf(__builtin_fmaf(-w, q, u), r, q);
-  q = v * r;
-  q = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
-  y = __builtin_fmaf(__builtin_fmaf(-w, q, v), r, q);
 }
 
 // Second part for the next N samples of a cut from position p on (advanced
@@ -1377,9 +1362,15 @@ void launch_iteration(const RefineJobDev* jobs, int n_jobs, int it, const Search
   k_refine_iter<<<grid, sh.block, sh.lds, s>>>(jobs, it, sh.per, samples(n_samples), grid_n, work);
 }
 
-// Markers from which k_refine_search takes over (22 cuts of 100 samples, 9
-// iterations and the read-out, k_refine_iter against k_refine_search: 128
-// markers 271 / 303 us, 160 markers 320 / 306, 256 markers 381 / 324).
+// Markers from which k_refine_search takes over: where the two meet at the
+// usual 22 cuts; they meet at about 105 markers of 8 cuts and 130 of 32.  100
+// samples, 9 iterations and the centres, k_refine_iter against
+// k_refine_search:
+//    8 cuts  100 markers 118 / 123 us, 128 142 / 124, 150 164 / 125, 256 194 / 129
+//   22 cuts  100 markers 183 / 259 us, 128 233 / 261, 150 277 / 266, 256 337 / 278
+//   32 cuts  100 markers 284 / 361 us, 128 355 / 364, 150 418 / 367, 256 504 / 383
+// The coarse step alone (with one descent step): 52 / 53 us at 128 markers of
+// 8 cuts, 71 / 71 at 150 of 22, 80 / 83 at 128 of 32.
 constexpr int kSearchMinJobs = 150;
 // Chunks per block: as few as keep an iteration's blocks within two per CU
 // (a third of nine wavefronts does not fit beside them; 100 markers 307 us
