@@ -23,9 +23,8 @@
 // dependence of the cut direction q_k on H).  What is asked for are
 // derivatives along directions of H: its free entries, or dH/dc of the closed
 // form (evaluated in forward mode with dual numbers) for the centre; each is
-// contracted cut by cut, without forming dC/dH.  Sample positions and
-// interpolation run in T (float in production, double for checking); lambda
-// and every sum are in double.
+// contracted cut by cut, without forming dC/dH.  Interpolation runs in T (float
+// in production, double for checking); lambda and every sum are in double.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -111,16 +110,17 @@ constexpr int kMaxGradWaves = kMaxGradBlock / 64;
 // and M = sum_i lambda_i per cut (u_ki = (t_i q_k, 1), so sum_i lambda_i u_i^T
 // = [L q_k^T, M]).
 //
-// LOCAL (the refiner's calls): positions are taken relative to (ox, oy), the
-// pixel of the centre.  A float position then errs by ulps of the marker's
-// size instead of the image's (2.5e-4 px at 4000 px; score and gradient of
-// 2048 markers in a 7360 px mosaic are off by 1.7e-5 instead of 8.3e-4, and 20
-// descent steps of 4096 markers end 2e-5 px from those with positions in
-// double, not 4e-3), and a cut's samples are w(t) = t A_k + H_{:,2} with
-// A_k = H_{:,01} q_k in double, three fused multiply-adds.  The quotients are
-// correctly rounded; a rounded reciprocal in their place and in the adjoint,
-// with a third value per sample kept between the passes, took longer (20
-// steps 1300 us).
+// LOCAL (the refiner's calls): a sample's place t, its numerators and its
+// denominator w(t) = t A_k + H_{:,2} (A_k = H_{:,01} q_k) are in double,
+// relative to (ox, oy), the pixel of the centre; T holds the pixel and the
+// offset into it (locate).  With all of it in float, positions in a 7360 px
+// mosaic erred by ulps of the image (2.5e-4 px), and score and gradient of 2048
+// markers by 2.8e-5 and 8.2e-4 against double sampling; relative to (ox, oy),
+// still in float, by 3.0e-7 and 1.6e-5; so by 1.2e-8 and 1.8e-8.  20 descent
+// steps of 4096 markers end within 1e-4 px of those with double sampling, not
+// 4e-3.  (A float position of ulp precision, 1 / w in float and kept as a
+// third value per sample between the passes, took as long for one evaluation
+// and 1300 us for the 20 steps.)
 // Otherwise (the identification): image coordinates, each float operation
 // rounded on its own and the adjoint in double, which keeps the identified
 // markers' qualities and homographies as they always were: a descent of 30
@@ -130,7 +130,7 @@ constexpr int kMaxGradWaves = kMaxGradBlock / 64;
 // Bound by instruction issue, at 4096 markers.  Before, the forward pass took
 // two double divisions per sample, the adjoint sampled the image again and
 // took three more, and the closed form, the inverse and the score's sum ran
-// on one lane: 20 steps of 4096 markers 4270 us, now 1000; one evaluation of
+// on one lane: 20 steps of 4096 markers 4270 us, now 1190; one evaluation of
 // 2048 markers 124 us, now 36.
 template <class T>
 struct EvalShared {
@@ -145,18 +145,41 @@ struct EvalShared {
   int ox, oy;
 };
 
-// u / w and v / w, correctly rounded; `plain`: w is in div2_rn's range.
-__device__ __forceinline__ void quotients(float u, float v, float w, bool plain, float& x, float& y) {
-  if (plain) {
-    div2_rn(u, v, w, x, y);
-  } else {
-    x = u / w;
-    y = v / w;
-  }
+// The image position (u / w, v / w): its pixel and the offsets into it.  In
+// float (`plain`: w is in div2_rn's range) the pixel comes from a rounded
+// quotient, the offset from what the pixel leaves of u, in double, so that it
+// is off by an ulp of its own, not of the position, and a pixel that the
+// rounding missed is put right.  A position within 2^-25 px of a pixel's
+// border is on it (offset 0), whichever side the doubles' rounding left it.
+__device__ __forceinline__ void locate(double u, double v, double w, bool plain, double& px, double& py,
+                                       double& fx, double& fy) {
+  const double x = u / w, y = v / w;
+  px = floor(x);
+  py = floor(y);
+  fx = x - px;
+  fy = y - py;
 }
-__device__ __forceinline__ void quotients(double u, double v, double w, bool, double& x, double& y) {
-  x = u / w;
-  y = v / w;
+__device__ __forceinline__ void locate(double u, double v, double w, bool plain, float& px, float& py,
+                                       float& fx, float& fy) {
+  if (plain) {
+    const float d = (float)w, r0 = __builtin_amdgcn_rcpf(d);
+    const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.f), r0, r0);
+    px = floorf((float)u * r);
+    py = floorf((float)v * r);
+    div2_rn((float)__builtin_fma(-(double)px, w, u), (float)__builtin_fma(-(double)py, w, v), d, fx, fy);
+    const float ex = floorf(fx + 0x1p-25f), ey = floorf(fy + 0x1p-25f);
+    px += ex;
+    py += ey;
+    fx -= ex;
+    fy -= ey;
+  } else {
+    double x, y, ox, oy;
+    locate(u, v, w, false, x, y, ox, oy);
+    px = (float)x;
+    py = (float)y;
+    fx = (float)ox;
+    fy = (float)oy;
+  }
 }
 __device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
@@ -207,59 +230,78 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
   const int tid = threadIdx.x, nc = J.n_cuts;
   const int k = tid / kLanesPerCut, j = tid % kLanesPerCut;
   const bool on = k < nc;
+  // the samples' places along the cut: in double, or (not LOCAL) as T rounds them
   const T b = (T)J.begin_sig, step = ((T)J.end_sig - (T)J.begin_sig) / (T)(n_samples - 1);
+  const double db = J.begin_sig, dstep = ((double)J.end_sig - db) / (n_samples - 1);
+  auto place = [&](int i) {
+    return LOCAL ? __builtin_fma((double)i, dstep, db) : (double)(b + (T)i * step);
+  };
   T gx[R], gy[R];  // per sample the doubled sample's derivatives along x and y
   if (on) {
     const T xlo = (T)(-E.ox), xhi = (T)(J.iw - 1 - E.ox), ylo = (T)(-E.oy), yhi = (T)(J.ih - 1 - E.oy);
     const int base = E.oy * J.iw + E.ox;
+    const double A[3] = {E.A[k][0], E.A[k][1], E.A[k][2]};
     T H[9];
     for (int e = 0; e < 9; ++e) H[e] = (T)E.H[e];
-    const T a0 = (T)E.A[k][0], a1 = (T)E.A[k][1], a2 = (T)E.A[k][2];
     const T qx = (T)E.q[k][0], qy = (T)E.q[k][1];
     const bool plain = (E.plain >> k) & 1u;
     bool out = false;
     constexpr int kBatch = 7;  // samples whose image reads are in flight together
 #pragma unroll
     for (int t0 = 0; t0 < R; t0 += kBatch) {
-      T x[kBatch], y[kBatch];
+      T fx[kBatch], fy[kBatch];
       uint32_t q[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         if (t0 + u >= R) continue;
         const int i = j + (t0 + u) * kLanesPerCut;
-        const T t = b + (T)i * step;
+        T px, py;  // the pixel
+        bool in;
         if constexpr (LOCAL) {
-          quotients(fused(t, a0, H[2]), fused(t, a1, H[5]), fused(t, a2, H[8]), plain, x[u], y[u]);
+          const double t = place(i);
+          locate(__builtin_fma(t, A[0], E.H[2]), __builtin_fma(t, A[1], E.H[5]),
+                 __builtin_fma(t, A[2], E.H[8]), plain, px, py, fx[u], fy[u]);
+          in = px >= xlo && px < xhi && py >= ylo && py < yhi;
         } else {
-          const T ux = t * qx, uy = t * qy;
+          const T t = b + (T)i * step, ux = t * qx, uy = t * qy;
           const T w0 = H[0] * ux + H[1] * uy + H[2], w1 = H[3] * ux + H[4] * uy + H[5],
                   w2 = H[6] * ux + H[7] * uy + H[8];
-          quotients(w0, w1, w2, plain, x[u], y[u]);
+          T x, y;
+          if (plain) {
+            div2_rn(w0, w1, w2, x, y);
+          } else {
+            x = w0 / w2;
+            y = w1 / w2;
+          }
+          in = x >= xlo && x < xhi && y >= ylo && y < yhi;
+          px = floor(x);
+          py = floor(y);
+          fx[u] = x - px;
+          fy[u] = y - py;
         }
-        const bool in = x[u] >= xlo && x[u] < xhi && y[u] >= ylo && y[u] < yhi;
         out |= i < n_samples && !in;
-        const int at = in && i < n_samples ? base + (int)floor(y[u]) * J.iw + (int)floor(x[u]) : 0;
+        const int at = in && i < n_samples ? base + (int)py * J.iw + (int)px : 0;
         q[u] = J.quad[(uint32_t)at];
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         if (t0 + u >= R) continue;
         const int i = j + (t0 + u) * kLanesPerCut;
-        const T fx = x[u] - floor(x[u]), fy = y[u] - floor(y[u]);
+        const T x = fx[u], y = fy[u];
         const T p00 = (T)(q[u] & 255u), p10 = (T)((q[u] >> 8) & 255u), p01 = (T)((q[u] >> 16) & 255u),
                 p11 = (T)(q[u] >> 24);
         const T d0 = p10 - p00, d1 = p11 - p01;
         T val;
         if constexpr (LOCAL) {
-          const T top = fused(fx, d0, p00), dy = fused(fx, d1, p01) - top;
-          val = fused(fy, dy, top);
-          gx[t0 + u] = fused(fy, d1 - d0, d0);
+          const T top = fused(x, d0, p00), dy = fused(x, d1, p01) - top;
+          val = fused(y, dy, top);
+          gx[t0 + u] = fused(y, d1 - d0, d0);
           gy[t0 + u] = dy;
         } else {
-          const T fx1 = (T)1 - fx, fy1 = (T)1 - fy;
-          val = p00 * fx1 * fy1 + p10 * fx * fy1 + p01 * fx1 * fy + p11 * fx * fy;
-          gx[t0 + u] = d0 * fy1 + d1 * fy;
-          gy[t0 + u] = (p01 - p00) * fx1 + (p11 - p10) * fx;
+          const T x1 = (T)1 - x, y1 = (T)1 - y;
+          val = p00 * x1 * y1 + p10 * x * y1 + p01 * x1 * y + p11 * x * y;
+          gx[t0 + u] = d0 * y1 + d1 * y;
+          gy[t0 + u] = (p01 - p00) * x1 + (p11 - p10) * x;
         }
         if (i < n_samples) sig[k * n_samples + i] = val;
       }
@@ -293,7 +335,7 @@ __device__ __forceinline__ uint32_t eval_marker(const GradJobDev& J, int n_sampl
       const int i = j + t * kLanesPerCut;
       if (i < n_samples) {
         const double d = dm * (double)sig[k * n_samples + i] - E.S[i];
-        const double tt = (double)(b + (T)i * step);
+        const double tt = place(i);
         cost = __builtin_fma(d, d, cost);
         const double rw = 1.0 / __builtin_fma(tt, A[2], E.H[8]);
         double g[3] = {(double)gx[t] * rw, (double)gy[t] * rw, 0.0};

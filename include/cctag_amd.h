@@ -363,9 +363,9 @@ int cctagx_refiner_set_markers(cctagx_refiner* r, const cctagx_refine_marker* ma
 /* Forward + adjoint at given homographies (n x 9, row-major): score (n) and
  * gradient (n x 10: d/dh00 .. d/dh21 with h22 held, then d/d of a
  * marker-plane translation (x, y) of the centre, H' = H [1 0 x; 0 1 y; 0 0 1]).
- * fp64 != 0 samples in double (checking), else in float: positions relative
- * to the pixel of the marker's centre and bilinear values, the quotients
- * correctly rounded; sums and the gradient's adjoint are in double either way.
+ * fp64 != 0 samples in double (checking), else the offsets into the pixels and
+ * the bilinear values are float; what is summed and the gradient's adjoint are
+ * in double either way.
  * A marker with fewer than two valid cuts scores DBL_MAX with a zero gradient. */
 int cctagx_refiner_cost_grad(cctagx_refiner* r, const float* H, int fp64, double* cost,
                              double* grad);

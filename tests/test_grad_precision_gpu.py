@@ -1,9 +1,10 @@
 """How the score's float sampling rounds.  A homography and its multiples are
 one map.  With samples on positions that a float holds exactly, and quotients
 and the adjoint's 1 / w correctly rounded or in double, a multiple's samples
-are the same to the bit: the score is equal and the gradient is the first one
-over the factor, to double rounding.  A rounded float reciprocal in either
-place would show at 1e-8 to 1e-7, on pixel borders at any size."""
+are the same: the score is equal and the gradient is the first one over the
+factor, to double rounding.  A rounded float reciprocal in either place would
+show at 1e-8 to 1e-7, on pixel borders (where many of these samples lie) at
+any size."""
 import numpy as np
 import pytest
 
