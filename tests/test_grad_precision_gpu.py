@@ -17,7 +17,7 @@ STOPS = [[80, 70], [50, 60], [66, 90], [71, 40], [58, 50], [75, 75], [40, 81], [
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("factor", [3, 5, 7, 11, -13])
+@pytest.mark.parametrize("factor", [3, 5, 7, 11, -13, 2.0**70, -2.0**-70])  # (the last two: w out of div2_rn's range)
 @pytest.mark.parametrize("shift", [0, 1792])
 def test_multiples_of_a_homography(factor, shift):
     y, x = np.mgrid[0:128, 0:128 + shift]
@@ -31,7 +31,7 @@ def test_multiples_of_a_homography(factor, shift):
         r.set_markers([{"ellipse": (64.0 + shift, 64.0, 16.0, 16.0, 0.0),
                         "center0": (64.0 + shift, 64.0), "stops": stops}])
         c1, g1 = r.cost_grad(H)
-        cf, gf = r.cost_grad(factor * H)
+        cf, gf = r.cost_grad(np.float32(factor) * H)
     gf[0, :8] *= factor
     print(factor, shift, c1, cf, flush=True)
     # double rounding: sums of fewer than 1000 terms in 2^-53
