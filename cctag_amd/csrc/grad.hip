@@ -121,6 +121,10 @@ int cctagx_refiner_set_image(cctagx_refiner* r, const uint8_t* gray, int width, 
                              size_t stride) {
   if (!r || !gray || width < 2 || height < 2 || stride < (size_t)width) return CCTAGX_ERR_ARG;
   if ((size_t)width * height > (size_t)INT32_MAX / 4) return CCTAGX_ERR_ARG;
+  // the markers point into the image that goes: none are left, nor an image,
+  // should what follows fail
+  r->n = 0;
+  r->w = 0;
   if (r->img.ensure((size_t)width * height) || r->quad.ensure(4 * (size_t)width * height))
     return CCTAGX_ERR_HIP;
   size_t pitch = 0;
@@ -132,7 +136,6 @@ int cctagx_refiner_set_image(cctagx_refiner* r, const uint8_t* gray, int width, 
   r->w = width;
   r->h = height;
   r->ident.set_image(r->quad.as<uint32_t>(), width, height);
-  r->n = 0;
   return CCTAGX_OK;
 }
 
